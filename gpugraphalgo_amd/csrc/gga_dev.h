@@ -39,7 +39,8 @@ typedef struct gga_dev_work {
     uint32_t *dist;
     uint32_t *mark;      /* queue steps: step number of a vertex's last listing (de-duplication) */
     uint8_t *flag;       /* flag steps: low byte of the step that last lowered a vertex (n bytes,
-                            set to the byte before the query's first step at query start) */
+                            set to the byte before the query's first step at query start);
+                            level-synchronous BFS: 0 until the vertex is reached */
     uint32_t *q0;
     uint32_t *q1;
     uint32_t *ctl;
@@ -52,6 +53,8 @@ typedef struct gga_dev_work {
     uint32_t dense_min;  /* a step whose list holds >= dense_min chunks is a flag step */
     uint32_t delta;      /* near-far bucket width (0: plain Bellman-Ford worklist) */
     uint32_t bmin;       /* fewest chunks per wave batch */
+    uint32_t epoch;      /* step number of the query's first step */
+    uint32_t lvl;        /* 1: BFS steps are levels (step epoch + k reaches level k + 1) */
 } gga_dev_work;
 
 /* Per-workgroup timeline record of an instrumented relax step: start on the

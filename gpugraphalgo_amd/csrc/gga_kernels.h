@@ -50,6 +50,8 @@ int ggak_scratch(int device, void **ptr);
 /* ---- traversal (relax.hip) ---- */
 int ggak_fill_u32(uint32_t *p, uint32_t value, uint64_t count, hipStream_t s);
 int ggak_query_init(gga_dev_graph g, gga_dev_work w, uint32_t src, uint32_t epoch, hipStream_t s);
+/* 1: worklist / persistent queries on this workspace step BFS level by level (the host sets w.lvl) */
+int ggak_level_sync(gga_dev_work w, int bfs);
 int ggak_topo_step(gga_dev_graph g, gga_dev_work w, int bfs, int count, hipStream_t s);
 /* tl != NULL: instrumented (counting) variant; workgroup b writes tl[b].
  * block: workgroup size, 128, 256 or 512 threads. */

@@ -158,6 +158,8 @@ static gga_dev_work dev_work(const gga_graph *g, uint32_t inf)
     w.tmin = NULL;
     w.delta = 0;
     w.bmin = 1;
+    w.epoch = 0;
+    w.lvl = 0;
     return w;
 }
 
@@ -675,6 +677,8 @@ static int run_query(gga_graph *g, gga_dev_graph dg, gga_dev_work dw, const quer
     const int tev = own && count;
     const uint32_t max_iters = p->max_iters;
     float ktime = 0.f;
+    dw.epoch = p->epoch;
+    dw.lvl = mode != GGA_MODE_TOPO && ggak_level_sync(dw, bfs) ? 1u : 0u;
     int ended = 0;   /* reach pass and control words already fetched */
     *adv = 0;
 

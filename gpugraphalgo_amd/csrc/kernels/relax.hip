@@ -65,6 +65,10 @@ constexpr uint32_t PBUF = 256;          // queued vertices staged per wave befor
 #define GGA_UNROLL 4
 #endif
 constexpr uint32_t UNROLL = GGA_UNROLL; // edge slots per lane per round in expand_batch
+#ifndef GGA_LVL_UNROLL
+#define GGA_LVL_UNROLL 4
+#endif
+constexpr uint32_t LVL_UNROLL = GGA_LVL_UNROLL;   // the same in expand_level
 // Meshes: vertices a wave may follow past its batch within one step (0: off),
 // its LDS queue of them, and the largest degree followed.
 #ifndef GGA_CONT
@@ -94,13 +98,14 @@ struct ChunkDesc {
     bool valid = false;
 };
 
+template <bool OWN = true>
 __device__ __forceinline__ ChunkDesc load_chunk(const gga_dev_graph &g, uint32_t c, bool valid) {
     ChunkDesc d;
     d.valid = valid;
     if (valid) {
         d.eb = stream_load(&g.cbeg[c]);
         d.ee = stream_load(&g.cbeg[c + 1]);
-        d.own = stream_load(&g.cown[c]);
+        if (OWN) d.own = stream_load(&g.cown[c]);
     }
     return d;
 }
@@ -321,6 +326,95 @@ __device__ __forceinline__ void expand_batch(const gga_dev_graph &g, const gga_d
     }
 }
 
+// Expand one batch of a level-synchronous BFS step (w.lvl): every listed
+// chunk's owner was reached in the step before, so its distance is the step's
+// level and is not read, and whatever a step reaches gets the same value,
+// `alt`.  The guard is therefore the byte flag[v] (0: not reached) instead of
+// dist[v] -- n bytes, which an XCD's 4 MB L2 holds where 4 n are gathered past
+// it -- and a flag step needs no atomic: racing (or stale) guards store the
+// same byte, and the compaction gives the stamped vertices their distance.  A
+// queue step takes the vertex with atomicMin's result, which is inf for
+// exactly one of the racers, and stamps it for later guards.
+//
+// What bounds it: the gathers, at the rate the L1s take misses (R-MAT s22,
+// the widest level: 45 M edges in 0.34 ms).  Against guarding with dist[v] and
+// a device-scope atomicMin per improvement: BFS on R-MAT s22 (T = 128) 878 ->
+// 727 us a query, on a 1.5 M-vertex R-MAT graph, ef 8, 450 -> 380 us on the
+// device.  A bitmap of the reached vertices in front of the bytes (hot words
+// in L1) gained 15% in the widest level and lost more in the one before,
+// where half the edges find an unset bit and read the byte as well.
+template <bool COUNT, int OUT>
+__device__ __forceinline__ void expand_level(const gga_dev_graph &g, const gga_dev_work &w, const ChunkDesc &d,
+                                             uint32_t alt, uint8_t stamp, uint32_t *pbuf, uint32_t &pcount,
+                                             uint32_t *qout, uint32_t *tail, Counters &cnt, uint32_t *tab,
+                                             uint32_t nown) {
+    const uint32_t l = lane_id();
+    uint8_t *__restrict__ flag = w.flag;
+    const uint32_t n = d.valid ? d.ee - d.eb : 0u;
+    const uint32_t incl = wave_incl_scan(n);
+    const uint32_t total = wave_last(incl);
+    if (COUNT) {
+        cnt.edges += __builtin_amdgcn_readfirstlane(total);
+        cnt.chunks += __builtin_amdgcn_readfirstlane((uint32_t)__popcll(__ballot(n > 0)));
+    }
+    tab[l] = d.eb - (incl - n);   // slot k of owner j is edge tab[j] + k (see expand_batch)
+    __builtin_amdgcn_wave_barrier();
+    const uint32_t half = nown <= 1u ? 0u : 1u << (31 - __builtin_clz(nown - 1u));
+    for (uint32_t base = 0; base < total; base += GGA_WAVE * LVL_UNROLL) {
+        uint32_t v[LVL_UNROLL], kk[LVL_UNROLL], own[LVL_UNROLL], seen[LVL_UNROLL];
+        const uint32_t left = total - base;
+#pragma unroll
+        for (uint32_t u = 0; u < LVL_UNROLL; u++) {
+            const uint32_t k = base + u * GGA_WAVE + l;
+            kk[u] = k < total ? k : total - 1u;
+            own[u] = 0;
+        }
+        for (uint32_t step = half; step != 0; step >>= 1) {
+#pragma unroll
+            for (uint32_t u = 0; u < LVL_UNROLL; u++) {
+                const uint32_t y = __shfl(incl, (int)(own[u] + step - 1), GGA_WAVE);
+                own[u] += y <= kk[u] ? step : 0u;
+            }
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < LVL_UNROLL; u++) {
+            if (u * GGA_WAVE >= left) break;
+            v[u] = stream_load(&g.col[tab[own[u]] + kk[u]]);
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < LVL_UNROLL; u++) {
+            if (u * GGA_WAVE >= left) break;
+            seen[u] = flag[v[u]];
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < LVL_UNROLL; u++) {
+            if (u * GGA_WAVE >= left) break;
+            bool imp = base + u * GGA_WAVE + l < total && seen[u] == 0u && alt < w.inf;
+            if (OUT == OUT_FLAG) {
+                if (imp) flag[v[u]] = stamp;
+            } else {
+                if (imp) imp = alt < atomic_min_u32(&w.dist[v[u]], alt);
+                if (imp) flag[v[u]] = stamp;
+                const uint64_t mask = __ballot(imp);
+                if (mask) {
+                    const uint32_t nw = (uint32_t)__popcll(mask);
+                    if (pcount + nw > PBUF) {
+                        flush_pushes(g, pbuf, pcount, qout, tail, w.qcap, w.ctl);
+                        pcount = 0;
+                    }
+                    if (imp)
+                        pbuf[pcount + __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32),
+                                                                __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u))] = v[u];
+                    pcount += nw;
+                    __builtin_amdgcn_wave_barrier();
+                }
+            }
+            if (COUNT) cnt.relax += __builtin_amdgcn_readfirstlane((uint32_t)__popcll(__ballot(imp)));
+        }
+    }
+    __builtin_amdgcn_wave_barrier();   // the table is read before the next batch writes it
+}
+
 // Work counters: lane 0 of each wave adds to one of GGA_CNT_SLOTS striped slots.
 template <bool COUNT>
 __device__ __forceinline__ void publish_counters(const gga_dev_work &w, const Counters &c) {
@@ -348,7 +442,8 @@ __global__ __launch_bounds__(BLOCK) void k_query_init(gga_dev_graph g, gga_dev_w
     const uint64_t tid = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const uint64_t nth = (uint64_t)gridDim.x * blockDim.x;
     for (uint64_t v = tid; v < g.n; v += nth) w.dist[v] = (v == src) ? 0u : w.inf;
-    for (uint64_t v = tid; v < g.n; v += nth) w.flag[v] = (uint8_t)(epoch - 1u);
+    for (uint64_t v = tid; v < g.n; v += nth)
+        w.flag[v] = w.lvl ? (v == src ? 255u : 0u) : (uint8_t)(epoch - 1u);
     if (w.last)
         for (uint64_t v = tid; v < g.n; v += nth) w.last[v] = w.inf;
     for (uint64_t i = tid; i < 4ull * GGA_CNT_SLOTS; i += nth) w.cnt[i] = 0;
@@ -397,6 +492,10 @@ __global__ __launch_bounds__(BLOCK) void k_topo_step(gga_dev_graph g, gga_dev_wo
 }
 
 // ------------------------------------------------------ worklist step
+// Level-synchronous BFS (w.lvl): the byte that marks a vertex reached at
+// `level` >= 1; never 0 (not reached), repeating every 254 levels (255: the source).
+__device__ __forceinline__ uint8_t level_stamp(uint32_t level) { return (uint8_t)(1u + (level - 1u) % 254u); }
+
 __device__ __forceinline__ bool flag_step(const gga_dev_work &w, uint32_t nq) {
     return nq >= w.dense_min;
 }
@@ -418,11 +517,14 @@ __device__ __forceinline__ void worklist_step(const gga_dev_graph &g, const gga_
     // 2.17 / 2.14 / 2.26 ms).  Uniform small chunks (meshes, bmin > 1): few
     // large batches -- every batch is a chain of dependent loads -- with one
     // batch per 1/1024 of the list, but at least bmin chunks (4: each wave
-    // then follows its own wavefront, see expand_batch)
+    // then follows its own wavefront, see expand_batch).
+    // Level-synchronous BFS has nothing to leave to the next step and takes 8
+    // batches per wave (R-MAT s22, 4 / 8 / 16 / 32: 773 / 739 / 755 / 802 us)
+    constexpr bool LVL = BFS && !CONT;
     const uint32_t wpb = blockDim.x / GGA_WAVE;   // waves per workgroup (128, 256 or 512 threads)
     const uint32_t waves = gridDim.x * wpb;
     const uint32_t wid = blockIdx.x * wpb + __builtin_amdgcn_readfirstlane(threadIdx.x / GGA_WAVE);
-    uint32_t bsz = w.bmin > 1u ? nq >> 10 : nq / (16u * waves);
+    uint32_t bsz = w.bmin > 1u ? nq >> 10 : nq / ((LVL ? 8u : 16u) * waves);
     bsz = bsz < w.bmin ? w.bmin : bsz;
     bsz = bsz < 1u ? 1u : (bsz > GGA_WAVE ? GGA_WAVE : bsz);
     const uint32_t nbatch = (nq + bsz - 1) / bsz;
@@ -431,6 +533,8 @@ __device__ __forceinline__ void worklist_step(const gga_dev_graph &g, const gga_
     const uint32_t thr = w.ctl[GGA_CTL_THR(step % 3u)];
     uint32_t pcount = 0;
     bool dummy = false;
+    const uint32_t alt = it - w.epoch + 1u;   // LVL: the level this step reaches
+    const uint8_t stamp = level_stamp(alt);
     uint32_t *const follow = (CONT && nq <= CONT_LIST) ? cq : nullptr;   // the continuation's queue
     // Software pipeline over the wave's batches b, b + waves, b + 2 waves...:
     // while a batch is expanded, the next batch's chunk descriptors and the
@@ -449,13 +553,19 @@ __device__ __forceinline__ void worklist_step(const gga_dev_graph &g, const gga_
         bool ok0;
         const uint32_t c0 = entry(wid, ok0);
         c_next = entry((uint64_t)wid + waves, ok_next);
-        cur = load_chunk(g, c0, ok0);
+        cur = load_chunk<!LVL>(g, c0, ok0);
     }
     for (uint64_t b = wid; b < nbatch; b += waves) {
         bool ok_after;
         const uint32_t c_after = entry(b + 2ull * waves, ok_after);
-        const ChunkDesc nxt = load_chunk(g, c_next, ok_next);
-        if (flags)
+        const ChunkDesc nxt = load_chunk<!LVL>(g, c_next, ok_next);
+        if (LVL && flags)
+            expand_level<COUNT, OUT_FLAG>(g, w, cur, alt, stamp, pbuf, pcount, qout, tail, cnt,
+                                          reinterpret_cast<uint32_t *>(tab), bsz);
+        else if (LVL)
+            expand_level<COUNT, OUT_QUEUE>(g, w, cur, alt, stamp, pbuf, pcount, qout, tail, cnt,
+                                           reinterpret_cast<uint32_t *>(tab), bsz);
+        else if (flags)
             expand_batch<BFS, COUNT, OUT_FLAG, CONT>(g, w, cur, it, pbuf, pcount, qout, tail, dummy, cnt, tab, bsz,
                                                      thr, follow);
         else
@@ -491,6 +601,43 @@ struct StampMarked {
         return m;
     }
 };
+
+// Level-synchronous BFS: the vertices a flag step stamped get their distance
+// here (write pass), each written by the thread that lists it.  From the
+// level on at which stamps repeat, a stamped vertex is new only while its
+// distance is still inf (the count pass sees it so too: it writes nothing).
+template <bool WRITE>
+struct LevelMarked {
+    const uint8_t *flag;
+    uint32_t *dist;
+    uint32_t level, inf;
+    uint8_t stamp;
+    static constexpr bool vec8 = true;
+    __device__ __forceinline__ bool operator()(uint32_t v) const {
+        if (flag[v] != stamp || (level > 254u && dist[v] != inf)) return false;
+        if (WRITE) dist[v] = level;
+        return true;
+    }
+    __device__ __forceinline__ uint32_t mark8(uint64_t v) const {
+        uint32_t m = StampMarked{flag, stamp}.mark8(v);
+        if (level > 254u) {
+#pragma unroll
+            for (uint32_t i = 0; i < 8; i++)
+                if (((m >> i) & 1u) && dist[v + i] != inf) m &= ~(1u << i);
+        }
+        if (WRITE) {
+#pragma unroll
+            for (uint32_t i = 0; i < 8; i++)
+                if ((m >> i) & 1u) dist[v + i] = level;
+        }
+        return m;
+    }
+};
+template <bool WRITE>
+__device__ __forceinline__ LevelMarked<WRITE> level_marked(const gga_dev_work &w, uint32_t it) {
+    const uint32_t level = it - w.epoch + 1u;
+    return LevelMarked<WRITE>{w.flag, w.dist, level, w.inf, level_stamp(level)};
+}
 
 // The single list of the plain layout for step `step`.
 __device__ __forceinline__ ListOut list_out(const gga_dev_graph &g, const gga_dev_work &w, uint32_t step) {
@@ -569,6 +716,7 @@ void k_wl_step(gga_dev_graph g, gga_dev_work w, uint32_t step, gga_wg_record *tl
 // queue step.  A count workgroup that finds stamped vertices marks the slot
 // LISTED (plain stores of the same value), so that the write pass knows
 // whether the list is empty without summing every count.
+template <bool LVL>
 __global__ __launch_bounds__(BLOCK) void k_compact_count(gga_dev_graph g, gga_dev_work w, uint32_t step) {
     __shared__ uint32_t s_wave[WAVES];
     const uint32_t nq = step_len(w, step);
@@ -577,7 +725,8 @@ __global__ __launch_bounds__(BLOCK) void k_compact_count(gga_dev_graph g, gga_de
     const uint32_t it = w.ctl[GGA_CTL_ITER(step % 3u)];
     uint32_t any = 0;
     for (uint32_t t = blockIdx.x; t < GGA_TILES(g.n); t += gridDim.x)
-        any |= compact_count_tile(o, g.n, t, StampMarked{w.flag, (uint8_t)it}, s_wave);
+        any |= LVL ? compact_count_tile(o, g.n, t, level_marked<false>(w, it), s_wave)
+                   : compact_count_tile(o, g.n, t, StampMarked{w.flag, (uint8_t)it}, s_wave);
     if (any && threadIdx.x == 0) w.ctl[GGA_CTL_LISTED((step + 1u) % 3u)] = 1u;
 }
 
@@ -717,6 +866,7 @@ __device__ __forceinline__ void refill_write_body(const gga_dev_graph &g, const 
 // which the compaction reads only when the list is not empty.)  Its first
 // thread records the threshold the refill lists under (RTHR) and that this
 // step refills (RSTEP = its step number).
+template <bool LVL>
 __global__ __launch_bounds__(BLOCK) void k_compact_write(gga_dev_graph g, gga_dev_work w, uint32_t step) {
     __shared__ uint32_t s_wave[WAVES], s_min[WAVES];
     const uint32_t nq = step_len(w, step), sout = (step + 1u) % 3u;
@@ -724,12 +874,14 @@ __global__ __launch_bounds__(BLOCK) void k_compact_write(gga_dev_graph g, gga_de
     if (flags) {
         if (!w.last || w.ctl[GGA_CTL_LISTED(sout)] != 0u) {
             const uint32_t it = w.ctl[GGA_CTL_ITER(step % 3u)];
-            compact_write_tiles(list_out(g, w, step), g.n, StampMarked{w.flag, (uint8_t)it}, s_wave);
+            if (LVL) compact_write_tiles(list_out(g, w, step), g.n, level_marked<true>(w, it), s_wave);
+            else compact_write_tiles(list_out(g, w, step), g.n, StampMarked{w.flag, (uint8_t)it}, s_wave);
             return;
         }
     } else if (!w.last || w.ctl[GGA_CTL_TAIL(sout)] != 0u) {
         return;
     }
+    if (LVL) return;   // (BFS has no buckets)
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         w.ctl[GGA_CTL_RTHR] = sat_add(w.ctl[GGA_CTL_THR(sout)], w.delta);
         w.ctl[GGA_CTL_RSTEP] = w.ctl[GGA_CTL_ITER(step % 3u)];
@@ -807,12 +959,15 @@ __global__ __launch_bounds__(BLOCK) void k_persistent(gga_dev_graph g, gga_dev_w
         if (flag_step(w, nq)) {
             const ListOut o = list_out(g, w, step);
             grid_barrier(w.ctl, gridDim.x, gen, spin_ticks);
-            for (uint32_t t = blockIdx.x; t < GGA_TILES(g.n); t += gridDim.x)
-                compact_count_tile(o, g.n, t, StampMarked{w.flag, (uint8_t)it}, s_wave);
+            for (uint32_t t = blockIdx.x; t < GGA_TILES(g.n); t += gridDim.x) {
+                if (BFS && !CONT) compact_count_tile(o, g.n, t, level_marked<false>(w, it), s_wave);
+                else compact_count_tile(o, g.n, t, StampMarked{w.flag, (uint8_t)it}, s_wave);
+            }
             grid_barrier(w.ctl, gridDim.x, gen, spin_ticks);
             // each workgroup sums the tile counts before its own tiles: no
             // serial scan between two more grid barriers
-            compact_write_tiles(o, g.n, StampMarked{w.flag, (uint8_t)it}, s_wave);
+            if (BFS && !CONT) compact_write_tiles(o, g.n, level_marked<true>(w, it), s_wave);
+            else compact_write_tiles(o, g.n, StampMarked{w.flag, (uint8_t)it}, s_wave);
         }
         grid_barrier(w.ctl, gridDim.x, gen, spin_ticks);
         // near-far: an empty next list is refilled from the deferred vertices,
@@ -1085,6 +1240,9 @@ static const void *persistent_fn(int cont) {
 }
 // cont: the graph is a mesh (bmin > 1) and the continuation is compiled in
 static int use_cont(const gga_dev_work &w) { return GGA_CONT > 0 && w.bmin > 1u; }
+// Level-synchronous BFS: worklist and persistent queries without the
+// continuation (which reaches levels out of order).
+extern "C" int ggak_level_sync(gga_dev_work w, int bfs) { return bfs && !use_cont(w); }
 static const void *pick_kernel(int persistent, int bfs, int count, uint32_t block, int cont) {
     if (persistent) {
         if (bfs) return count ? persistent_fn<true, true>(cont) : persistent_fn<true, false>(cont);
@@ -1144,8 +1302,13 @@ extern "C" int ggak_refill(gga_dev_graph g, gga_dev_work w, uint32_t step, hipSt
 extern "C" int ggak_compact(gga_dev_graph g, gga_dev_work w, uint32_t step, hipStream_t s) {
     const uint32_t ntiles = GGA_TILES(g.n);
     const uint32_t grid = ntiles < 2048u ? (ntiles ? ntiles : 1u) : 2048u;
-    k_compact_count<<<grid, BLOCK, 0, s>>>(g, w, step);
-    k_compact_write<<<grid, BLOCK, 0, s>>>(g, w, step);
+    if (w.lvl) {
+        k_compact_count<true><<<grid, BLOCK, 0, s>>>(g, w, step);
+        k_compact_write<true><<<grid, BLOCK, 0, s>>>(g, w, step);
+    } else {
+        k_compact_count<false><<<grid, BLOCK, 0, s>>>(g, w, step);
+        k_compact_write<false><<<grid, BLOCK, 0, s>>>(g, w, step);
+    }
     return launch_status();
 }
 
