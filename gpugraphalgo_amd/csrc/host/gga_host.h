@@ -23,6 +23,7 @@ int gga_graph_view(gga_graph *g, gga_graph_view_t *v);
 /* The graph's cached engine for gga_multi_sp (freed with the graph or a re-split). */
 gga_ms **gga_graph_ms_slot(gga_graph *g);
 /* Tuned defaults (tune.c) that traversals use when their opts leave them 0. */
+uint32_t gga_graph_default_dense(const gga_graph *g, int mode);   /* opts.dense_min when neither given nor tuned */
 void gga_graph_set_tuned(gga_graph *g, uint32_t grid, uint32_t dense_min, uint32_t layout);
 uint32_t gga_graph_tuned_layout(const gga_graph *g);
 /* mode < 0: no tuned mode; delta 0xFFFFFFFF: near-far tuned off, 0: untuned. */

@@ -920,10 +920,30 @@ static void plan_query(const gga_graph *g, int bfs, const gga_opts *o, query_pla
         p->max_iters = (uint64_t)64u * (g->n + 1u) < 0xFFFFFFF0ull ? 64u * (g->n + 1u) : 0xFFFFFFF0u;
 }
 
-static uint32_t dense_default(const gga_graph *g, const gga_opts *o)
+/* The list length from which a step records the next frontier as stamps.
+ * What a push costs grows with the edges behind the list, not with its
+ * length: on graphs that are not mesh-like a few thousand hub chunks hold
+ * millions of edges, and a rebuild's two passes read one byte per vertex, so
+ * lists are pushed only below 512 chunks (n / 8192 on larger graphs).  R-MAT,
+ * four sources each, device us at 512 / 2048 / 16384 / 65536 chunks: BFS on
+ * s22 618-655 / 609-656 / 627-721 / 626-841, on 1.5 M vertices unsplit
+ * 248-258 / 244-290 / 244-346 / 289-410, SSSP on s22 1793-2293 / 1787-2315 /
+ * 1779-2283 / 1900-2313, on 2^17 vertices 378-465 / 382-464 / 394-479 /
+ * 515-673 (128: within 1% of 512).  On meshes a chunk is a vertex of a few
+ * edges and short lists are followed within the step: a pure 1024^2 grid
+ * takes 8.0-9.9 ms at n / 64 and 8.8-11.2 at 512.  In the persistent kernel a
+ * rebuild costs two grid barriers that a push does not (8 us each): n / 64
+ * there too. */
+uint32_t gga_graph_default_dense(const gga_graph *g, int mode)
 {
-    return o->dense_min ? o->dense_min
-                        : g->tuned_dense ? g->tuned_dense : (g->n / 64u > 4096u ? g->n / 64u : 4096u);
+    const int low = mode == GGA_MODE_WORKLIST && !mesh_like(g);
+    const uint32_t lo = low ? 512u : 4096u, scaled = g->n / (low ? 8192u : 64u);
+    return scaled > lo ? scaled : lo;
+}
+
+static uint32_t dense_default(const gga_graph *g, const gga_opts *o, int mode)
+{
+    return o->dense_min ? o->dense_min : g->tuned_dense ? g->tuned_dense : gga_graph_default_dense(g, mode);
 }
 
 static int traverse(gga_graph *g, uint32_t src, int bfs, uint32_t *out, const gga_opts *user,
@@ -965,7 +985,7 @@ static int traverse(gga_graph *g, uint32_t src, int bfs, uint32_t *out, const gg
     p.epoch = g->epoch;
     gga_dev_graph dg = dev_graph(g);
     gga_dev_work dw = dev_work(g, inf);
-    dw.dense_min = dense_default(g, &o);
+    dw.dense_min = dense_default(g, &o, p.mode);
     dw.bmin = mesh_like(g) ? GGA_MESH_BMIN : 1u;
     /* near-far buckets: SSSP only (BFS levels are already one bucket per level) */
     if (delta) {
@@ -1095,7 +1115,7 @@ int gga_sssp_noalloc(gga_graph *g, uint32_t src, uint32_t *d_out, const gga_opts
         dw.cnt = (uint64_t *)(b + L.cnt);
         dw.tiles = (uint32_t *)(b + L.tiles);
         dw.qcap = g->C;
-        dw.dense_min = dense_default(g, &o);
+        dw.dense_min = dense_default(g, &o, p.mode);
         dw.bmin = mesh_like(g) ? GGA_MESH_BMIN : 1u;
         if (delta) {
             dw.last = (uint32_t *)(b + L.last);

@@ -155,7 +155,7 @@ int gga_tune(gga_graph *g, uint32_t src, uint32_t flags, gga_tune_result *r)
         }
     }
     o.grid = r->grid;
-    const uint32_t d0 = n / 64u > 4096u ? n / 64u : 4096u;
+    const uint32_t d0 = gga_graph_default_dense(g, GGA_MODE_WORKLIST);
     r->dense_min = d0;
     const uint32_t dcand[] = {d0 / 4u, d0 * 4u};
     for (size_t i = 0; i < 2; i++) {

@@ -198,7 +198,8 @@ typedef struct gga_opts {
     uint32_t grid;        /* PERSISTENT / WORKLIST grid in workgroups, 0 -> occupancy bound */
     uint32_t dense_min;   /* WORKLIST / PERSISTENT: a step whose list holds >= dense_min chunks
                              records the next frontier as step stamps + compaction instead of
-                             queue pushes; 0 -> max(4096, n / 64); 0xFFFFFFFF -> never */
+                             queue pushes; 0 -> max(4096, n / 64), WORKLIST on graphs that are not
+                             mesh-like max(512, n / 8192); 0xFFFFFFFF -> never */
     uint32_t pull_alpha;  /* gga_multi_bfs: a level runs bottom-up (pull over in-edges) when the
                              frontier's out-edges x pull_alpha > m; 0 -> 14; 0xFFFFFFFF -> never */
     uint32_t ms_layout;   /* gga_multi_sp: GGA_MS_* engine layout (0 -> GGA_MS_AUTO) */
