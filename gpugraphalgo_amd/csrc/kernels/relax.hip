@@ -70,11 +70,22 @@ constexpr uint32_t UNROLL = GGA_UNROLL; // edge slots per lane per round in expa
 #endif
 constexpr uint32_t LVL_UNROLL = GGA_LVL_UNROLL;   // the same in expand_level
 // Meshes: vertices a wave may follow past its batch within one step (0: off),
-// its LDS queue of them, and the largest degree followed.
+// its LDS queue of them, 16-vertex groups expanded per round, and the largest
+// degree followed.  SSSP on a pure 1024^2 grid / the 4096^2 grid with 0.5%
+// shortcuts, ms: queue of 256, one group 6.43 / 6.94, two 6.14 / 7.18; queue
+// of 512, one 6.45 / 6.40, two 6.23 / 6.33, four 6.34 / 6.34 (a short queue
+// overflows into the list); following 256 / 512 / 1024 / 2048 (queue of 512,
+// four groups): 6.94 / 6.38 / 6.34 / 6.80 and 6.55 / 6.42 / 6.34 / 6.92.
 #ifndef GGA_CONT
 #define GGA_CONT 1024
 #endif
-constexpr uint32_t CQ = 128;
+#ifndef GGA_CQ
+#define GGA_CQ 512
+#endif
+#ifndef GGA_CONT_GROUPS
+#define GGA_CONT_GROUPS 2
+#endif
+constexpr uint32_t CQ = GGA_CQ;
 constexpr uint32_t CONT_DEG = 16;
 // Only steps whose list is at most this many chunks follow: a thin wavefront
 // leaves most of the chip idle and each step is a chain of dependent loads;
@@ -98,16 +109,177 @@ struct ChunkDesc {
     bool valid = false;
 };
 
-template <bool OWN = true>
+// Edge arrays, lists and chunk descriptors are read with plain loads: a chunk's
+// run and its neighbours' share lines, and a thin mesh front comes back to the
+// same edges.  Against non-temporal loads: SSSP on R-MAT s22 2204 -> 2118 us,
+// on 2^17 vertices 442 -> 412, 32 engine lanes on R-MAT s20 5634 -> 5500, on
+// the 4096^2 grid 256 -> 246 ms.  The exception is a mesh batch's own edges,
+// which the wide steps of a large mesh stream once (4096^2 grid + 0.5%
+// shortcuts, SSSP: 6.86 ms non-temporal, 7.01 plain).
+template <bool STREAM>
+__device__ __forceinline__ uint32_t edge_load(const uint32_t *p) {
+    return STREAM ? stream_load(p) : *p;
+}
+
+template <bool CONT, bool OWN = true>
 __device__ __forceinline__ ChunkDesc load_chunk(const gga_dev_graph &g, uint32_t c, bool valid) {
     ChunkDesc d;
     d.valid = valid;
     if (valid) {
-        d.eb = stream_load(&g.cbeg[c]);
-        d.ee = stream_load(&g.cbeg[c + 1]);
-        if (OWN) d.own = stream_load(&g.cown[c]);
+        d.eb = edge_load<CONT>(&g.cbeg[c]);
+        d.ee = edge_load<CONT>(&g.cbeg[c + 1]);
+        if (OWN) d.own = edge_load<CONT>(&g.cown[c]);
     }
     return d;
+}
+
+// Lists x for the next step where `want`: the step's flag byte, or (queue
+// steps) the step stamp taken by exchange and a push.  PLAIN: every vertex
+// comes once, no stamp needed.  Whole-wave call.
+template <bool PLAIN, int OUT>
+__device__ __forceinline__ void list_vertex(const gga_dev_graph &g, const gga_dev_work &w, bool want, uint32_t x,
+                                            uint32_t it, uint32_t *pbuf, uint32_t &pcount, uint32_t *qout,
+                                            uint32_t *tail) {
+    if (OUT == OUT_FLAG) {
+        if (want) w.flag[x] = (uint8_t)it;
+    } else if (OUT == OUT_QUEUE) {
+        if (!PLAIN && want) want = (w.mark[x] != it) && (atomic_xchg_u32(&w.mark[x], it) != it);
+        const uint64_t mask = __ballot(want);
+        if (mask) {
+            const uint32_t nw = (uint32_t)__popcll(mask);
+            if (pcount + nw > PBUF) {
+                flush_pushes(g, pbuf, pcount, qout, tail, w.qcap, w.ctl);
+                pcount = 0;
+            }
+            if (want)
+                pbuf[pcount + __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32),
+                                                        __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u))] = x;
+            pcount += nw;
+            __builtin_amdgcn_wave_barrier();
+        }
+    }
+}
+
+// Queues (x, the distance this wave wrote there, its edge range) where `near`,
+// as far as the queue [qh, qt) has room; true on the lanes queued.  Whole-wave
+// call.
+__device__ __forceinline__ bool queue_near(bool near, uint32_t x, uint32_t d, uint32_t r0, uint32_t r1, uint4 *cq,
+                                           uint32_t qh, uint32_t &qt) {
+    const uint64_t qm = __ballot(near);
+    if (!qm) return false;
+    const uint32_t rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(qm >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)qm, 0u));
+    const uint32_t room = CQ - (qt - qh), nnear = (uint32_t)__popcll(qm);
+    const bool queued = near && rank < room;
+    if (queued) cq[(qt + rank) % CQ] = make_uint4(x, d, r0, r1);
+    qt += nnear < room ? nnear : room;
+    return queued;
+}
+
+// Meshes: a wave follows its own front within the step.  Each round expands
+// up to 64 vertices of the wave's queue -- vertices it lowered below the
+// threshold, each from the distance it wrote there, all edges -- until the
+// queue empties or GGA_CONT vertices were followed; what is then left, what
+// found the queue full and what has more than CONT_DEG edges is listed for
+// the next step.  So every improvement is either expanded at the distance
+// written or listed, as in a plain step, and distances converge to the same
+// fixed point.  A followed vertex records the distance it was expanded at
+// (near-far), as a listed one does when the next step expands it.
+//
+// What bounds it: the chain of dependent accesses of a round.  A queue entry
+// holds the vertex's edge range, fetched beside the atomic that lowered it,
+// and four neighbouring lanes take a vertex's edges (four at a time), so a
+// round needs no chunk lookup, scan or owner search: edge, dist[v], atomic
+// (it was chunk start, chunk bounds, edge, dist[v], atomic, behind a
+// 6-shuffle search).  With the queue of 512, SSSP: pure 1024^2 grid 8.9 -> 6.2
+// ms, a 100 x 77 grid 0.80 -> 0.60, 4096^2 with shortcuts 6.8 -> 6.3; BFS on
+// the pure 1024^2 / 4096^2 grid 4.1-4.6 -> 2.9-3.2 / 19-25 -> 13-18 ms.
+template <bool BFS, bool COUNT, int OUT>
+__device__ __forceinline__ void follow_front(const gga_dev_graph &g, const gga_dev_work &w, uint32_t it,
+                                             uint32_t *pbuf, uint32_t &pcount, uint32_t *qout, uint32_t *tail,
+                                             Counters &cnt, uint32_t thr, uint4 *cq, uint32_t qt) {
+    constexpr uint32_t PER = GGA_WAVE / 4u, G = GGA_CONT_GROUPS;   // vertices per group, groups per round
+    const uint32_t l = lane_id(), sub = l & 3u;
+    uint32_t *__restrict__ dist = w.dist;
+    const uint32_t inf = w.inf;
+    uint32_t qh = 0, budget = (uint32_t)GGA_CONT;
+    while (qh != qt) {
+        __builtin_amdgcn_wave_barrier();
+        const uint32_t avail = qt - qh;
+        // budget spent, or too little room for what a round may queue: the
+        // oldest entries are listed
+        const bool drain = budget == 0u || CQ - avail < GGA_WAVE * G;
+        uint32_t take = drain ? GGA_WAVE : PER * G;
+        take = take < avail ? take : avail;
+        take = drain || take < budget ? take : budget;
+        {
+            const uint4 q = cq[(qh + l) % CQ];
+            const bool mine = l < take, hub = q.w - q.z > CONT_DEG;
+            list_vertex<false, OUT>(g, w, mine && (drain || hub), q.x, it, pbuf, pcount, qout, tail);
+            if (w.last && mine && !drain && !hub) w.last[q.x] = q.y;
+            if (COUNT && !drain) {
+                cnt.edges += wave_last(wave_incl_scan(mine && !hub ? q.w - q.z : 0u));
+                cnt.chunks += __builtin_amdgcn_readfirstlane((uint32_t)__popcll(__ballot(mine && !hub && q.w != q.z)));
+            }
+        }
+        const uint32_t head = qh;
+        qh += take;
+        if (drain) continue;
+        budget -= take;
+        uint32_t eb[G], n[G], du[G], most = 0;
+#pragma unroll
+        for (uint32_t u = 0; u < G; u++) {
+            const uint32_t i = u * PER + (l >> 2);
+            const uint4 q = cq[(head + i) % CQ];
+            du[u] = q.y;
+            eb[u] = q.z;
+            n[u] = i < take && q.w - q.z <= CONT_DEG ? q.w - q.z : 0u;
+            most = n[u] > most ? n[u] : most;
+        }
+        __builtin_amdgcn_wave_barrier();   // the entries are read before the pushes below write the queue
+        for (uint32_t j = sub;; j += 4u) {
+            uint32_t v[G], alt[G], cur[G], r0[G], r1[G];
+            bool act[G];
+#pragma unroll
+            for (uint32_t u = 0; u < G; u++) {
+                if (u * PER >= take) break;
+                act[u] = j < n[u];
+                const uint32_t e = act[u] ? eb[u] + j : 0u;   // (the graph has an edge: slot 0 is in bounds)
+                v[u] = g.col[e];
+                alt[u] = du[u] + (BFS ? 1u : g.w[e]);
+            }
+#pragma unroll
+            for (uint32_t u = 0; u < G; u++) {
+                if (u * PER >= take) break;
+                cur[u] = dist[v[u]];
+            }
+#pragma unroll
+            for (uint32_t u = 0; u < G; u++) {
+                if (u * PER >= take) break;
+                act[u] = act[u] && alt[u] >= du[u] && alt[u] < inf && alt[u] < cur[u];
+                if (act[u]) {
+                    cur[u] = atomic_min_u32(&dist[v[u]], alt[u]);
+                    r0[u] = g.row[v[u]];
+                    r1[u] = g.row[v[u] + 1u];
+                }
+            }
+#pragma unroll
+            for (uint32_t u = 0; u < G; u++) {
+                if (u * PER >= take) break;
+                const bool imp = act[u] && alt[u] < cur[u];
+                if (COUNT) cnt.relax += __builtin_amdgcn_readfirstlane((uint32_t)__popcll(__ballot(imp)));
+                const bool queued = queue_near(imp && alt[u] < thr, v[u], alt[u], r0[u], r1[u], cq, qh, qt);
+                (void)queued;
+            }
+            if (__ballot(j + 4u < most) == 0ull) break;
+            // a vertex of more than four edges: room for the next four
+            while (CQ - (qt - qh) < GGA_WAVE * G) {
+                __builtin_amdgcn_wave_barrier();
+                const uint32_t x = cq[(qh + l) % CQ].x;
+                list_vertex<false, OUT>(g, w, l < qt - qh, x, it, pbuf, pcount, qout, tail);
+                qh += qt - qh < GGA_WAVE ? qt - qh : GGA_WAVE;
+            }
+        }
+    }
 }
 
 // Expand one batch of chunks (this lane's chunk d when d.valid).
@@ -117,20 +289,16 @@ __device__ __forceinline__ ChunkDesc load_chunk(const gga_dev_graph &g, uint32_t
 // deferred vertex is recognised by dist < last.  thr = 0xFFFFFFFF: plain
 // worklist (every improvement is listed).
 //
-// CONT (meshes), cq given (a short list), list steps: after the batch, the wave follows
-// its own wavefront -- each later round expands up to 64 vertices that this
-// wave lowered below the threshold in an earlier round, from the distance it
-// wrote there, all their edges (degree <= CONT_DEG), until its queue empties
-// or GGA_CONT vertices were followed.  Every such vertex is listed for the
-// next step all the same (stamp or flag), so the extra rounds only bring
-// improvements forward: distances converge to the same fixed point.  (BFS
-// then takes the stamp too: levels reached out of order can drop twice.)
+// CONT (meshes), cq given (a short list), list steps: the vertices that the
+// batch lowers below the threshold go to the wave's queue instead of the list,
+// and follow_front expands them within the step.  (BFS then takes the step
+// stamp too: levels reached out of order can drop twice.)
 template <bool BFS, bool COUNT, int OUT, bool CONT = false>
 __device__ __forceinline__ void expand_batch(const gga_dev_graph &g, const gga_dev_work &w,
                                              const ChunkDesc &d, uint32_t it, uint32_t *pbuf,
                                              uint32_t &pcount, uint32_t *qout, uint32_t *tail,
                                              bool &improved, Counters &cnt, uint2 *tab, uint32_t nown,
-                                             uint32_t thr = 0xFFFFFFFFu, uint32_t *cq = nullptr) {
+                                             uint32_t thr = 0xFFFFFFFFu, uint4 *cq = nullptr) {
     const uint32_t l = lane_id();
     uint32_t *__restrict__ dist = w.dist;
     const uint32_t inf = w.inf;
@@ -163,31 +331,7 @@ __device__ __forceinline__ void expand_batch(const gga_dev_graph &g, const gga_d
         if (w.last && go) w.last[own] = du;
     }
     constexpr bool cont = CONT && OUT != OUT_CHANGED;
-    uint32_t *const cqv = cq, *const cqa = cq + CQ;   // vertex, the distance this wave wrote
-    uint32_t qh = 0, qt = 0, budget = (cont && cq) ? (uint32_t)GGA_CONT : 0u;   // wave-uniform
-    // Lists x for the next step where `want`: the step's flag byte, or (queue
-    // steps) the step stamp taken by exchange and a push.  Whole-wave call.
-    auto list_vertex = [&](bool want, uint32_t x) {
-        if (OUT == OUT_FLAG) {
-            if (want) w.flag[x] = (uint8_t)it;
-        } else if (OUT == OUT_QUEUE) {
-            if ((!BFS || cont) && want) want = (w.mark[x] != it) && (atomic_xchg_u32(&w.mark[x], it) != it);
-            const uint64_t mask = __ballot(want);
-            if (mask) {
-                const uint32_t nw = (uint32_t)__popcll(mask);
-                if (pcount + nw > PBUF) {
-                    flush_pushes(g, pbuf, pcount, qout, tail, w.qcap, w.ctl);
-                    pcount = 0;
-                }
-                if (want)
-                    pbuf[pcount + __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32),
-                                                            __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u))] = x;
-                pcount += nw;
-                __builtin_amdgcn_wave_barrier();
-            }
-        }
-    };
-    for (;;) {
+    uint32_t qt = 0;   // vertices queued (wave-uniform)
     const uint32_t incl = wave_incl_scan(n);
     const uint32_t total = wave_last(incl);
     if (COUNT) {
@@ -211,6 +355,7 @@ __device__ __forceinline__ void expand_batch(const gga_dev_graph &g, const gga_d
     // chunk of a dozen edges, runs one group, not UNROLL.
     for (uint32_t base = 0; base < total; base += GGA_WAVE * UNROLL) {
         uint32_t e[UNROLL], ds[UNROLL], v[UNROLL], wt[UNROLL], cur[UNROLL], kk[UNROLL], own[UNROLL];
+        uint32_t r0[UNROLL] = {}, r1[UNROLL] = {};
         bool act[UNROLL];
         const uint32_t left = total - base;   // > 0
 #pragma unroll
@@ -240,8 +385,8 @@ __device__ __forceinline__ void expand_batch(const gga_dev_graph &g, const gga_d
 #pragma unroll
         for (uint32_t u = 0; u < UNROLL; u++) {
             if (u * GGA_WAVE >= left) break;
-            v[u] = stream_load(&g.col[e[u]]);
-            wt[u] = BFS ? 1u : stream_load(&g.w[e[u]]);
+            v[u] = edge_load<CONT>(&g.col[e[u]]);
+            wt[u] = BFS ? 1u : edge_load<CONT>(&g.w[e[u]]);
         }
 #pragma unroll
         for (uint32_t u = 0; u < UNROLL; u++) {
@@ -254,6 +399,10 @@ __device__ __forceinline__ void expand_batch(const gga_dev_graph &g, const gga_d
             bool imp = false;
             const uint32_t alt = ds[u] + wt[u];
             if (act[u] && alt >= ds[u] && alt < inf && alt < cur[u]) {
+                if (cont && cq) {   // the queue's row offsets, on their way beside the atomic
+                    r0[u] = g.row[v[u]];
+                    r1[u] = g.row[v[u] + 1u];
+                }
                 if (OUT == OUT_FLAG) {
                     (void)atomic_min_u32(&dist[v[u]], alt);  // result unused: no-return atomic
                     imp = true;
@@ -269,61 +418,12 @@ __device__ __forceinline__ void expand_batch(const gga_dev_graph &g, const gga_d
             }
             const bool near = imp && alt < thr;
             bool queued = false;
-            if (budget) {
-                // queue the vertex for a later round; listed now only when the queue is full
-                const uint64_t qm = __ballot(near);
-                if (qm) {
-                    const uint32_t rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(qm >> 32),
-                                                                    __builtin_amdgcn_mbcnt_lo((uint32_t)qm, 0u));
-                    const uint32_t room = CQ - (qt - qh), nnear = (uint32_t)__popcll(qm);
-                    queued = near && rank < room;
-                    if (queued) {
-                        cqv[(qt + rank) % CQ] = v[u];
-                        cqa[(qt + rank) % CQ] = alt;
-                    }
-                    qt += nnear < room ? nnear : room;
-                }
-            }
-            list_vertex(near && !queued, v[u]);
+            if (cont && cq) queued = queue_near(near, v[u], alt, r0[u], r1[u], cq, 0u, qt);
+            list_vertex<BFS && !cont, OUT>(g, w, near && !queued, v[u], it, pbuf, pcount, qout, tail);
         }
     }
-    if (qh == qt) break;
-    __builtin_amdgcn_wave_barrier();   // (also: this round's table reads precede the next round's writes)
-    if (budget == 0) {
-        // budget spent: what is still queued is listed for the next step
-        for (; qh != qt; qh += (qt - qh) < GGA_WAVE ? (qt - qh) : GGA_WAVE) {
-            const bool has = l < qt - qh;
-            list_vertex(has, has ? cqv[(qh + l) % CQ] : 0u);
-        }
-        break;
-    }
-    // the next round: up to 64 queued vertices, one per wave lane; a vertex
-    // with more than CONT_DEG edges is listed instead.  A followed vertex
-    // records the distance it was expanded at (near-far), as a listed one
-    // would when the next step expands it.
-    const uint32_t avail = qt - qh;
-    uint32_t take = avail < GGA_WAVE ? avail : GGA_WAVE;
-    take = take < budget ? take : budget;
-    eb = 0;
-    n = 0;
-    du = inf;
-    bool hub = false;
-    uint32_t x = 0;
-    if (l < take) {
-        const uint32_t slot = (qh + l) % CQ;
-        x = cqv[slot];
-        du = cqa[slot];
-        eb = g.cbeg[g.cstart[x]];
-        n = g.cbeg[g.cstart[x + 1]] - eb;
-        hub = n > CONT_DEG;
-        if (hub) n = 0;
-        else if (w.last) w.last[x] = du;
-    }
-    list_vertex(hub, x);
-    qh += take;
-    budget -= take;
-    nown = take;
-    }
+    if (cont && cq && qt != 0u)
+        follow_front<BFS, COUNT, OUT>(g, w, it, pbuf, pcount, qout, tail, cnt, thr, cq, qt);
 }
 
 // Expand one batch of a level-synchronous BFS step (w.lvl): every listed
@@ -379,7 +479,7 @@ __device__ __forceinline__ void expand_level(const gga_dev_graph &g, const gga_d
 #pragma unroll
         for (uint32_t u = 0; u < LVL_UNROLL; u++) {
             if (u * GGA_WAVE >= left) break;
-            v[u] = stream_load(&g.col[tab[own[u]] + kk[u]]);
+            v[u] = g.col[tab[own[u]] + kk[u]];
         }
 #pragma unroll
         for (uint32_t u = 0; u < LVL_UNROLL; u++) {
@@ -484,7 +584,7 @@ __global__ __launch_bounds__(BLOCK) void k_topo_step(gga_dev_graph g, gga_dev_wo
     uint32_t pcount = 0;
     Counters cnt;
     __shared__ uint2 s_tab[WAVES][GGA_WAVE];
-    expand_batch<BFS, COUNT, OUT_CHANGED>(g, w, load_chunk(g, valid ? (uint32_t)c : 0u, valid), 0u, nullptr,
+    expand_batch<BFS, COUNT, OUT_CHANGED>(g, w, load_chunk<false>(g, valid ? (uint32_t)c : 0u, valid), 0u, nullptr,
                                           pcount, nullptr, nullptr, improved, cnt,
                                           s_tab[__builtin_amdgcn_readfirstlane(threadIdx.x / GGA_WAVE)], GGA_WAVE);
     if (__ballot(improved) && lane_id() == 0) w.ctl[GGA_CTL_CHANGED] = 1u;  // *changed = true
@@ -504,7 +604,7 @@ __device__ __forceinline__ bool flag_step(const gga_dev_work &w, uint32_t nq) {
 template <bool BFS, bool COUNT, bool CONT>
 __device__ __forceinline__ void worklist_step(const gga_dev_graph &g, const gga_dev_work &w,
                                               uint32_t step, uint32_t nq, uint32_t it,
-                                              uint32_t *pbuf, uint32_t *cq, uint2 *tab, Counters &cnt) {
+                                              uint32_t *pbuf, uint4 *cq, uint2 *tab, Counters &cnt) {
     const uint32_t sout = (step + 1u) % 3u;
     const uint32_t *qin = (step & 1u) ? w.q1 : w.q0;
     uint32_t *qout = (step & 1u) ? w.q0 : w.q1;
@@ -535,7 +635,7 @@ __device__ __forceinline__ void worklist_step(const gga_dev_graph &g, const gga_
     bool dummy = false;
     const uint32_t alt = it - w.epoch + 1u;   // LVL: the level this step reaches
     const uint8_t stamp = level_stamp(alt);
-    uint32_t *const follow = (CONT && nq <= CONT_LIST) ? cq : nullptr;   // the continuation's queue
+    uint4 *const follow = (CONT && nq <= CONT_LIST) ? cq : nullptr;   // the continuation's queue
     // Software pipeline over the wave's batches b, b + waves, b + 2 waves...:
     // while a batch is expanded, the next batch's chunk descriptors and the
     // list entries of the one after it are already in flight, so a batch
@@ -544,7 +644,7 @@ __device__ __forceinline__ void worklist_step(const gga_dev_graph &g, const gga_
     auto entry = [&](uint64_t bb, bool &ok) -> uint32_t {
         const uint64_t idx = bb * bsz + l;
         ok = bb < nbatch && l < bsz && idx < nq;
-        return ok ? stream_load(&qin[idx]) : 0u;
+        return ok ? edge_load<CONT>(&qin[idx]) : 0u;
     };
     bool ok_next;
     uint32_t c_next;
@@ -553,12 +653,12 @@ __device__ __forceinline__ void worklist_step(const gga_dev_graph &g, const gga_
         bool ok0;
         const uint32_t c0 = entry(wid, ok0);
         c_next = entry((uint64_t)wid + waves, ok_next);
-        cur = load_chunk<!LVL>(g, c0, ok0);
+        cur = load_chunk<CONT, !LVL>(g, c0, ok0);
     }
     for (uint64_t b = wid; b < nbatch; b += waves) {
         bool ok_after;
         const uint32_t c_after = entry(b + 2ull * waves, ok_after);
-        const ChunkDesc nxt = load_chunk<!LVL>(g, c_next, ok_next);
+        const ChunkDesc nxt = load_chunk<CONT, !LVL>(g, c_next, ok_next);
         if (LVL && flags)
             expand_level<COUNT, OUT_FLAG>(g, w, cur, alt, stamp, pbuf, pcount, qout, tail, cnt,
                                           reinterpret_cast<uint32_t *>(tab), bsz);
@@ -685,7 +785,8 @@ __device__ __forceinline__ uint32_t hw_place() {
 template <bool BFS, bool COUNT, bool TL, uint32_t BS, bool CONT>
 __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(8, 8)))
 void k_wl_step(gga_dev_graph g, gga_dev_work w, uint32_t step, gga_wg_record *tl) {
-    __shared__ uint32_t s_pbuf[BS / GGA_WAVE][PBUF], s_cq[CONT ? BS / GGA_WAVE : 1][CONT ? 2 * CQ : 1];
+    __shared__ uint32_t s_pbuf[BS / GGA_WAVE][PBUF];
+    __shared__ uint4 s_cq[CONT ? BS / GGA_WAVE : 1][CONT ? CQ : 1];
     __shared__ uint2 s_tab[BS / GGA_WAVE][GGA_WAVE];
     uint64_t t0 = 0;
     if (TL && threadIdx.x == 0) t0 = wall_clock64();
@@ -934,7 +1035,8 @@ __global__ __launch_bounds__(BLOCK) void k_refill_write(gga_dev_graph g, gga_dev
 template <bool BFS, bool COUNT, bool CONT>
 __global__ __launch_bounds__(BLOCK) void k_persistent(gga_dev_graph g, gga_dev_work w,
                                                       uint32_t max_steps, uint64_t spin_ticks) {
-    __shared__ uint32_t s_pbuf[WAVES][PBUF], s_cq[CONT ? WAVES : 1][CONT ? 2 * CQ : 1];
+    __shared__ uint32_t s_pbuf[WAVES][PBUF];
+    __shared__ uint4 s_cq[CONT ? WAVES : 1][CONT ? CQ : 1];
     __shared__ uint2 s_tab[WAVES][GGA_WAVE];
     __shared__ uint32_t s_state[2];
     __shared__ uint32_t s_wave[WAVES], s_min[WAVES];
