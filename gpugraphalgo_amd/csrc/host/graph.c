@@ -19,7 +19,8 @@
 #include "gga_host.h"
 
 #ifndef GGA_MESH_BMIN
-#define GGA_MESH_BMIN 4u    /* chunks per wave batch on mesh-like graphs */
+#define GGA_MESH_BMIN 2u    /* chunks per wave batch on mesh-like graphs (2 / 4 / 8, SSSP: pure 1024^2 grid
+                               6.08 / 6.23 / 6.42 ms, 4096^2 with shortcuts 6.34 / 6.33 / 6.41) */
 #endif
 static int mesh_like(const gga_graph *g);
 
@@ -615,37 +616,39 @@ static int mesh_like(const gga_graph *g)
 /* AUTO: the tuned mode; else the worklist launches (full occupancy for a
  * few big steps), switching to the persistent kernel once a query on this
  * graph needed more than 256 steps (one launch and a grid barrier per step
- * then beat per-step launches and host checks: measured 2.3x on a pure
- * 1024^2 grid at ~2 400 steps, 0.8x on a shortcut 4096^2 grid at ~160). */
+ * then beat per-step launches and host checks) -- except on mesh-like graphs,
+ * where waves follow their front and a step is long: SSSP, worklist against
+ * persistent, 4.8 / 7.6 ms on a pure 1024^2 grid (80 steps), 13.9 / 23.2 on
+ * 2048^2 (184), 18.6 / 25.9 on 30 x 9000 (400); BFS equal. */
 static int choose_mode(const gga_graph *g, int bfs)
 {
     if (g->tuned_mode) return g->tuned_mode - 1;
-    return g->last_steps[bfs ? 1 : 0] > 256u ? GGA_MODE_PERSISTENT : GGA_MODE_WORKLIST;
+    return g->last_steps[bfs ? 1 : 0] > 256u && !mesh_like(g) ? GGA_MODE_PERSISTENT : GGA_MODE_WORKLIST;
 }
 
 /* Near-far width when opts leave it 0: the tuned one; else, for SSSP on
- * mesh-like graphs, 32 mean edge weights (pure 1024^2 grid: single source
- * 53 / 51 ms at 8 / 32 mean weights, 32-lane engine 350 / 283 ms); else off. */
+ * mesh-like graphs, 8 mean edge weights (at 4 / 8 / 16 / 32 mean weights, two
+ * sources each: pure 1024^2 grid 5.4-6.6 / 4.3-5.5 / 5.2-6.5 / 5.5-6.5 ms and
+ * 8 / 12 / 19 / 35 M edges inspected, 4096^2 grid with 0.5% shortcuts 5.6 /
+ * 5.2-5.3 / 5.4 / 6.2-6.3 ms); else off. */
 static uint32_t auto_delta(const gga_graph *g, int bfs)
 {
     if (g->tuned_delta) return g->tuned_delta == 0xFFFFFFFFu ? 0u : g->tuned_delta;
     if (bfs || !mesh_like(g)) return 0u;
-    const uint64_t d = 32ull * g->wmean;
+    const uint64_t d = 8ull * g->wmean;
     return d < 0xFFFFFFF0ull ? (uint32_t)d : 0xFFFFFFF0u;
 }
 
 uint32_t gga_graph_auto_delta(const gga_graph *g, int bfs) { return g ? auto_delta(g, bfs) : 0u; }
 
-/* The engines' default bucket width: half the single-source one (a tuned
- * width is kept).  With waves following their wavefronts, 32 lanes on the
- * 4096^2 grid converged in 312 ms at 16 mean weights against 345 at 32,
- * 473 at 64 (8 lanes: 157 / 165 / 168 ms), while single sources were
- * fastest at 32. */
+/* The engines' default bucket width: twice the single-source one (a tuned
+ * width is kept).  32 lanes on the 4096^2 grid converged in 312 ms at 16 mean
+ * weights against 345 at 32, 473 at 64 (8 lanes: 157 / 165 / 168 ms). */
 uint32_t gga_graph_engine_delta(const gga_graph *g)
 {
     if (!g) return 0u;
     const uint32_t d = auto_delta(g, 0);
-    return g->tuned_delta || d < 2u ? d : d / 2u;
+    return g->tuned_delta || d >= 0x7FFFFFF8u ? d : 2u * d;
 }
 int gga_graph_mesh_like(const gga_graph *g) { return g ? mesh_like(g) : 0; }
 

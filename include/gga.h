@@ -207,7 +207,7 @@ typedef struct gga_opts {
                              only while its distance is below the current threshold, the rest
                              wait until the threshold passes them (Davidson et al. 2014), so
                              fewer vertices are expanded more than once; 0 -> the tuned width
-                             (gga_tune), else 32 mean edge weights on mesh-like graphs (max
+                             (gga_tune), else 8 mean edge weights on mesh-like graphs (max
                              degree within 4x the mean + 8), else off; 0xFFFFFFFF -> off */
     /* WORKLIST instrumentation (both off when NULL) */
     gga_wg_record *timeline;    /* host buffer: grid records per step, steps in order */
@@ -346,7 +346,7 @@ int gga_ms_free(gga_ms *e);
 /* Near-far buckets per SSSP lane (as opts.delta for one source): a lane's
  * improvement at or beyond its threshold waits until a refill reaches it.
  * Set at creation from the graph (gga_tune's width, or 16 mean weights on
- * mesh-like graphs -- half the single-source default -- else off); delta 0 or
+ * mesh-like graphs -- twice the single-source default -- else off); delta 0 or
  * 0xFFFFFFFF turns it off.  gga_multi_sp uses the same default.  Only while
  * no lane runs; near-far engines run in step mode (GGA_MODE_WORKLIST).
  * +4 B per vertex (the far masks). */
