@@ -641,15 +641,11 @@ static uint32_t auto_delta(const gga_graph *g, int bfs)
 
 uint32_t gga_graph_auto_delta(const gga_graph *g, int bfs) { return g ? auto_delta(g, bfs) : 0u; }
 
-/* The engines' default bucket width: twice the single-source one (a tuned
- * width is kept).  32 lanes on the 4096^2 grid converged in 312 ms at 16 mean
- * weights against 345 at 32, 473 at 64 (8 lanes: 157 / 165 / 168 ms). */
-uint32_t gga_graph_engine_delta(const gga_graph *g)
-{
-    if (!g) return 0u;
-    const uint32_t d = auto_delta(g, 0);
-    return g->tuned_delta || d >= 0x7FFFFFF8u ? d : 2u * d;
-}
+/* The engines' default bucket width is the single-source one: a burst of 48
+ * queries on two R-MAT s16 and two 512^2 / 256 x 512 grids took 17.1 / 11.8 /
+ * 12.1 ms at 4 / 8 / 16 mean weights, 32 lanes on the 4096^2 grid 180 / 199 /
+ * 189-202 ms. */
+uint32_t gga_graph_engine_delta(const gga_graph *g) { return g ? auto_delta(g, 0) : 0u; }
 int gga_graph_mesh_like(const gga_graph *g) { return g ? mesh_like(g) : 0; }
 
 /* One query on a prepared workspace: dist init, the relax loop of the chosen

@@ -51,13 +51,17 @@ constexpr uint32_t FLAT_UNROLL = GGA_MS_FLAT_UNROLL;
 // a batch averaging at most GGA_MS_FLAT lanes per edge slot is flattened
 constexpr uint32_t PBUF = 256;                 // pushed vertices staged per wave before a flush
 // Mesh engines: (vertex, lane) pairs a wave may follow past its batch within
-// one step (0: off), the wave's LDS queue of them, and the largest degree
-// followed (a hub is left to the next step's chunks).
+// one step (0: off), the wave's LDS queue of them, 16-pair groups expanded per
+// round, and the largest degree followed (a hub is left to the next step's
+// chunks).
 #ifndef GGA_MS_CONT
 #define GGA_MS_CONT 1024
 #endif
 #ifndef GGA_MS_CQ
-#define GGA_MS_CQ 128
+#define GGA_MS_CQ 512
+#endif
+#ifndef GGA_MS_GROUPS
+#define GGA_MS_GROUPS 2
 #endif
 constexpr uint32_t CQ = GGA_MS_CQ;
 constexpr uint32_t CONT_DEG = 16;
@@ -140,11 +144,138 @@ __device__ __forceinline__ uint32_t wave_or(uint32_t x) {
 // ---------------------------------------------------------------- relax
 __device__ __forceinline__ bool ms_flag_step(const gga_dev_ms &ms, uint32_t nq) { return nq >= ms.dense_min; }
 
+// One (edge, lane) pair per wave lane: lowers D[v][s] to a where `pass` (the
+// guard held), defers an improvement at or beyond the lane's threshold, and
+// otherwise queues the pair for a later round (CONT, as far as the queue
+// [qh, qt) has room) or lists it.  True where the distance dropped.  Whole-wave
+// call.
+template <bool LM, bool CONT, class List>
+__device__ __forceinline__ bool relax_pair(const gga_dev_graph &g, const gga_dev_ms &ms, bool pass, uint32_t v,
+                                           uint32_t s, uint32_t a, uint32_t thr, uint4 *cq, uint32_t qh, uint32_t &qt,
+                                           const List &list) {
+    bool imp = false;
+    uint32_t r0 = 0, r1 = 0;
+    if (pass) {
+        const uint32_t old = atomic_min_u32(&ms.D[LM ? (uint64_t)s * g.n + v : (uint64_t)v * LANES + s], a);
+        if (CONT) {   // the edge range of the queue entry, on its way beside the atomic
+            r0 = g.row[v];
+            r1 = g.row[v + 1u];
+        }
+        imp = a < old;
+    }
+    const bool near = imp && a < thr;
+    if (imp && !near && ms.far) {
+        atomicOr(&ms.far[v], 1u << s);
+        // the tile's lane summary (bits are only added during a step, so a
+        // stale read shows a subset)
+        if (!(ms.tfar[v >> 6] & (1u << s))) atomicOr(&ms.tfar[v >> 6], 1u << s);
+    }
+    bool queued = false;
+    if (CONT) {
+        const bool fit = near && r1 - r0 <= CONT_DEG;   // a hub is listed
+        const uint64_t qm = __ballot(fit);
+        if (qm) {
+            const uint32_t rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(qm >> 32),
+                                                            __builtin_amdgcn_mbcnt_lo((uint32_t)qm, 0u));
+            const uint32_t room = CQ - (qt - qh), nfit = (uint32_t)__popcll(qm);
+            queued = fit && rank < room;
+            if (queued) cq[(qt + rank) % CQ] = make_uint4(v, a, r0, (r1 - r0) | s << 8);
+            qt += nfit < room ? nfit : room;
+        }
+    }
+    list(near && !queued, v, s);
+    return imp;
+}
+
+// Mesh engines: a wave follows its own front within the step.  Each round
+// expands up to 16 * GGA_MS_GROUPS queued (vertex, lane) pairs -- pairs this
+// wave lowered below the lane's threshold, each from the distance it wrote --
+// until the queue empties or GGA_MS_CONT pairs were followed; the rest is
+// listed for the next step, so each improvement is either expanded at its
+// value or listed, as in a plain step, and the fixed point is unchanged.  Four
+// neighbouring lanes take a pair's edges, whose range the entry holds: a round
+// is edge, D[v][s], atomic, with no lookup, scan or owner search before them
+// (it was chunk start, chunk bounds, edge, D, atomic).  32 lanes (16 BFS, 16
+// SSSP) on the pure 4096^2 grid 246 -> 189-202 ms, a burst of 48 queries on
+// two R-MAT s16 and two 512^2 / 256 x 512 grids 15.2 -> 12.1 ms; queue of 256
+// with one / two groups 198 / 213 ms and 12.6 / 12.3 ms.
+template <bool COUNT, bool LM, class List>
+__device__ __forceinline__ void follow_pairs(const gga_dev_graph &g, const gga_dev_ms &ms, uint32_t unit_word,
+                                             uint32_t thr_s, uint4 *cq, uint32_t qt, const List &list, Counters &cnt) {
+    constexpr uint32_t PER = GGA_WAVE / 4u, G = GGA_MS_GROUPS;
+    const uint32_t l = lane_id(), sub = l & 3u, inf = ms.inf;
+    uint32_t qh = 0, budget = (uint32_t)GGA_MS_CONT;
+    while (qh != qt) {
+        __builtin_amdgcn_wave_barrier();
+        const uint32_t avail = qt - qh;
+        const bool drain = budget == 0u || CQ - avail < GGA_WAVE * G;   // list the oldest pairs
+        uint32_t take = drain ? GGA_WAVE : PER * G;
+        take = take < avail ? take : avail;
+        take = drain || take < budget ? take : budget;
+        {
+            const uint4 q = cq[(qh + l) % CQ];
+            const bool mine = l < take;
+            const uint32_t m = 1u << ((q.w >> 8) & (LANES - 1u));
+            if (drain) list(mine, q.x, (q.w >> 8) & (LANES - 1u));
+            // followed from below the threshold: a far bit of the lane here is
+            // stale (no deferral below the threshold can follow it)
+            else if (mine && ms.far && (ms.far[q.x] & m)) atomicAnd(&ms.far[q.x], ~m);
+        }
+        const uint32_t head = qh;
+        qh += take;
+        if (drain) continue;
+        budget -= take;
+        uint32_t eb[G], n[G], du[G], sl[G], most = 0;
+#pragma unroll
+        for (uint32_t i = 0; i < G; i++) {
+            const uint32_t k = i * PER + (l >> 2);
+            const uint4 q = cq[(head + k) % CQ];
+            du[i] = q.y;
+            eb[i] = q.z;
+            n[i] = k < take ? q.w & 0xFFu : 0u;
+            sl[i] = (q.w >> 8) & (LANES - 1u);
+            most = n[i] > most ? n[i] : most;
+        }
+        __builtin_amdgcn_wave_barrier();   // the entries are read before the pushes below write the queue
+        for (uint32_t j = sub;; j += 4u) {
+            uint32_t v[G], a[G], dv[G];
+            bool act[G];
+#pragma unroll
+            for (uint32_t i = 0; i < G; i++) {
+                if (i * PER >= take) break;
+                act[i] = j < n[i];
+                const uint32_t e = act[i] ? eb[i] + j : 0u;   // (the graph has an edge: slot 0 is in bounds)
+                v[i] = g.col[e];
+                a[i] = du[i] + (((unit_word >> sl[i]) & 1u) ? 1u : g.w[e]);
+            }
+#pragma unroll
+            for (uint32_t i = 0; i < G; i++) {
+                if (i * PER >= take) break;
+                dv[i] = ms.D[LM ? (uint64_t)sl[i] * g.n + v[i] : (uint64_t)v[i] * LANES + sl[i]];
+            }
+#pragma unroll
+            for (uint32_t i = 0; i < G; i++) {
+                if (i * PER >= take) break;
+                const uint32_t thr = (uint32_t)__shfl(thr_s, (int)sl[i], GGA_WAVE);
+                const bool pass = act[i] && a[i] >= du[i] && a[i] < inf && a[i] < dv[i];
+                const bool imp = relax_pair<LM, true>(g, ms, pass, v[i], sl[i], a[i], thr, cq, qh, qt, list);
+                if (COUNT) {
+                    cnt.edges += (uint32_t)__popcll(__ballot(act[i]));
+                    cnt.relax += (uint32_t)__popcll(__ballot(imp));
+                }
+            }
+            if (__ballot(j + 4u < most) == 0ull) break;
+        }
+    }
+}
+
 // LM: lane-major layout (compile-time, so the vertex-major loop keeps its
-// unconditional full-line loads)
-template <bool COUNT, bool LM>
+// unconditional full-line loads).  CONT: mesh engines, whose waves follow
+// their fronts (cq: the wave's queue; kernels of their own, so that the
+// others keep their LDS and registers).
+template <bool COUNT, bool LM, bool CONT>
 __device__ __forceinline__ void ms_relax(const gga_dev_graph &g, const gga_dev_ms &ms, uint32_t step,
-                                         uint32_t nq, uint32_t *pbuf, uint32_t *nl, uint32_t *cq,
+                                         uint32_t nq, uint32_t *pbuf, uint32_t *nl, uint4 *cq,
                                          Counters &cnt) {
     const bool push = !ms_flag_step(ms, nq);
     uint32_t *qout = (step & 1u) ? ms.q0 : ms.q1;
@@ -168,8 +299,6 @@ __device__ __forceinline__ void ms_relax(const gga_dev_graph &g, const gga_dev_m
     // distance but is deferred (no mask bit, a far bit instead) until a refill
     // reaches it
     const uint32_t thr_s = ms.far ? ms.ctl[GGA_CTL_LTHR(s)] : 0xFFFFFFFFu;
-    const bool cont = GGA_MS_CONT > 0 && ms.bmin > 1u;
-    uint32_t *const cqv = cq, *const cqs = cq + CQ, *const cqa = cq + 2u * CQ;   // vertex, lane, distance
     // lanes the wave sets in next masks, ORed into its LDS word (no register
     // stays live across the loop for it)
     if (lane_id() == 0) *nl = 0u;
@@ -202,11 +331,11 @@ __device__ __forceinline__ void ms_relax(const gga_dev_graph &g, const gga_dev_m
         const bool valid = l < bsz && idx < nq;
         uint32_t eb = 0, ne = 0, u = 0, m = 0;
         if (valid) {
-            const uint32_t c = stream_load(&qin[idx]);
-            u = stream_load(&g.cown[c]);
+            const uint32_t c = qin[idx];
+            u = g.cown[c];
             m = mcur[u];
-            eb = stream_load(&g.cbeg[c]);
-            ne = m ? stream_load(&g.cbeg[c + 1]) - eb : 0u;
+            eb = g.cbeg[c];
+            ne = m ? g.cbeg[c + 1] - eb : 0u;
         }
         const uint32_t incl = wave_incl_scan(ne);
         const uint32_t total = wave_last(incl);
@@ -219,20 +348,7 @@ __device__ __forceinline__ void ms_relax(const gga_dev_graph &g, const gga_dev_m
         uint32_t pincl = wave_incl_scan(pairs);
         uint32_t ptotal = wave_last(pincl);
         if (ptotal <= GGA_MS_FLAT * total) {
-            // Round 0 walks the batch's owners.  On meshes (cont) each later
-            // round walks up to 64 (vertex, lane) pairs that this wave
-            // improved below the lane's threshold in an earlier round, from
-            // the distance it wrote there: the wave follows its own wavefront
-            // a few hops further within the step.  A queued pair is listed
-            // for the next step only if it is not followed (queue full,
-            // budget spent, degree above CONT_DEG); a followed pair had every
-            // edge relaxed from the distance written, so each improvement is
-            // either expanded at its value or listed, as in a plain step, and
-            // the fixed point -- the result -- is unchanged.
-            bool later = false;          // a continuation round (wave-uniform)
-            uint32_t from = 0;           // its pair's distance at the owner
-            uint32_t qh = 0, qt = 0, budget = cont ? (uint32_t)GGA_MS_CONT : 0u;
-            for (;;) {
+            uint32_t qt = 0;   // pairs queued (CONT; wave-uniform)
             const uint32_t pexcl = pincl - pairs;
             for (uint32_t base = 0; base < ptotal; base += GGA_WAVE * FLAT_UNROLL) {
                 uint32_t v[FLAT_UNROLL], wt[FLAT_UNROLL], du[FLAT_UNROLL], dv[FLAT_UNROLL], sl[FLAT_UNROLL];
@@ -251,9 +367,9 @@ __device__ __forceinline__ void ms_relax(const gga_dev_graph &g, const gga_dev_m
                     sl[i] = nth_set_bit(wave_bcast(m, j), r - eo * pcj);
                     const uint32_t e = wave_bcast(eb, j) + eo;
                     const uint32_t uu = wave_bcast(u, j);
-                    v[i] = stream_load(&g.col[e]);
-                    wt[i] = stream_load(&g.w[e]);
-                    du[i] = later ? wave_bcast(from, j) : D[LM ? (uint64_t)sl[i] * g.n + uu : (uint64_t)uu * LANES + sl[i]];
+                    v[i] = g.col[e];
+                    wt[i] = g.w[e];
+                    du[i] = D[LM ? (uint64_t)sl[i] * g.n + uu : (uint64_t)uu * LANES + sl[i]];
                 }
 #pragma unroll
                 for (uint32_t i = 0; i < FLAT_UNROLL; i++)
@@ -263,86 +379,15 @@ __device__ __forceinline__ void ms_relax(const gga_dev_graph &g, const gga_dev_m
                     const uint32_t thr = (uint32_t)__shfl(thr_s, (int)sl[i], GGA_WAVE);
                     const bool on = act[i] && du[i] < inf;
                     const uint32_t a = du[i] + (((unit_word >> sl[i]) & 1u) ? 1u : wt[i]);
-                    bool imp = false, first = false;
-                    if (on && a >= du[i] && a < inf && a < dv[i]) {
-                        const uint32_t old = atomic_min_u32(
-                            &D[LM ? (uint64_t)sl[i] * g.n + v[i] : (uint64_t)v[i] * LANES + sl[i]], a);
-                        imp = a < old;
-                    }
-                    const bool near = imp && a < thr;
-                    if (imp && !near && ms.far) {
-                        atomicOr(&ms.far[v[i]], 1u << sl[i]);
-                        // the tile's lane summary (bits are only added during
-                        // a step, so a stale read shows a subset)
-                        if (!(ms.tfar[v[i] >> 6] & (1u << sl[i]))) atomicOr(&ms.tfar[v[i] >> 6], 1u << sl[i]);
-                    }
-                    bool queued = false;
-                    if (budget) {
-                        // queue the pair for a later round; listed now only when the queue is full
-                        const uint64_t qm = __ballot(near);
-                        if (qm) {
-                            const uint32_t rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(qm >> 32),
-                                                                            __builtin_amdgcn_mbcnt_lo((uint32_t)qm, 0u));
-                            const uint32_t room = CQ - (qt - qh), nnear = (uint32_t)__popcll(qm);
-                            queued = near && rank < room;
-                            if (queued) {
-                                const uint32_t slot = (qt + rank) % CQ;
-                                cqv[slot] = v[i];
-                                cqs[slot] = sl[i];
-                                cqa[slot] = a;
-                            }
-                            qt += nnear < room ? nnear : room;
-                        }
-                    }
+                    const bool pass = on && a >= du[i] && a < inf && a < dv[i];
+                    const bool imp = relax_pair<LM, CONT>(g, ms, pass, v[i], sl[i], a, thr, cq, 0u, qt, list_pair);
                     if (COUNT) {
                         cnt.edges += (uint32_t)__popcll(__ballot(on));
                         cnt.relax += (uint32_t)__popcll(__ballot(imp));
                     }
-                    list_pair(near && !queued, v[i], sl[i]);
                 }
             }
-            if (qh == qt) break;
-            __builtin_amdgcn_wave_barrier();
-            if (budget == 0) {
-                // budget spent: what is still queued is listed for the next step
-                for (; qh != qt; qh += (qt - qh) < GGA_WAVE ? (qt - qh) : GGA_WAVE) {
-                    const bool has = l < qt - qh;
-                    const uint32_t slot = (qh + l) % CQ;
-                    list_pair(has, has ? cqv[slot] : 0u, has ? cqs[slot] : 0u);
-                }
-                break;
-            }
-            // the next round: up to 64 queued pairs, one per wave lane, each
-            // owning all edges of its vertex
-            const uint32_t avail = qt - qh;
-            uint32_t take = avail < GGA_WAVE ? avail : GGA_WAVE;
-            take = take < budget ? take : budget;
-            later = true;
-            u = 0; m = 0; eb = 0; from = 0;
-            uint32_t ne1 = 0, sq = 0;
-            bool hub = false;
-            if (l < take) {
-                const uint32_t slot = (qh + l) % CQ;
-                u = cqv[slot];
-                sq = cqs[slot];
-                m = 1u << sq;
-                from = cqa[slot];
-                eb = g.cbeg[g.cstart[u]];
-                ne1 = g.cbeg[g.cstart[u + 1]] - eb;
-                hub = ne1 > CONT_DEG;
-                if (hub) ne1 = 0;
-                // followed from below the threshold: a far bit of the lane
-                // here is stale (no deferral below the threshold can follow it)
-                else if (ms.far && (ms.far[u] & m)) atomicAnd(&ms.far[u], ~m);
-            }
-            list_pair(hub, u, sq);   // too many edges to follow: the next step expands it
-            qh += take;
-            budget -= take;
-            pc = l < take ? 1u : 0u;
-            pairs = pc * ne1;
-            pincl = wave_incl_scan(pairs);
-            ptotal = wave_last(pincl);
-            }
+            if (CONT && qt != 0u) follow_pairs<COUNT, LM>(g, ms, unit_word, thr_s, cq, qt, list_pair, cnt);
             continue;
         }
         // edge slot k goes to half (k & 1); slots past the end are clamped to
@@ -359,8 +404,8 @@ __device__ __forceinline__ void ms_relax(const gga_dev_graph &g, const gga_dev_m
                 const uint32_t e = wave_bcast(eb, j) + (kk - wave_bcast(excl, j));
                 const uint32_t uu = wave_bcast(u, j);
                 mm[i] = wave_bcast(m, j);
-                v[i] = stream_load(&g.col[e]);
-                wt[i] = stream_load(&g.w[e]);
+                v[i] = g.col[e];
+                wt[i] = g.w[e];
                 // vertex-major: the whole line comes in anyway, every lane loads;
                 // lane-major: only the lanes to relax gather their own word
                 if (LM) du[i] = ((mm[i] >> s) & 1u) ? D[(uint64_t)s * g.n + uu] : inf;
@@ -519,18 +564,20 @@ __global__ __launch_bounds__(64) void k_ms_seed(gga_dev_graph g, gga_dev_ms ms, 
     for (uint32_t k = 0; k < nch; k++) queue_store(q, pos + k, cs + k, ms.qcap, ms.ctl);
 }
 
-template <bool COUNT, bool LM>
+template <bool COUNT, bool LM, bool CONT>
 // Eight waves per SIMD (64 VGPRs): the compiler's own choice, 67 VGPRs, allows
 // seven; the eighth wave of memory-bound relax took 32 SSSP lanes on R-MAT s20
-// from 7.4 to 5.9 ms (grids unchanged).
-__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(8, 8)))
+// from 7.4 to 5.9 ms.  Mesh engines, bound by the chain of a front's rounds,
+// hold a queue of 8 KB per wave and get four.
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(CONT ? 4 : 8, 8)))
 void k_ms_step(gga_dev_graph g, gga_dev_ms ms, uint32_t step) {
-    __shared__ uint32_t s_pbuf[WAVES][PBUF], s_nl[WAVES], s_cq[WAVES][3 * CQ];
+    __shared__ uint32_t s_pbuf[WAVES][PBUF], s_nl[WAVES];
+    __shared__ uint4 s_cq[CONT ? WAVES : 1][CONT ? CQ : 1];
     const uint32_t nq = ms_len(ms, step);
     if (nq == 0) return;
     Counters cnt;
     const uint32_t wv = __builtin_amdgcn_readfirstlane(threadIdx.x / GGA_WAVE);   // wave-uniform
-    ms_relax<COUNT, LM>(g, ms, step, nq, s_pbuf[wv], &s_nl[wv], s_cq[wv], cnt);
+    ms_relax<COUNT, LM, CONT>(g, ms, step, nq, s_pbuf[wv], &s_nl[wv], s_cq[CONT ? wv : 0], cnt);
     publish_counters<COUNT>(ms, cnt);
 }
 
@@ -689,11 +736,12 @@ __global__ __launch_bounds__(BLOCK) void k_ms_tail(gga_dev_graph g, gga_dev_ms m
 
 // All steps in one cooperative launch: relax, then the compaction's count
 // and write passes, separated by grid barriers.  Step numbers continue from `step0`.
-template <bool COUNT, bool LM>
+template <bool COUNT, bool LM, bool CONT>
 __global__ __launch_bounds__(BLOCK) void k_ms_persistent(gga_dev_graph g, gga_dev_ms ms, uint32_t step0,
                                                          uint32_t max_steps, uint64_t spin_ticks) {
     __shared__ uint32_t s_pbuf[WAVES][PBUF];
-    __shared__ uint32_t s_wave[WAVES], s_state[2], s_nl[WAVES], s_cq[WAVES][3 * CQ];
+    __shared__ uint32_t s_wave[WAVES], s_state[2], s_nl[WAVES];
+    __shared__ uint4 s_cq[CONT ? WAVES : 1][CONT ? CQ : 1];
     uint32_t gen = 0;
     if (threadIdx.x == 0)
         gen = __hip_atomic_load(&ms.ctl[GGA_CTL_BARGEN], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -710,7 +758,7 @@ __global__ __launch_bounds__(BLOCK) void k_ms_persistent(gga_dev_graph g, gga_de
         __syncthreads();
         if (nq == 0 || err) break;
         const uint32_t wv = __builtin_amdgcn_readfirstlane(threadIdx.x / GGA_WAVE);
-        ms_relax<COUNT, LM>(g, ms, step, nq, s_pbuf[wv], &s_nl[wv], s_cq[wv], cnt);
+        ms_relax<COUNT, LM, CONT>(g, ms, step, nq, s_pbuf[wv], &s_nl[wv], s_cq[CONT ? wv : 0], cnt);
         grid_barrier(ms.ctl, gridDim.x, gen, spin_ticks);
         if (ms_flag_step(ms, nq)) {
             const ListOut o = ms_list_out(g, ms, step);
@@ -970,27 +1018,25 @@ extern "C" int ggak_ms_start(gga_dev_graph g, gga_dev_ms ms, uint32_t lanes, uin
 }
 
 template <bool COUNT, bool LM>
-static const void *step_fn() {
-    return reinterpret_cast<const void *>(&k_ms_step<COUNT, LM>);
+static const void *kernel_fn(int persistent, int cont) {
+    if (persistent)
+        return cont ? reinterpret_cast<const void *>(&k_ms_persistent<COUNT, LM, true>)
+                    : reinterpret_cast<const void *>(&k_ms_persistent<COUNT, LM, false>);
+    return cont ? reinterpret_cast<const void *>(&k_ms_step<COUNT, LM, true>)
+                : reinterpret_cast<const void *>(&k_ms_step<COUNT, LM, false>);
 }
-template <bool COUNT, bool LM>
-static const void *persistent_fn() {
-    return reinterpret_cast<const void *>(&k_ms_persistent<COUNT, LM>);
-}
-static const void *pick(int persistent, int count, uint32_t lm) {
-    static const void *const st[4] = {step_fn<false, false>(), step_fn<false, true>(), step_fn<true, false>(),
-                                      step_fn<true, true>()};
-    static const void *const pk[4] = {persistent_fn<false, false>(), persistent_fn<false, true>(),
-                                      persistent_fn<true, false>(), persistent_fn<true, true>()};
-    const int i = (count ? 2 : 0) | (lm ? 1 : 0);
-    return persistent ? pk[i] : st[i];
+// cont: the engine's graph is a mesh (bmin > 1) and following is compiled in
+static int use_cont(const gga_dev_ms &ms) { return GGA_MS_CONT > 0 && ms.bmin > 1u; }
+static const void *pick(int persistent, int count, uint32_t lm, int cont) {
+    if (count) return lm ? kernel_fn<true, true>(persistent, cont) : kernel_fn<true, false>(persistent, cont);
+    return lm ? kernel_fn<false, true>(persistent, cont) : kernel_fn<false, false>(persistent, cont);
 }
 
 extern "C" int ggak_ms_step(gga_dev_graph g, gga_dev_ms ms, uint32_t step, int count, uint32_t grid,
                             hipStream_t s) {
     if (grid == 0) return (int)hipErrorInvalidValue;
     void *args[] = {&g, &ms, &step};
-    hipError_t e = hipLaunchKernel(pick(0, count, ms.lane_major), dim3(grid), dim3(BLOCK), args, 0, s);
+    hipError_t e = hipLaunchKernel(pick(0, count, ms.lane_major, use_cont(ms)), dim3(grid), dim3(BLOCK), args, 0, s);
     if (e != hipSuccess) return (int)e;
     const uint32_t cg = compact_grid(g.n);
     if (ms.dense_min != 0xFFFFFFFFu) {   // push-only engines never rebuild from the masks
@@ -1005,7 +1051,7 @@ extern "C" int ggak_ms_step(gga_dev_graph g, gga_dev_ms ms, uint32_t step, int c
 extern "C" uint32_t ggak_ms_grid(int device, int persistent, int count) {
     int cus = 0, per = 0;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess) return 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, pick(persistent, count, 0), BLOCK, 0) != hipSuccess ||
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, pick(persistent, count, 0, 0), BLOCK, 0) != hipSuccess ||
         per <= 0)
         return 0;
     // cooperative launch: stay well under the co-residency measured for these
@@ -1023,7 +1069,7 @@ extern "C" int ggak_ms_persistent(gga_dev_graph g, gga_dev_ms ms, uint32_t step0
         khz = 100000;
     uint64_t spin_ticks = (uint64_t)spin_limit_ms * (uint64_t)khz;
     void *args[] = {&g, &ms, &step0, &max_steps, &spin_ticks};
-    hipError_t e = hipLaunchCooperativeKernel(pick(1, count, ms.lane_major), dim3(grid), dim3(BLOCK), args, 0, s);
+    hipError_t e = hipLaunchCooperativeKernel(pick(1, count, ms.lane_major, use_cont(ms)), dim3(grid), dim3(BLOCK), args, 0, s);
     if (e != hipSuccess) return (int)e;
     return launch_status();
 }

@@ -780,10 +780,11 @@ __device__ __forceinline__ uint32_t hw_place() {
 // which stores each block's clock64 span): each workgroup writes its start,
 // duration and placement to tl[blockIdx.x].  Every variant keeps eight waves
 // per SIMD (at most 64 VGPRs; the counting variants would otherwise take 62-65
-// and drop to seven): the relax is bound by the latency of its gathers.
+// and drop to seven): the relax is bound by the latency of its gathers.  (The
+// mesh variants' queues, 8 KB of LDS per wave, leave room for four.)
 // BS: workgroup size, 128, 256 or 512 threads (the tuner times all three).
 template <bool BFS, bool COUNT, bool TL, uint32_t BS, bool CONT>
-__global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(8, 8)))
+__global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(CONT ? 4 : 8, 8)))
 void k_wl_step(gga_dev_graph g, gga_dev_work w, uint32_t step, gga_wg_record *tl) {
     __shared__ uint32_t s_pbuf[BS / GGA_WAVE][PBUF];
     __shared__ uint4 s_cq[CONT ? BS / GGA_WAVE : 1][CONT ? CQ : 1];
@@ -874,10 +875,6 @@ struct DeferredUnder {
 __device__ __forceinline__ uint32_t sat_add(uint32_t a, uint32_t b) {
     const uint32_t s = a + b;
     return s < a ? 0xFFFFFFFFu : s;
-}
-
-__device__ __forceinline__ bool refill_needed(const gga_dev_work &w, uint32_t step) {
-    return w.last && w.ctl[GGA_CTL_TAIL((step + 1u) % 3u)] == 0u;
 }
 
 // count: chunk ids per tile under thr + delta, and the tile's smallest deferred distance

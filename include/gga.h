@@ -345,8 +345,8 @@ int gga_ms_create(gga_graph *g, uint32_t inf, uint32_t layout, gga_ms **out);
 int gga_ms_free(gga_ms *e);
 /* Near-far buckets per SSSP lane (as opts.delta for one source): a lane's
  * improvement at or beyond its threshold waits until a refill reaches it.
- * Set at creation from the graph (gga_tune's width, or 16 mean weights on
- * mesh-like graphs -- twice the single-source default -- else off); delta 0 or
+ * Set at creation from the graph (gga_tune's width, or 8 mean weights on
+ * mesh-like graphs, as for one source, else off); delta 0 or
  * 0xFFFFFFFF turns it off.  gga_multi_sp uses the same default.  Only while
  * no lane runs; near-far engines run in step mode (GGA_MODE_WORKLIST).
  * +4 B per vertex (the far masks). */

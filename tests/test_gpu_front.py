@@ -51,3 +51,24 @@ def test_followed_fronts(gpu, name, n, degrees, reach, mode):
                     got, st = dg.sssp(src, mode=mode, dense_min=dense_min, delta=delta)
                     np.testing.assert_array_equal(got, dist)
                     assert st["reached"] == int((dist < gga.INF).sum())
+
+
+@pytest.mark.parametrize("name,n,degrees,reach", CASES, ids=[c[0] for c in CASES])
+@pytest.mark.parametrize("layout", [1, 2], ids=["vertex", "lane"])
+def test_followed_fronts_of_engine_lanes(gpu, name, n, degrees, reach, layout):
+    g = spread_graph(n, degrees, reach, seed=n + 1)
+    ones = np.ones(g.m, dtype=np.uint32)
+    rng = np.random.default_rng(n)
+    srcs = rng.integers(0, n, 32).astype(np.uint32)
+    unit = 0x0F0F00FF                    # BFS lanes
+    want = [oracle.dijkstra(g.row_ptr, g.dst, ones if (unit >> i) & 1 else g.w, int(s)) for i, s in enumerate(srcs)]
+    with gga.DeviceGraph(g) as dg:
+        dg.split()
+        for k in (1, 32):
+            for dense_min in (0, 1, 0xFFFFFFFF):
+                for delta in (0, 1000, 0xFFFFFFFF):
+                    print(f"[gpu] {name} layout={layout} k={k} dense_min={dense_min} delta={delta}", flush=True)
+                    got, _ = dg.multi_sp(srcs[:k], bfs_lanes=unit & ((1 << k) - 1), ms_layout=layout,
+                                         dense_min=dense_min, delta=delta)
+                    for i in range(k):
+                        np.testing.assert_array_equal(got[i], want[i], err_msg=f"lane {i}")
