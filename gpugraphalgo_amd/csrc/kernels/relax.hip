@@ -28,8 +28,7 @@
 //     succeeds once per vertex).  Queued vertices are staged in wave-private
 //     LDS and flushed as chunk ids with one atomicAdd per 64 vertices.
 //   flag step (large frontier): fire-and-forget atomicMin and a plain store of
-//     the step's low byte into flag[v] (a byte array: a quarter of mark[]'s
-//     lines); then a three-pass compaction (count per tile, scan of tile
+//     a stamp into flag[v] (a byte array: a quarter of mark[]'s lines); then a three-pass compaction (count per tile, scan of tile
 //     counts, write) rebuilds the list from flag[] with no shared counter.
 // Device-scope atomics on MI355X execute past the per-XCD L2 and atomics on
 // one address serialize (~16 ns each), so no hot path funnels through a single
@@ -141,7 +140,7 @@ __device__ __forceinline__ void list_vertex(const gga_dev_graph &g, const gga_de
                                             uint32_t it, uint32_t *pbuf, uint32_t &pcount, uint32_t *qout,
                                             uint32_t *tail) {
     if (OUT == OUT_FLAG) {
-        if (want) w.flag[x] = (uint8_t)it;
+        if (want) w.flag[x] = 1;
     } else if (OUT == OUT_QUEUE) {
         if (!PLAIN && want) want = (w.mark[x] != it) && (atomic_xchg_u32(&w.mark[x], it) != it);
         const uint64_t mask = __ballot(want);
@@ -313,19 +312,16 @@ __device__ __forceinline__ void expand_batch(const gga_dev_graph &g, const gga_d
         // every edge at least as far -- expanding it now would only repeat
         // that work, so its chunks are left to the next step.
         bool again = false;
-        if (!BFS && OUT == OUT_FLAG) again = w.flag[own] == (uint8_t)it;
+        if (!BFS && OUT == OUT_FLAG) again = w.flag[own] != 0;
         if (!BFS && OUT == OUT_QUEUE) again = w.mark[own] == it;
-        // Near-far: only an owner below the threshold is expanded.  Every
-        // vertex listed by a stamp or a refill is; a flag byte repeats every
-        // 256 steps, so a deferred vertex (dist >= thr) can also match the
-        // step's byte and be listed.  Expanding it could go wrong: a
-        // concurrent improvement of it would be >= thr, deferred rather than
-        // stamped, and found later only through dist < last -- but with
-        // several chunks reading different distances, the chunk that saw the
-        // newer one may write last[] after the others, leaving dist == last
-        // while edges expanded with the older distance are never relaxed
-        // again.  Skipped, it is still deferred (dist < last) and a refill
-        // lists it when the threshold passes it.
+        // Near-far: only an owner below the threshold is expanded (every
+        // vertex listed by a stamp or a refill is).  Expanding a deferred one
+        // could go wrong: a concurrent improvement of it would be >= thr,
+        // deferred rather than stamped, and found later only through dist <
+        // last -- but with several chunks reading different distances, the
+        // chunk that saw the newer one may write last[] after the others,
+        // leaving dist == last while edges expanded with the older distance
+        // are never relaxed again.
         const bool go = du < inf && !again && du < thr;
         n = go ? ee - eb : 0u;
         if (w.last && go) w.last[own] = du;
@@ -543,7 +539,7 @@ __global__ __launch_bounds__(BLOCK) void k_query_init(gga_dev_graph g, gga_dev_w
     const uint64_t nth = (uint64_t)gridDim.x * blockDim.x;
     for (uint64_t v = tid; v < g.n; v += nth) w.dist[v] = (v == src) ? 0u : w.inf;
     for (uint64_t v = tid; v < g.n; v += nth)
-        w.flag[v] = w.lvl ? (v == src ? 255u : 0u) : (uint8_t)(epoch - 1u);
+        w.flag[v] = w.lvl && v == src ? 255u : 0u;
     if (w.last)
         for (uint64_t v = tid; v < g.n; v += nth) w.last[v] = w.inf;
     for (uint64_t i = tid; i < 4ull * GGA_CNT_SLOTS; i += nth) w.cnt[i] = 0;
@@ -678,26 +674,30 @@ __device__ __forceinline__ void worklist_step(const gga_dev_graph &g, const gga_
     if (pcount) flush_pushes(g, pbuf, pcount, qout, tail, w.qcap, w.ctl);
 }
 
-// A vertex belongs to the next list when the current (flag) step stamped it.
-// One byte per vertex, so the two passes over the stamps read n bytes, not
-// 4n.  The byte repeats every 256 steps of a query: a vertex last stamped 256
-// steps before is listed again -- one extra expansion at an unchanged
-// distance (none at all for a near-far vertex at or above the threshold,
-// see expand_batch), no effect on any result.
+// A vertex belongs to the next list when the current (flag) step stamped it
+// (a non-zero byte).  One byte per vertex, so the two passes over the stamps
+// read n bytes, not 4n; the write pass (CLEAR) takes the stamps back, each
+// cleared by the thread that lists its vertex, so that no later step meets
+// them.
+template <bool CLEAR>
 struct StampMarked {
-    const uint8_t *flag;
-    uint8_t it8;
+    uint8_t *flag;
     static constexpr bool vec8 = true;
-    __device__ __forceinline__ bool operator()(uint32_t v) const { return flag[v] == it8; }
-    // bit i: vertex v + i holds the stamp (v a multiple of 8)
+    __device__ __forceinline__ bool operator()(uint32_t v) const {
+        const bool m = flag[v] != 0;
+        if (CLEAR && m) flag[v] = 0;
+        return m;
+    }
+    // bit i: vertex v + i is stamped (v a multiple of 8)
     __device__ __forceinline__ uint32_t mark8(uint64_t v) const {
         const uint2 x = *reinterpret_cast<const uint2 *>(flag + v);
         uint32_t m = 0;
 #pragma unroll
         for (uint32_t i = 0; i < 4; i++) {
-            m |= ((x.x >> (8u * i)) & 0xFFu) == it8 ? 1u << i : 0u;
-            m |= ((x.y >> (8u * i)) & 0xFFu) == it8 ? 1u << (4u + i) : 0u;
+            m |= ((x.x >> (8u * i)) & 0xFFu) != 0u ? 1u << i : 0u;
+            m |= ((x.y >> (8u * i)) & 0xFFu) != 0u ? 1u << (4u + i) : 0u;
         }
+        if (CLEAR && m) *reinterpret_cast<uint2 *>(flag + v) = make_uint2(0u, 0u);
         return m;
     }
 };
@@ -719,7 +719,13 @@ struct LevelMarked {
         return true;
     }
     __device__ __forceinline__ uint32_t mark8(uint64_t v) const {
-        uint32_t m = StampMarked{flag, stamp}.mark8(v);
+        const uint2 x = *reinterpret_cast<const uint2 *>(flag + v);
+        uint32_t m = 0;
+#pragma unroll
+        for (uint32_t i = 0; i < 4; i++) {
+            m |= ((x.x >> (8u * i)) & 0xFFu) == stamp ? 1u << i : 0u;
+            m |= ((x.y >> (8u * i)) & 0xFFu) == stamp ? 1u << (4u + i) : 0u;
+        }
         if (level > 254u) {
 #pragma unroll
             for (uint32_t i = 0; i < 8; i++)
@@ -828,7 +834,7 @@ __global__ __launch_bounds__(BLOCK) void k_compact_count(gga_dev_graph g, gga_de
     uint32_t any = 0;
     for (uint32_t t = blockIdx.x; t < GGA_TILES(g.n); t += gridDim.x)
         any |= LVL ? compact_count_tile(o, g.n, t, level_marked<false>(w, it), s_wave)
-                   : compact_count_tile(o, g.n, t, StampMarked{w.flag, (uint8_t)it}, s_wave);
+                   : compact_count_tile(o, g.n, t, StampMarked<false>{w.flag}, s_wave);
     if (any && threadIdx.x == 0) w.ctl[GGA_CTL_LISTED((step + 1u) % 3u)] = 1u;
 }
 
@@ -973,7 +979,7 @@ __global__ __launch_bounds__(BLOCK) void k_compact_write(gga_dev_graph g, gga_de
         if (!w.last || w.ctl[GGA_CTL_LISTED(sout)] != 0u) {
             const uint32_t it = w.ctl[GGA_CTL_ITER(step % 3u)];
             if (LVL) compact_write_tiles(list_out(g, w, step), g.n, level_marked<true>(w, it), s_wave);
-            else compact_write_tiles(list_out(g, w, step), g.n, StampMarked{w.flag, (uint8_t)it}, s_wave);
+            else compact_write_tiles(list_out(g, w, step), g.n, StampMarked<true>{w.flag}, s_wave);
             return;
         }
     } else if (!w.last || w.ctl[GGA_CTL_TAIL(sout)] != 0u) {
@@ -1060,13 +1066,13 @@ __global__ __launch_bounds__(BLOCK) void k_persistent(gga_dev_graph g, gga_dev_w
             grid_barrier(w.ctl, gridDim.x, gen, spin_ticks);
             for (uint32_t t = blockIdx.x; t < GGA_TILES(g.n); t += gridDim.x) {
                 if (BFS && !CONT) compact_count_tile(o, g.n, t, level_marked<false>(w, it), s_wave);
-                else compact_count_tile(o, g.n, t, StampMarked{w.flag, (uint8_t)it}, s_wave);
+                else compact_count_tile(o, g.n, t, StampMarked<false>{w.flag}, s_wave);
             }
             grid_barrier(w.ctl, gridDim.x, gen, spin_ticks);
             // each workgroup sums the tile counts before its own tiles: no
             // serial scan between two more grid barriers
             if (BFS && !CONT) compact_write_tiles(o, g.n, level_marked<true>(w, it), s_wave);
-            else compact_write_tiles(o, g.n, StampMarked{w.flag, (uint8_t)it}, s_wave);
+            else compact_write_tiles(o, g.n, StampMarked<true>{w.flag}, s_wave);
         }
         grid_barrier(w.ctl, gridDim.x, gen, spin_ticks);
         // near-far: an empty next list is refilled from the deferred vertices,
