@@ -53,6 +53,7 @@ typedef struct gga_dev_work {
     uint32_t delta;      /* near-far bucket width (0: plain Bellman-Ford worklist) */
     uint32_t bmin;       /* fewest chunks per wave batch */
     uint32_t epoch;      /* step number of the query's first step */
+    uint32_t cap;        /* most steps of a query run one phase per launch */
     uint32_t lvl;        /* 1: BFS steps are levels (step epoch + k reaches level k + 1) */
 } gga_dev_work;
 
@@ -168,6 +169,14 @@ typedef struct gga_dev_msbfs {
 #define GGA_CTL_STEPS     (7u * GGA_CTL_LINE + 1u)      /* steps that had a non-empty list */
 #define GGA_CTL_ERR       (7u * GGA_CTL_LINE + 2u)      /* error bits (see GGA_DEVERR_*) */
 #define GGA_CTL_CNT       (8u * GGA_CTL_LINE)           /* 3 x uint64: edges, chunks, relaxations */
+/* single-source queries, one launch per phase: the phase that launch i ran
+ * (ring of three records), its step and that step's list length; phases run;
+ * wall clock at the query's start (u64) */
+#define GGA_CTL_PHASE(i)  (8u * GGA_CTL_LINE + 12u + 4u * ((i) % 3u))
+#define GGA_CTL_PSTEP(i)  (GGA_CTL_PHASE(i) + 1u)
+#define GGA_CTL_PLEN(i)   (GGA_CTL_PHASE(i) + 2u)
+#define GGA_CTL_PHASES    (8u * GGA_CTL_LINE + 24u)
+#define GGA_CTL_T0        (8u * GGA_CTL_LINE + 26u)
 #define GGA_CTL_BAR       (9u * GGA_CTL_LINE)           /* grid barrier: arrivals of group leaders */
 #define GGA_CTL_BARGEN    (10u * GGA_CTL_LINE)          /* grid barrier generation */
 #define GGA_CTL_RED       (11u * GGA_CTL_LINE)          /* reductions: 4 x uint64 scratch */
@@ -191,6 +200,53 @@ typedef struct gga_dev_msbfs {
 /* multi-source engine: lanes relaxing with weight 1; kept on the device (not a
  * kernel argument) so that steps replayed from a captured graph see restarts */
 #define GGA_CTL_UNIT      (7u * GGA_CTL_LINE + 12u)
+
+/* What a query's pinned read-back area holds behind the control words: the
+ * reach partials of each workgroup (reached, out-degree sum; u64), then the
+ * wall clock at the query's start and end (u64). */
+#define GGA_FIN_BLOCKS    512u
+#define GGA_FIN_PART      GGA_CTL_WORDS                          /* word offset, 8-byte aligned */
+#define GGA_FIN_CLOCK     (GGA_FIN_PART + 4u * GGA_FIN_BLOCKS)
+#define GGA_FIN_WORDS     (GGA_FIN_CLOCK + 4u)
+
+/* Phases of a single-source worklist query (kernels/relax.hip, k_wl_phase). */
+enum { GGA_PH_START, GGA_PH_RELAX, GGA_PH_COUNT, GGA_PH_WRITE, GGA_PH_RCOUNT, GGA_PH_RWRITE, GGA_PH_DONE,
+       GGA_PH_CAPPED };
+#ifdef __HIPCC__
+#define GGA_HOSTDEV __host__ __device__
+#else
+#define GGA_HOSTDEV
+#endif
+/* The phase of launch `launch` and its step, from the record of the launch
+ * before and the words that launch left: every workgroup of a launch computes
+ * it for itself (no launch changes a word it reads here), and the host knows
+ * from a read-back whether the query is done.  A queue step is one launch, a
+ * flag step three (relax, count, write), an empty list of a near-far query
+ * two more (count the deferred vertices, list them; a threshold jump that
+ * lists nothing is followed by an empty step).  No step past `cap` steps
+ * begins: the query ends in GGA_PH_CAPPED instead. */
+static inline GGA_HOSTDEV uint32_t gga_next_phase(const uint32_t *ctl, uint32_t launch, uint32_t dense_min,
+                                                  int near_far, uint32_t cap, uint32_t *step)
+{
+    const uint32_t prev = ctl[GGA_CTL_PHASE(launch + 2u)], s = ctl[GGA_CTL_PSTEP(launch + 2u)];
+    const uint32_t out = (s + 1u) % 3u;
+    uint32_t next;
+    *step = s;
+    if (prev == GGA_PH_START) return GGA_PH_RELAX;
+    if (prev == GGA_PH_RCOUNT) return GGA_PH_RWRITE;
+    if (prev == GGA_PH_DONE || prev == GGA_PH_CAPPED) return prev;
+    if (prev == GGA_PH_RELAX && ctl[GGA_CTL_PLEN(launch + 2u)] >= dense_min) return GGA_PH_COUNT;
+    if (prev == GGA_PH_COUNT && ctl[GGA_CTL_LISTED(out)] != 0u) return GGA_PH_WRITE;
+    if (prev == GGA_PH_COUNT) next = near_far ? GGA_PH_RCOUNT : GGA_PH_DONE;
+    else if (ctl[GGA_CTL_TAIL(out)] != 0u) next = GGA_PH_RELAX;
+    else if (prev == GGA_PH_RWRITE) next = ctl[GGA_CTL_FAR] != 0u ? GGA_PH_RELAX : GGA_PH_DONE;
+    else next = near_far ? GGA_PH_RCOUNT : GGA_PH_DONE;
+    if (next == GGA_PH_RELAX) {
+        *step = s + 1u;
+        if (s + 1u >= cap) return GGA_PH_CAPPED;
+    }
+    return next;
+}
 
 #define GGA_DEVERR_SPIN   1u   /* barrier spin limit hit */
 #define GGA_DEVERR_QFULL  2u   /* worklist overflow (cannot happen with de-duplication) */

@@ -65,6 +65,12 @@ int ggak_compact(gga_dev_graph g, gga_dev_work w, uint32_t phase, hipStream_t s)
 /* Near-far (w.last != NULL): after ggak_compact(phase), when the next list is
  * empty, lists the deferred vertices under the next threshold. */
 int ggak_refill(gga_dev_graph g, gga_dev_work w, uint32_t phase, hipStream_t s);
+/* Launch `launch` (0, 1, ...) of a query run one phase per launch (256 threads; w.last: near-far). */
+int ggak_wl_phase(gga_dev_graph g, gga_dev_work w, uint32_t launch, int bfs, uint32_t grid, hipStream_t s);
+/* Control words, reach partials (*blocks rows of reached, out-degree sum) and
+ * the clock at the query's start and now -> host, GGA_FIN_WORDS words of
+ * pinned memory by its device address. */
+int ggak_finish(gga_dev_graph g, gga_dev_work w, uint32_t *host, uint32_t *blocks, hipStream_t s);
 /* Occupancy-bound grid (workgroups of `block` threads) for the worklist
  * kernel, or for the persistent kernel (always 256 threads); 0 on error. */
 uint32_t ggak_wl_grid(int device, int persistent, int bfs, int count, uint32_t block);

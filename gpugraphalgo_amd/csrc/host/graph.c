@@ -44,7 +44,9 @@ struct gga_graph {
     uint8_t *d_flag;
     uint64_t *d_cnt;
     uint32_t qcap;
-    uint32_t *h_pin;          /* pinned: GGA_CTL_WORDS words */
+    uint32_t *h_pin;          /* pinned: GGA_FIN_WORDS words (the control words first) */
+    uint32_t *d_pin;          /* its device address */
+    uint32_t clock_khz;       /* device wall clock */
     uint32_t epoch;           /* step number of the next query's first step (mark[] stamps are below it) */
     int mark_dirty;           /* mark[] holds stamps of unknown step numbers: refill before the next query */
     int have_result;
@@ -57,6 +59,7 @@ struct gga_graph {
     uint32_t tuned_delta;
     int32_t tuned_mode;          /* 0: none; else GGA_MODE_* + 1 */
     uint32_t last_steps[2];      /* [bfs] relax steps of the last query (AUTO's evidence) */
+    uint32_t last_phases[2];     /* [bfs] phases of the last query run one phase per launch */
     uint32_t wmean;              /* mean edge weight, rounded up (>= 1) */
     uint32_t *d_last, *d_tmin;   /* near-far state (allocated on first use) */
     void *msbfs;              /* transposed graph + state of gga_multi_bfs (msbfs.c) */
@@ -160,6 +163,7 @@ static gga_dev_work dev_work(const gga_graph *g, uint32_t inf)
     w.delta = 0;
     w.bmin = 1;
     w.epoch = 0;
+    w.cap = 0xFFFFFFFFu;
     w.lvl = 0;
     return w;
 }
@@ -242,7 +246,14 @@ static int graph_create(uint32_t n, uint32_t m, const uint32_t *row_ptr, const u
     HIP_TRY(hipSetDevice(device));
     HIP_TRY(hipStreamCreateWithFlags(&g->stream, hipStreamNonBlocking));
     for (int i = 0; i < 4; i++) HIP_TRY(hipEventCreate(&g->ev[i]));
-    HIP_TRY(hipHostMalloc((void **)&g->h_pin, 4ull * GGA_CTL_WORDS, hipHostMallocDefault));
+    HIP_TRY(hipHostMalloc((void **)&g->h_pin, 4ull * GGA_FIN_WORDS, hipHostMallocDefault));
+    HIP_TRY(hipHostGetDevicePointer((void **)&g->d_pin, g->h_pin, 0));
+    {
+        int khz = 0;
+        if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, device) != hipSuccess || khz <= 0)
+            khz = 100000;   /* 100 MHz */
+        g->clock_khz = (uint32_t)khz;
+    }
     if ((rc = dmalloc(g, (void **)&g->d_row, 4ull * ((uint64_t)n + 1)))) goto fail;
     if ((rc = dmalloc(g, (void **)&g->d_col, 4ull * m))) goto fail;
     if ((rc = dmalloc(g, (void **)&g->d_w, 4ull * m))) goto fail;
@@ -679,9 +690,14 @@ static int run_query(gga_graph *g, gga_dev_graph dg, gga_dev_work dw, const quer
     dw.epoch = p->epoch;
     dw.lvl = mode != GGA_MODE_TOPO && ggak_level_sync(dw, bfs) ? 1u : 0u;
     int ended = 0;   /* reach pass and control words already fetched */
+    uint32_t fin = 0;   /* phase launches: rows of reach partials in the read-back area */
+    /* one launch per phase, unless the query is instrumented (each launch of
+     * a step timed, recorded or compared) or tuned to another workgroup size */
+    const int phased = mode == GGA_MODE_WORKLIST && !count && wl_block(g, o) == 256u &&
+                       !(own && (o->timeline || o->conv_rows));
     *adv = 0;
 
-    HIP_TRY(hipEventRecord(g->ev[0], g->stream));              /* bfs_sssp.cu:350 */
+    if (!phased) HIP_TRY(hipEventRecord(g->ev[0], g->stream)); /* bfs_sssp.cu:350 */
     K_TRY(ggak_query_init(dg, dw, p->src, p->epoch, g->stream));
     if (mode == GGA_MODE_TOPO) {
         /* the reference's loop: changed = false; relax; read changed (bfs_sssp.cu:372-468) */
@@ -733,6 +749,36 @@ static int run_query(gga_graph *g, gga_dev_graph dg, gga_dev_work dw, const quer
         const uint32_t per = o->sync_every ? o->sync_every : 8u;
         const uint32_t prev = g->last_steps[bfs ? 1 : 0];
         uint32_t nb = o->sync_every ? per : (prev ? (prev < 31u ? prev + 1u : 32u) : per);
+        if (phased) {
+            /* the step cap falls where the step launches look at it: after
+             * nb steps and then every `per` */
+            uint64_t cap = nb;
+            if (max_iters > nb) cap += ((uint64_t)max_iters - nb + per - 1u) / per * per;
+            dw.cap = cap < 0xFFFFFFFFull ? (uint32_t)cap : 0xFFFFFFFFu;
+            /* launches per host check: two more than the phases of the last
+             * query on this graph, 20 on the first */
+            const uint32_t prevp = g->last_phases[bfs ? 1 : 0];
+            uint32_t nl = o->sync_every ? 3u * o->sync_every : prevp ? (prevp < 254u ? prevp + 2u : 256u) : 20u;
+            uint32_t launch = 0, step = 0;
+            for (;;) {
+                for (uint32_t k = 0; k < nl; k++)
+                    K_TRY(ggak_wl_phase(dg, dw, launch++, bfs, grid, g->stream));
+                K_TRY(ggak_finish(dg, dw, g->d_pin, &fin, g->stream));
+                HIP_TRY(hipStreamSynchronize(g->stream));
+                s->launches += nl;
+                const uint32_t next =
+                    gga_next_phase(g->h_pin, launch, dw.dense_min, dw.last != NULL, dw.cap, &step);
+                if (next == GGA_PH_DONE) break;
+                if (next == GGA_PH_CAPPED) {
+                    rc = GGA_ETIMEDOUT;
+                    gga_set_error("worklist mode: %u steps without convergence", dw.cap);
+                    goto fail;
+                }
+                if (!o->sync_every) nl = 24u;
+            }
+            g->last_phases[bfs ? 1 : 0] = g->h_pin[GGA_CTL_PHASES];
+            ended = 1;
+        } else {
         if (tev && (rc = ensure_kev(g, 3 * (nb > per ? nb : per)))) goto fail;
         /* instrumentation buffers (freed below, also on failure) */
         const uint32_t tl_steps = own && o->timeline && o->timeline_cap >= grid ? o->timeline_cap / grid : 0u;
@@ -812,6 +858,7 @@ static int run_query(gga_graph *g, gga_dev_graph dg, gga_dev_work dw, const quer
             free(h);
             s->conv_steps = ns;
         }
+        }
     } else { /* GGA_MODE_PERSISTENT */
         const uint32_t maxg = wl_grid(g, 1, bfs, count, 256u);
         /* half the grid once a query on this graph ran more than 1024 steps:
@@ -847,7 +894,12 @@ static int run_query(gga_graph *g, gga_dev_graph dg, gga_dev_work dw, const quer
         HIP_TRY(hipMemcpyAsync(g->h_pin, dw.ctl, 4ull * GGA_CTL_WORDS, hipMemcpyDeviceToHost, g->stream));
         HIP_TRY(hipStreamSynchronize(g->stream));
     }
-    HIP_TRY(hipEventElapsedTime(&s->time_ms, g->ev[0], g->ev[1]));
+    if (fin) {
+        const uint64_t *t = (const uint64_t *)(g->h_pin + GGA_FIN_CLOCK);
+        s->time_ms = (float)((double)(t[1] - t[0]) / g->clock_khz);
+    } else {
+        HIP_TRY(hipEventElapsedTime(&s->time_ms, g->ev[0], g->ev[1]));
+    }
     {
         const uint32_t *c = g->h_pin;
         for (uint32_t i = 0; i < 3; i++) {
@@ -875,13 +927,23 @@ static int run_query(gga_graph *g, gga_dev_graph dg, gga_dev_work dw, const quer
                 }
             }
         }
-        const uint64_t *c64 = (const uint64_t *)(c + GGA_CTL_CNT);
-        s->edges_inspected = c64[0];
-        s->chunks_expanded = c64[1];
-        s->relaxations = c64[2];
-        const uint64_t *r64 = (const uint64_t *)(c + GGA_CTL_RED);
-        s->reached = (uint32_t)r64[0];
-        s->m_reach = r64[1];
+        if (fin) {
+            const uint64_t *part = (const uint64_t *)(c + GGA_FIN_PART);
+            uint64_t reached = 0;
+            for (uint32_t i = 0; i < fin; i++) {
+                reached += part[2u * i];
+                s->m_reach += part[2u * i + 1u];
+            }
+            s->reached = (uint32_t)reached;
+        } else {
+            const uint64_t *c64 = (const uint64_t *)(c + GGA_CTL_CNT);
+            s->edges_inspected = c64[0];
+            s->chunks_expanded = c64[1];
+            s->relaxations = c64[2];
+            const uint64_t *r64 = (const uint64_t *)(c + GGA_CTL_RED);
+            s->reached = (uint32_t)r64[0];
+            s->m_reach = r64[1];
+        }
     }
     s->ktime_ms = ktime;
     s->sktime_ms = 0.f;

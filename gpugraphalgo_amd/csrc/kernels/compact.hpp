@@ -175,11 +175,14 @@ __device__ __forceinline__ void compact_scan(const ListOut &o, uint32_t n, uint3
 // their own wave they made that wave the whole pass's long pole (62 of the
 // 154 us of an R-MAT s22 SSSP query's list writes, in one pass).  All threads of
 // the workgroup must call this (it synchronises).
+// `stage`: CSTAGE words of LDS (the caller's, so that a kernel which also holds
+// other buffers can lend one of them).
 constexpr uint32_t CBIG = 256;   // long runs staged per round
+constexpr uint32_t CSTAGE = 3u * CBIG + 1u;
 __device__ __forceinline__ void write_items(const ListOut &o, const uint32_t *cs, const uint32_t *nch,
-                                            uint32_t pos) {
-    __shared__ uint32_t s_bpos[CBIG], s_bcs[CBIG], s_bcnt[CBIG];
-    __shared__ uint32_t s_nb;
+                                            uint32_t pos, uint32_t *stage) {
+    uint32_t *const s_bpos = stage, *const s_bcs = stage + CBIG, *const s_bcnt = stage + 2u * CBIG;
+    uint32_t &s_nb = stage[3u * CBIG];
     uint32_t bpos[CITEMS];
     uint32_t pending = 0;   // bit i: item i is a long run not staged yet
 #pragma unroll
@@ -225,11 +228,11 @@ __device__ __forceinline__ void write_items(const ListOut &o, const uint32_t *cs
 // pass 3, one tile: write
 template <class Marked>
 __device__ __forceinline__ void compact_write_tile(const ListOut &o, uint32_t n, uint32_t t, const Marked &marked,
-                                                   uint32_t *s_wave) {
+                                                   uint32_t *s_wave, uint32_t *stage) {
     uint32_t cs[CITEMS], nch[CITEMS], excl;
     const uint32_t mine = tile_items(o, n, t, marked, cs, nch);
     block_excl_scan(mine, excl, s_wave);
-    write_items(o, cs, nch, o.tiles[t] + excl);
+    write_items(o, cs, nch, o.tiles[t] + excl, stage);
 }
 
 // Passes 2 and 3 in one launch (every workgroup of the grid calls this):
@@ -240,7 +243,7 @@ __device__ __forceinline__ void compact_write_tile(const ListOut &o, uint32_t n,
 // the last tile stores the list length.
 template <class Marked>
 __device__ __forceinline__ void compact_write_tiles(const ListOut &o, uint32_t n, const Marked &marked,
-                                                    uint32_t *s_wave) {
+                                                    uint32_t *s_wave, uint32_t *stage) {
     const uint32_t ntiles = (uint32_t)GGA_TILES((uint64_t)n);
     uint32_t off = 0, upto = 0;   // off = tiles[0] + ... + tiles[upto - 1]
     for (uint32_t t = blockIdx.x; t < ntiles; t += gridDim.x) {
@@ -251,7 +254,7 @@ __device__ __forceinline__ void compact_write_tiles(const ListOut &o, uint32_t n
         uint32_t cs[CITEMS], nch[CITEMS], excl;
         const uint32_t mine = tile_items(o, n, t, marked, cs, nch);
         const uint32_t tot = block_excl_scan(mine, excl, s_wave);
-        write_items(o, cs, nch, off + excl);
+        write_items(o, cs, nch, off + excl, stage);
         if (t == ntiles - 1u && threadIdx.x == 0) *o.tail = off + tot;
     }
 }

@@ -593,10 +593,10 @@ __global__ __launch_bounds__(CBLOCK) void k_ms_count(gga_dev_graph g, gga_dev_ms
 }
 
 __global__ __launch_bounds__(CBLOCK) void k_ms_write(gga_dev_graph g, gga_dev_ms ms, uint32_t step) {
-    __shared__ uint32_t s_wave[CBLOCK / GGA_WAVE];
+    __shared__ uint32_t s_wave[CBLOCK / GGA_WAVE], s_stage[CSTAGE];
     const uint32_t nq = ms_len(ms, step);
     if (nq == 0 || !ms_flag_step(ms, nq)) return;
-    compact_write_tiles(ms_list_out(g, ms, step), g.n, MaskMarked{ms_mnxt(ms, step)}, s_wave);
+    compact_write_tiles(ms_list_out(g, ms, step), g.n, MaskMarked{ms_mnxt(ms, step)}, s_wave, s_stage);
 }
 
 // ---- the tail of a step: the finish pass, then (near-far) the refill of
@@ -766,7 +766,7 @@ __global__ __launch_bounds__(BLOCK) void k_ms_persistent(gga_dev_graph g, gga_de
             for (uint32_t t = blockIdx.x; t < GGA_TILES(g.n); t += gridDim.x) compact_count_tile(o, g.n, t, mk, s_wave);
             grid_barrier(ms.ctl, gridDim.x, gen, spin_ticks);
             // each workgroup sums the tile counts before its own tiles
-            compact_write_tiles(o, g.n, mk, s_wave);
+            compact_write_tiles(o, g.n, mk, s_wave, &s_pbuf[0][0]);
             grid_barrier(ms.ctl, gridDim.x, gen, spin_ticks);
         }
         ms_finish(g, ms, step);

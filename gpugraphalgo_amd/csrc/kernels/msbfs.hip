@@ -355,15 +355,15 @@ __global__ __launch_bounds__(CBLOCK) void k_msbfs_list_scan(gga_dev_graph g, gga
     compact_scan(bfs_list(g, b), g.n, s_wave);
 }
 __global__ __launch_bounds__(CBLOCK) void k_msbfs_list_write(gga_dev_graph g, gga_dev_msbfs b) {
-    __shared__ uint32_t s_wave[CBLOCK / GGA_WAVE];
+    __shared__ uint32_t s_wave[CBLOCK / GGA_WAVE], s_stage[CSTAGE];
     const ListOut o = bfs_list(g, b);
     for (uint32_t t = blockIdx.x; t < GGA_TILES(g.n); t += gridDim.x)
-        compact_write_tile(o, g.n, t, FrontMarked{b.front}, s_wave);
+        compact_write_tile(o, g.n, t, FrontMarked{b.front}, s_wave, s_stage);
 }
 
 __global__ __launch_bounds__(BLOCK) void k_msbfs(gga_dev_graph g, gga_dev_graph t, gga_dev_msbfs b,
                                                  uint32_t max_levels, uint64_t spin_ticks) {
-    __shared__ uint32_t s_wave[WAVES];
+    __shared__ uint32_t s_wave[WAVES], s_stage[CSTAGE];
     __shared__ uint64_t s_red[WAVES];
     __shared__ uint32_t s_state[3];
     uint32_t gen = 0;
@@ -423,7 +423,7 @@ __global__ __launch_bounds__(BLOCK) void k_msbfs(gga_dev_graph g, gga_dev_graph 
         if (!pull) {
             // the list of the next level: each workgroup sums the counts of
             // the tiles before its own, the last tile's stores the length
-            compact_write_tiles(o, g.n, FrontMarked{nfront}, s_wave);
+            compact_write_tiles(o, g.n, FrontMarked{nfront}, s_wave, s_stage);
             grid_barrier(b.ctl, gridDim.x, gen, spin_ticks);
         }
         dir = pull ? 1u : 0u;

@@ -554,6 +554,14 @@ __global__ __launch_bounds__(BLOCK) void k_query_init(gga_dev_graph g, gga_dev_w
         }
         if (threadIdx.x == 0) {
             w.ctl[GGA_CTL_FAR] = 0;
+            for (uint32_t i = 0; i < 3; i++) {
+                w.ctl[GGA_CTL_PHASE(i)] = GGA_PH_START;
+                w.ctl[GGA_CTL_PSTEP(i)] = 0;
+                w.ctl[GGA_CTL_PLEN(i)] = 0;
+                w.ctl[GGA_CTL_LISTED(i)] = 0;
+            }
+            w.ctl[GGA_CTL_PHASES] = 0;
+            *reinterpret_cast<uint64_t *>(w.ctl + GGA_CTL_T0) = wall_clock64();
             w.ctl[GGA_CTL_RSTEP] = epoch - 1u;   // no refill yet (step numbers start at epoch)
         }
         if (threadIdx.x < GGA_BAR_GROUPS) w.ctl[GGA_CTL_BARG(threadIdx.x)] = 0;
@@ -947,10 +955,10 @@ __device__ __forceinline__ void refill_scan_body(const gga_dev_graph &g, const g
 }
 
 __device__ __forceinline__ void refill_write_body(const gga_dev_graph &g, const gga_dev_work &w, uint32_t step,
-                                                  uint32_t *s_wave) {
+                                                  uint32_t *s_wave, uint32_t *stage) {
     const ListOut o = list_out(g, w, step);
     const DeferredUnder pred{w.dist, w.last, w.ctl[GGA_CTL_RTHR]};
-    for (uint32_t t = blockIdx.x; t < GGA_TILES(g.n); t += gridDim.x) compact_write_tile(o, g.n, t, pred, s_wave);
+    for (uint32_t t = blockIdx.x; t < GGA_TILES(g.n); t += gridDim.x) compact_write_tile(o, g.n, t, pred, s_wave, stage);
 }
 
 // The standalone refill is two launches: its count runs in the compaction's
@@ -972,14 +980,14 @@ __device__ __forceinline__ void refill_write_body(const gga_dev_graph &g, const 
 // step refills (RSTEP = its step number).
 template <bool LVL>
 __global__ __launch_bounds__(BLOCK) void k_compact_write(gga_dev_graph g, gga_dev_work w, uint32_t step) {
-    __shared__ uint32_t s_wave[WAVES], s_min[WAVES];
+    __shared__ uint32_t s_wave[WAVES], s_min[WAVES], s_stage[CSTAGE];
     const uint32_t nq = step_len(w, step), sout = (step + 1u) % 3u;
     const bool flags = nq != 0 && flag_step(w, nq);
     if (flags) {
         if (!w.last || w.ctl[GGA_CTL_LISTED(sout)] != 0u) {
             const uint32_t it = w.ctl[GGA_CTL_ITER(step % 3u)];
-            if (LVL) compact_write_tiles(list_out(g, w, step), g.n, level_marked<true>(w, it), s_wave);
-            else compact_write_tiles(list_out(g, w, step), g.n, StampMarked<true>{w.flag}, s_wave);
+            if (LVL) compact_write_tiles(list_out(g, w, step), g.n, level_marked<true>(w, it), s_wave, s_stage);
+            else compact_write_tiles(list_out(g, w, step), g.n, StampMarked<true>{w.flag}, s_wave, s_stage);
             return;
         }
     } else if (!w.last || w.ctl[GGA_CTL_TAIL(sout)] != 0u) {
@@ -993,10 +1001,9 @@ __global__ __launch_bounds__(BLOCK) void k_compact_write(gga_dev_graph g, gga_de
     refill_count_body(g, w, step, s_wave, s_min);
 }
 
-__global__ __launch_bounds__(BLOCK) void k_refill_write(gga_dev_graph g, gga_dev_work w, uint32_t step) {
-    __shared__ uint32_t s_wave[WAVES], s_min[WAVES];
-    if (!w.last) return;
-    if (w.ctl[GGA_CTL_RSTEP] != w.ctl[GGA_CTL_ITER(step % 3u)]) return;  // no refill after this step
+// (every workgroup of the grid calls this; s_min: one entry per wave)
+__device__ __forceinline__ void refill_list_body(const gga_dev_graph &g, const gga_dev_work &w, uint32_t step,
+                                                 uint32_t *s_wave, uint32_t *s_min, uint32_t *stage) {
     const uint32_t sout = (step + 1u) % 3u, t1 = w.ctl[GGA_CTL_RTHR];
     const ListOut o = list_out(g, w, step);
     if (blockIdx.x == 0) {
@@ -1031,7 +1038,68 @@ __global__ __launch_bounds__(BLOCK) void k_refill_write(gga_dev_graph g, gga_dev
         }
         __syncthreads();
     }
-    compact_write_tiles(o, g.n, DeferredUnder{w.dist, w.last, t1}, s_wave);
+    compact_write_tiles(o, g.n, DeferredUnder{w.dist, w.last, t1}, s_wave, stage);
+}
+
+__global__ __launch_bounds__(BLOCK) void k_refill_write(gga_dev_graph g, gga_dev_work w, uint32_t step) {
+    __shared__ uint32_t s_wave[WAVES], s_min[WAVES], s_stage[CSTAGE];
+    if (!w.last) return;
+    if (w.ctl[GGA_CTL_RSTEP] != w.ctl[GGA_CTL_ITER(step % 3u)]) return;  // no refill after this step
+    refill_list_body(g, w, step, s_wave, s_min, s_stage);
+}
+
+// ------------------------------------------------------ one launch per phase
+// A query's steps as a chain of launches of this kernel, each running the next
+// phase (gga_next_phase).  The launches of a step as kernels of their own --
+// relax, count, write, refill -- cost a kernel boundary (~4.5 us) and a host
+// enqueue each whether the step needs them or not: a queue step needs one of
+// the four.
+template <bool BFS, bool CONT>
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(CONT ? 4 : 8, 8)))
+void k_wl_phase(gga_dev_graph g, gga_dev_work w, uint32_t launch) {
+    __shared__ uint32_t s_pbuf[WAVES][PBUF];
+    __shared__ uint4 s_cq[CONT ? WAVES : 1][CONT ? CQ : 1];
+    __shared__ uint2 s_tab[WAVES][GGA_WAVE];
+    __shared__ uint32_t s_wave[WAVES], s_min[WAVES];
+    constexpr bool LVL = BFS && !CONT;
+    uint32_t *const stage = &s_pbuf[0][0];   // (the push buffers are free outside the relax phase)
+    static_assert(CSTAGE <= WAVES * PBUF, "staging fits the push buffers");
+    uint32_t step;
+    const uint32_t phase = gga_next_phase(w.ctl, launch, w.dense_min, !BFS && w.last != nullptr, w.cap, &step);
+    if (phase == GGA_PH_DONE || phase == GGA_PH_CAPPED) {
+        if (blockIdx.x == 0 && threadIdx.x == 0) w.ctl[GGA_CTL_PHASE(launch)] = phase;
+        return;
+    }
+    const uint32_t it = w.ctl[GGA_CTL_ITER(step % 3u)], sout = (step + 1u) % 3u;
+    const uint32_t nq = phase == GGA_PH_RELAX ? step_len(w, step) : 0u;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        w.ctl[GGA_CTL_PHASE(launch)] = phase;
+        w.ctl[GGA_CTL_PSTEP(launch)] = step;
+        w.ctl[GGA_CTL_PLEN(launch)] = nq;
+        w.ctl[GGA_CTL_PHASES] += 1u;
+        if (phase == GGA_PH_RELAX) step_bookkeeping(w.ctl, step, it, nq);
+        if (phase == GGA_PH_RCOUNT) w.ctl[GGA_CTL_RTHR] = sat_add(w.ctl[GGA_CTL_THR(sout)], w.delta);
+    }
+    if (phase == GGA_PH_RELAX) {
+        Counters cnt;
+        const uint32_t wv = __builtin_amdgcn_readfirstlane(threadIdx.x / GGA_WAVE);
+        worklist_step<BFS, false, CONT>(g, w, step, nq, it, s_pbuf[wv], s_cq[CONT ? wv : 0], s_tab[wv], cnt);
+    } else if (phase == GGA_PH_COUNT) {
+        const ListOut o = list_out(g, w, step);
+        uint32_t any = 0;
+        for (uint32_t t = blockIdx.x; t < GGA_TILES(g.n); t += gridDim.x)
+            any |= LVL ? compact_count_tile(o, g.n, t, level_marked<false>(w, it), s_wave)
+                       : compact_count_tile(o, g.n, t, StampMarked<false>{w.flag}, s_wave);
+        if (any && threadIdx.x == 0) w.ctl[GGA_CTL_LISTED(sout)] = 1u;
+    } else if (phase == GGA_PH_WRITE) {
+        const ListOut o = list_out(g, w, step);
+        if (LVL) compact_write_tiles(o, g.n, level_marked<true>(w, it), s_wave, stage);
+        else compact_write_tiles(o, g.n, StampMarked<true>{w.flag}, s_wave, stage);
+    } else if (!BFS && phase == GGA_PH_RCOUNT) {
+        refill_count_body(g, w, step, s_wave, s_min);
+    } else if (!BFS) {
+        refill_list_body(g, w, step, s_wave, s_min, stage);
+    }
 }
 
 // ------------------------------------------------------ persistent kernel
@@ -1071,8 +1139,8 @@ __global__ __launch_bounds__(BLOCK) void k_persistent(gga_dev_graph g, gga_dev_w
             grid_barrier(w.ctl, gridDim.x, gen, spin_ticks);
             // each workgroup sums the tile counts before its own tiles: no
             // serial scan between two more grid barriers
-            if (BFS && !CONT) compact_write_tiles(o, g.n, level_marked<true>(w, it), s_wave);
-            else compact_write_tiles(o, g.n, StampMarked<true>{w.flag}, s_wave);
+            if (BFS && !CONT) compact_write_tiles(o, g.n, level_marked<true>(w, it), s_wave, &s_pbuf[0][0]);
+            else compact_write_tiles(o, g.n, StampMarked<true>{w.flag}, s_wave, &s_pbuf[0][0]);
         }
         grid_barrier(w.ctl, gridDim.x, gen, spin_ticks);
         // near-far: an empty next list is refilled from the deferred vertices,
@@ -1100,7 +1168,7 @@ __global__ __launch_bounds__(BLOCK) void k_persistent(gga_dev_graph g, gga_dev_w
             const uint32_t listed = s_state[0], far = s_state[1];
             __syncthreads();
             if (listed) {
-                refill_write_body(g, w, step, s_wave);
+                refill_write_body(g, w, step, s_wave, &s_pbuf[0][0]);
                 grid_barrier(w.ctl, gridDim.x, gen, spin_ticks);
                 break;
             }
@@ -1126,9 +1194,10 @@ __device__ __forceinline__ uint64_t block_sum64(uint64_t x, uint64_t *s_red) {
 // into cnt slots [0, REACH_BLOCKS) word 3 and [REACH_BLOCKS, 2 REACH_BLOCKS)
 // word 3 -- plain stores, no shared counter.
 constexpr uint32_t REACH_BLOCKS = GGA_CNT_SLOTS / 2;
-__global__ __launch_bounds__(BLOCK) void k_reach(gga_dev_graph g, gga_dev_work w) {
-    __shared__ uint64_t s_red[WAVES];
-    uint64_t reached = 0, mr = 0;
+// A thread's reached vertices and their out-degree sum.
+__device__ __forceinline__ void reach_sum(const gga_dev_graph &g, const gga_dev_work &w, uint64_t &reached,
+                                          uint64_t &mr) {
+    reached = mr = 0;
     const uint64_t S = (uint64_t)gridDim.x * blockDim.x;
     uint64_t v = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     // four vertices S apart per round, every load issued before the first
@@ -1154,6 +1223,12 @@ __global__ __launch_bounds__(BLOCK) void k_reach(gga_dev_graph g, gga_dev_work w
             mr += g.row[v + 1] - g.row[v];
         }
     }
+}
+
+__global__ __launch_bounds__(BLOCK) void k_reach(gga_dev_graph g, gga_dev_work w) {
+    __shared__ uint64_t s_red[WAVES];
+    uint64_t reached, mr;
+    reach_sum(g, w, reached, mr);
     reached = block_sum64(reached, s_red);
     mr = block_sum64(mr, s_red);
     if (threadIdx.x == 0) {
@@ -1179,6 +1254,30 @@ __global__ __launch_bounds__(BLOCK) void k_reach_fold(gga_dev_work w) {
             if (k < 3) cnt[k] = t;
             else red[k - 3] = t;
         }
+    }
+}
+
+// The ending of a phase-launched query: reach partials and the control words
+// (lines 0 to 8) straight to the pinned read-back area, one launch where the
+// reach pass, its fold and a copy were three.
+__global__ __launch_bounds__(BLOCK) void k_finish(gga_dev_graph g, gga_dev_work w, uint32_t *host) {
+    __shared__ uint64_t s_red[WAVES];
+    uint64_t *part = reinterpret_cast<uint64_t *>(host + GGA_FIN_PART);
+    if (blockIdx.x == 0) {
+        if (threadIdx.x == 0) {
+            uint64_t *clock = reinterpret_cast<uint64_t *>(host + GGA_FIN_CLOCK);
+            clock[1] = wall_clock64();
+            clock[0] = *reinterpret_cast<uint64_t *>(w.ctl + GGA_CTL_T0);
+        }
+        for (uint32_t i = threadIdx.x; i < 9u * GGA_CTL_LINE; i += blockDim.x) host[i] = w.ctl[i];
+    }
+    uint64_t reached, mr;
+    reach_sum(g, w, reached, mr);
+    reached = block_sum64(reached, s_red);
+    mr = block_sum64(mr, s_red);
+    if (threadIdx.x == 0) {
+        part[2u * blockIdx.x] = reached;
+        part[2u * blockIdx.x + 1u] = mr;
     }
 }
 
@@ -1393,6 +1492,24 @@ __global__ __launch_bounds__(BLOCK) void k_conv(const uint32_t *dist, const uint
 
 extern "C" int ggak_conv(const uint32_t *dist, const uint32_t *fin, uint32_t n, uint64_t *rows, hipStream_t s) {
     k_conv<<<grid_for(n, 1024), BLOCK, 0, s>>>(dist, fin, n, rows);
+    return launch_status();
+}
+
+extern "C" int ggak_wl_phase(gga_dev_graph g, gga_dev_work w, uint32_t launch, int bfs, uint32_t grid, hipStream_t s) {
+    if (grid == 0) return (int)hipErrorInvalidValue;
+    if (bfs) {
+        if (use_cont(w)) k_wl_phase<true, true><<<grid, BLOCK, 0, s>>>(g, w, launch % 3u);
+        else k_wl_phase<true, false><<<grid, BLOCK, 0, s>>>(g, w, launch % 3u);
+    } else {
+        if (use_cont(w)) k_wl_phase<false, true><<<grid, BLOCK, 0, s>>>(g, w, launch % 3u);
+        else k_wl_phase<false, false><<<grid, BLOCK, 0, s>>>(g, w, launch % 3u);
+    }
+    return launch_status();
+}
+
+extern "C" int ggak_finish(gga_dev_graph g, gga_dev_work w, uint32_t *host, uint32_t *blocks, hipStream_t s) {
+    *blocks = grid_for(g.n, GGA_FIN_BLOCKS);
+    k_finish<<<*blocks, BLOCK, 0, s>>>(g, w, host);
     return launch_status();
 }
 

@@ -233,7 +233,7 @@ typedef struct gga_stats {
     uint64_t chunks_expanded; /* I_v  (opts.count) */
     uint64_t relaxations;     /* R: successful atomicMin (opts.count) */
     uint64_t m_reach;         /* sum of out-degrees of reached vertices */
-    uint64_t launches;        /* relax-kernel launches */
+    uint64_t launches;        /* relax-kernel launches (uninstrumented WORKLIST: launches of its phases) */
     uint32_t pull_levels;     /* gga_multi_bfs: levels run bottom-up */
     uint32_t timeline_records;/* records written to opts.timeline */
     uint32_t timeline_grid;   /* workgroups per step in it */
