@@ -69,8 +69,9 @@ int ggak_refill(gga_dev_graph g, gga_dev_work w, uint32_t phase, hipStream_t s);
 int ggak_wl_phase(gga_dev_graph g, gga_dev_work w, uint32_t launch, int bfs, uint32_t grid, hipStream_t s);
 /* Control words, reach partials (*blocks rows of reached, out-degree sum) and
  * the clock at the query's start and now -> host, GGA_FIN_WORDS words of
- * pinned memory by its device address. */
-int ggak_finish(gga_dev_graph g, gga_dev_work w, uint32_t *host, uint32_t *blocks, hipStream_t s);
+ * pinned memory by its device address; the distances -> stage (n words,
+ * likewise; NULL: not). */
+int ggak_finish(gga_dev_graph g, gga_dev_work w, uint32_t *host, uint32_t *stage, uint32_t *blocks, hipStream_t s);
 /* Occupancy-bound grid (workgroups of `block` threads) for the worklist
  * kernel, or for the persistent kernel (always 256 threads); 0 on error. */
 uint32_t ggak_wl_grid(int device, int persistent, int bfs, int count, uint32_t block);

@@ -42,6 +42,13 @@ void gga_graph_set_tuned_block(gga_graph *g, uint32_t block);
 void **gga_graph_msbfs_slot(gga_graph *g);
 void gga_msbfs_release(void *state);
 
+/* dst (host, any allocation) = bytes at src (on `device`, current), after the
+ * work queued on s; returns when dst holds them (copyout.c).  Handles that copy
+ * out are counted: the pinned slots are given back with the last one. */
+hipError_t gga_copy_out(int device, hipStream_t s, void *dst, const void *src, uint64_t bytes);
+void gga_copy_retain(void);
+void gga_copy_release(void);
+
 /* Cooperative launches (persistent kernels) of one process run one at a time:
  * each holds this lock from its launch until its stream has drained.  Two
  * such grids at once could each hold execution slots the other's grid

@@ -22,6 +22,9 @@
 #define GGA_MESH_BMIN 2u    /* chunks per wave batch on mesh-like graphs (2 / 4 / 8, SSSP: pure 1024^2 grid
                                6.08 / 6.23 / 6.42 ms, 4096^2 with shortcuts 6.34 / 6.33 / 6.41) */
 #endif
+/* Up to this many vertices the query's last kernel writes the result into
+ * pinned memory itself (1 MiB, ~20 us over the link) instead of a copy behind it. */
+#define STAGE_N (1u << 18)
 static int mesh_like(const gga_graph *g);
 
 #define GGA_VERSION "gga 0.1.0 (gfx950)"
@@ -47,6 +50,7 @@ struct gga_graph {
     uint32_t *h_pin;          /* pinned: GGA_FIN_WORDS words (the control words first) */
     uint32_t *d_pin;          /* its device address */
     uint32_t clock_khz;       /* device wall clock */
+    uint32_t *h_stage, *d_stage; /* pinned: n words for the result of a small graph (else NULL), device address */
     uint32_t epoch;           /* step number of the next query's first step (mark[] stamps are below it) */
     int mark_dirty;           /* mark[] holds stamps of unknown step numbers: refill before the next query */
     int have_result;
@@ -216,6 +220,7 @@ int gga_graph_free(gga_graph *g)
         if (g->kev[i]) hipEventDestroy(g->kev[i]);
     free(g->kev);
     if (g->stream) hipStreamDestroy(g->stream);
+    gga_copy_release();
     free(g);
     return GGA_OK;
 }
@@ -240,14 +245,22 @@ static int graph_create(uint32_t n, uint32_t m, const uint32_t *row_ptr, const u
     if (device < 0 || device >= ndev) return GGA_EINVAL;
     gga_graph *g = (gga_graph *)calloc(1, sizeof *g);
     if (!g) return GGA_ENOMEM;
+    gga_copy_retain();
     g->device = device;
     g->n = n;
     g->m = m;
     HIP_TRY(hipSetDevice(device));
     HIP_TRY(hipStreamCreateWithFlags(&g->stream, hipStreamNonBlocking));
     for (int i = 0; i < 4; i++) HIP_TRY(hipEventCreate(&g->ev[i]));
-    HIP_TRY(hipHostMalloc((void **)&g->h_pin, 4ull * GGA_FIN_WORDS, hipHostMallocDefault));
-    HIP_TRY(hipHostGetDevicePointer((void **)&g->d_pin, g->h_pin, 0));
+    {
+        const uint64_t stage = n <= STAGE_N ? n : 0u;
+        HIP_TRY(hipHostMalloc((void **)&g->h_pin, 4ull * (GGA_FIN_WORDS + stage), hipHostMallocDefault));
+        HIP_TRY(hipHostGetDevicePointer((void **)&g->d_pin, g->h_pin, 0));
+        if (stage) {
+            g->h_stage = g->h_pin + GGA_FIN_WORDS;
+            g->d_stage = g->d_pin + GGA_FIN_WORDS;
+        }
+    }
     {
         int khz = 0;
         if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, device) != hipSuccess || khz <= 0)
@@ -526,9 +539,8 @@ int gga_graph_chunks(gga_graph *g, uint32_t *chunk_begin, uint32_t *owner)
     /* the reference's table (NodeSplit's layout), also where the kernels walk a cut one */
     const uint32_t *cb = g->d_rcbeg ? g->d_rcbeg : g->d_cbeg, *co = g->d_rcown ? g->d_rcown : g->d_cown;
     if (chunk_begin)
-        HIP_TRY(hipMemcpyAsync(chunk_begin, cb, 4ull * ((uint64_t)g->Cref + 1), hipMemcpyDeviceToHost, g->stream));
-    if (owner) HIP_TRY(hipMemcpyAsync(owner, co, 4ull * g->Cref, hipMemcpyDeviceToHost, g->stream));
-    HIP_TRY(hipStreamSynchronize(g->stream));
+        HIP_TRY(gga_copy_out(g->device, g->stream, chunk_begin, cb, 4ull * ((uint64_t)g->Cref + 1)));
+    if (owner) HIP_TRY(gga_copy_out(g->device, g->stream, owner, co, 4ull * g->Cref));
     return GGA_OK;
 fail:
     return rc;
@@ -670,9 +682,11 @@ int gga_graph_mesh_like(const gga_graph *g) { return g ? mesh_like(g) : 0; }
 typedef struct query_plan {
     int bfs, mode, count, own;
     uint32_t src, max_iters, epoch;
+    uint32_t *stage;   /* pinned area for the distances (device address), or NULL */
+    int staged;        /* set when the query left them there */
 } query_plan;
 
-static int run_query(gga_graph *g, gga_dev_graph dg, gga_dev_work dw, const query_plan *p, gga_opts *o,
+static int run_query(gga_graph *g, gga_dev_graph dg, gga_dev_work dw, query_plan *p, gga_opts *o,
                      gga_stats *s, uint32_t *adv)
 {
     int rc = GGA_OK;
@@ -763,7 +777,7 @@ static int run_query(gga_graph *g, gga_dev_graph dg, gga_dev_work dw, const quer
             for (;;) {
                 for (uint32_t k = 0; k < nl; k++)
                     K_TRY(ggak_wl_phase(dg, dw, launch++, bfs, grid, g->stream));
-                K_TRY(ggak_finish(dg, dw, g->d_pin, &fin, g->stream));
+                K_TRY(ggak_finish(dg, dw, g->d_pin, p->stage, &fin, g->stream));
                 HIP_TRY(hipStreamSynchronize(g->stream));
                 s->launches += nl;
                 const uint32_t next =
@@ -777,6 +791,7 @@ static int run_query(gga_graph *g, gga_dev_graph dg, gga_dev_work dw, const quer
                 if (!o->sync_every) nl = 24u;
             }
             g->last_phases[bfs ? 1 : 0] = g->h_pin[GGA_CTL_PHASES];
+            p->staged = p->stage != NULL;
             ended = 1;
         } else {
         if (tev && (rc = ensure_kev(g, 3 * (nb > per ? nb : per)))) goto fail;
@@ -965,6 +980,7 @@ fail:
  * query). */
 static void plan_query(const gga_graph *g, int bfs, const gga_opts *o, query_plan *p, uint32_t *delta)
 {
+    memset(p, 0, sizeof *p);
     p->bfs = bfs;
     p->count = o->count ? 1 : 0;
     int mode = o->mode;
@@ -1057,11 +1073,14 @@ static int traverse(gga_graph *g, uint32_t src, int bfs, uint32_t *out, const gg
         dw.delta = delta;
     }
     s.mode = p.mode;
+    if (out) p.stage = g->d_stage;
     rc = run_query(g, dg, dw, &p, &o, &s, &adv);
     if (rc) goto fail;
     g->epoch = p.epoch + adv + 1u;
     g->have_result = 1;
-    if (out) HIP_TRY(hipMemcpy(out, g->d_dist, 4ull * g->n, hipMemcpyDeviceToHost));   /* bfs_sssp.cu:489 */
+    /* the result (bfs_sssp.cu:489): on a small graph it came with the query's ending */
+    if (out && p.staged) memcpy(out, g->h_stage, 4ull * g->n);
+    else if (out) HIP_TRY(gga_copy_out(g->device, g->stream, out, g->d_dist, 4ull * g->n));
     if (st) *st = s;
     return GGA_OK;
 fail:
@@ -1207,7 +1226,7 @@ int gga_graph_copy_dist(gga_graph *g, uint32_t *out)
     if (!g || !out) return GGA_EINVAL;
     if (!g->have_result) return GGA_EINVAL;
     HIP_TRY(hipSetDevice(g->device));
-    HIP_TRY(hipMemcpy(out, g->d_dist, 4ull * g->n, hipMemcpyDeviceToHost));
+    HIP_TRY(gga_copy_out(g->device, g->stream, out, g->d_dist, 4ull * g->n));
     return GGA_OK;
 fail:
     return rc;

@@ -597,10 +597,14 @@ int gga_ms_fetch(gga_ms *e, uint32_t lanes, uint32_t *const *out, int on_device)
         }
     K_TRY(ggak_ms_harvest(e->v.dg, e->d, lanes, po, e->v.stream));
     if (!on_device)
-        for (uint32_t i = 0; i < GGA_MS_LANES; i++)
+        for (uint32_t i = 0, k; i < GGA_MS_LANES; i += k) {
+            /* rows that follow each other in the caller's memory too: one copy */
+            for (k = 1; i + k < GGA_MS_LANES && ((lanes >> i) & 1u) && ((lanes >> (i + k)) & 1u) &&
+                        out[i + k] == out[i] + (uint64_t)k * e->n; k++) {}
             if ((lanes >> i) & 1u)
-                HIP_TRY(hipMemcpyAsync(out[i], po.p[i], 4ull * e->n, hipMemcpyDeviceToHost, e->v.stream));
-    HIP_TRY(hipStreamSynchronize(e->v.stream));
+                HIP_TRY(gga_copy_out(e->v.device, e->v.stream, out[i], po.p[i], 4ull * k * e->n));
+        }
+    else HIP_TRY(hipStreamSynchronize(e->v.stream));
     return GGA_OK;
 fail:
     return rc;

@@ -303,7 +303,7 @@ int gga_multi_bfs(gga_graph *g, const uint32_t *srcs, uint32_t k, uint32_t *out,
     r.ktime_ms = r.time_ms;
     r.mode = GGA_MODE_PERSISTENT;
     r.launches = 1;
-    if (out) HIP_TRY(hipMemcpy(out, s->lev, 4ull * k * v.dg.n, hipMemcpyDeviceToHost));
+    if (out) HIP_TRY(gga_copy_out(v.device, v.stream, out, s->lev, 4ull * k * v.dg.n));
     if (st) *st = r;
     return GGA_OK;
 fail:

@@ -1259,8 +1259,9 @@ __global__ __launch_bounds__(BLOCK) void k_reach_fold(gga_dev_work w) {
 
 // The ending of a phase-launched query: reach partials and the control words
 // (lines 0 to 8) straight to the pinned read-back area, one launch where the
-// reach pass, its fold and a copy were three.
-__global__ __launch_bounds__(BLOCK) void k_finish(gga_dev_graph g, gga_dev_work w, uint32_t *host) {
+// reach pass, its fold and a copy were three; stage: the distances of a small
+// graph go to pinned memory with it.
+__global__ __launch_bounds__(BLOCK) void k_finish(gga_dev_graph g, gga_dev_work w, uint32_t *host, uint32_t *stage) {
     __shared__ uint64_t s_red[WAVES];
     uint64_t *part = reinterpret_cast<uint64_t *>(host + GGA_FIN_PART);
     if (blockIdx.x == 0) {
@@ -1271,6 +1272,9 @@ __global__ __launch_bounds__(BLOCK) void k_finish(gga_dev_graph g, gga_dev_work 
         }
         for (uint32_t i = threadIdx.x; i < 9u * GGA_CTL_LINE; i += blockDim.x) host[i] = w.ctl[i];
     }
+    if (stage)
+        for (uint64_t v = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; v < g.n; v += (uint64_t)gridDim.x * blockDim.x)
+            stage[v] = w.dist[v];
     uint64_t reached, mr;
     reach_sum(g, w, reached, mr);
     reached = block_sum64(reached, s_red);
@@ -1507,9 +1511,10 @@ extern "C" int ggak_wl_phase(gga_dev_graph g, gga_dev_work w, uint32_t launch, i
     return launch_status();
 }
 
-extern "C" int ggak_finish(gga_dev_graph g, gga_dev_work w, uint32_t *host, uint32_t *blocks, hipStream_t s) {
+extern "C" int ggak_finish(gga_dev_graph g, gga_dev_work w, uint32_t *host, uint32_t *stage, uint32_t *blocks,
+                           hipStream_t s) {
     *blocks = grid_for(g.n, GGA_FIN_BLOCKS);
-    k_finish<<<*blocks, BLOCK, 0, s>>>(g, w, host);
+    k_finish<<<*blocks, BLOCK, 0, s>>>(g, w, host, stage);
     return launch_status();
 }
 
