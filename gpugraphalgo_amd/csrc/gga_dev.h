@@ -47,6 +47,9 @@ typedef struct gga_dev_work {
     uint32_t *tiles;     /* list compaction: per-tile counts, then offsets (GGA_TILES(n) + 1) */
     uint32_t *last;      /* near-far: distance of each vertex at its last expansion (NULL: off) */
     uint32_t *tmin;      /* near-far: per-tile minimum deferred distance (GGA_TILES(n)) */
+    uint32_t *sdist;     /* spread distances (SSSP on skewed graphs; NULL: dist takes the atomics):
+                            vertex v's is word gga_spread(v, smask) */
+    uint32_t smask;      /* its words - 1: gga_spread_words(n) - 1 */
     uint32_t inf;
     uint32_t qcap;       /* capacity of q0 / q1 in entries (>= C) */
     uint32_t dense_min;  /* a step whose list holds >= dense_min chunks is a flag step */
@@ -56,6 +59,11 @@ typedef struct gga_dev_work {
     uint32_t cap;        /* most steps of a query run one phase per launch */
     uint32_t lvl;        /* 1: BFS steps are levels (step epoch + k reaches level k + 1) */
 } gga_dev_work;
+
+/* An odd multiplier permutes the residues of a power of two: neighbouring
+ * vertices lie far apart, each on a word of its own. */
+#define GGA_SPREAD_MUL    2654435761u
+#define GGA_SPREAD_MIN    65536u   /* words, at least: 256 KiB reach every memory channel */
 
 /* Per-workgroup timeline record of an instrumented relax step: start on the
  * 100 MHz device wall clock, duration in its ticks, placement = XCC id << 8 |
@@ -201,6 +209,19 @@ typedef struct gga_dev_msbfs {
  * kernel argument) so that steps replayed from a captured graph see restarts */
 #define GGA_CTL_UNIT      (7u * GGA_CTL_LINE + 12u)
 
+#ifdef __HIPCC__
+#define GGA_HOSTDEV __host__ __device__
+#else
+#define GGA_HOSTDEV
+#endif
+static inline GGA_HOSTDEV uint32_t gga_spread(uint32_t v, uint32_t smask) { return (v * GGA_SPREAD_MUL) & smask; }
+static inline GGA_HOSTDEV uint64_t gga_spread_words(uint64_t n)
+{
+    uint64_t s = GGA_SPREAD_MIN;
+    while (s < n) s *= 2u;
+    return s;
+}
+
 /* What a query's pinned read-back area holds behind the control words: the
  * reach partials of each workgroup (reached, out-degree sum; u64), then the
  * wall clock at the query's start and end (u64). */
@@ -212,11 +233,6 @@ typedef struct gga_dev_msbfs {
 /* Phases of a single-source worklist query (kernels/relax.hip, k_wl_phase). */
 enum { GGA_PH_START, GGA_PH_RELAX, GGA_PH_COUNT, GGA_PH_WRITE, GGA_PH_RCOUNT, GGA_PH_RWRITE, GGA_PH_DONE,
        GGA_PH_CAPPED };
-#ifdef __HIPCC__
-#define GGA_HOSTDEV __host__ __device__
-#else
-#define GGA_HOSTDEV
-#endif
 /* The phase of launch `launch` and its step, from the record of the launch
  * before and the words that launch left: every workgroup of a launch computes
  * it for itself (no launch changes a word it reads here), and the host knows

@@ -292,7 +292,24 @@ __device__ __forceinline__ void follow_front(const gga_dev_graph &g, const gga_d
 // batch lowers below the threshold go to the wave's queue instead of the list,
 // and follow_front expands them within the step.  (BFS then takes the step
 // stamp too: levels reached out of order can drop twice.)
-template <bool BFS, bool COUNT, int OUT, bool CONT = false>
+//
+// SPREAD (SSSP on graphs whose hubs are neighbours, w.sdist set): atomics run at
+// 26 G/s over distinct memory channels on MI355X, but at 3.8 (2^17 vertices)
+// to 7 G/s (2^22) where they fall as R-MAT destinations do, because the hubs'
+// words share a few 256-byte granules.  They go to a permuted copy of the
+// distances instead, sdist, which decides; dist, in vertex order, whose
+// gathers profit from the same neighbourhood, stays the guard.  Whoever lowers
+// sdist (the atomic's result says so, in flag steps too) stores its distance
+// to dist; racing stores may leave dist above sdist, never below, and each of
+// them lists its vertex, whose next expansion starts from sdist and brings
+// dist up to date.  So when no list is left, dist equals sdist.  SSSP, three
+// sources each, without / with: R-MAT 2^16 320 / 280 / 274 -> 268 / 224 / 232
+// us, 2^17 (T = 992) 396 / 349 / 433 -> 347 / 307 / 381, 2^20 781 / 950 / 740
+// -> 667 / 787 / 626, 2^21 1098 / 1204 / 1494 -> 1070 / 1144 / 1414; 2^22 2090
+// -> 2186 (the copy falls out of the caches there: see skewed() for the rule).
+// Stores and stamps by everyone who passes the guard, no result awaited, left
+// dist loose enough to expand a quarter more edges (2^22: 2650 us).
+template <bool BFS, bool COUNT, int OUT, bool CONT = false, bool SPREAD = false>
 __device__ __forceinline__ void expand_batch(const gga_dev_graph &g, const gga_dev_work &w,
                                              const ChunkDesc &d, uint32_t it, uint32_t *pbuf,
                                              uint32_t &pcount, uint32_t *qout, uint32_t *tail,
@@ -306,7 +323,7 @@ __device__ __forceinline__ void expand_batch(const gga_dev_graph &g, const gga_d
         eb = d.eb;
         const uint32_t ee = d.ee;
         const uint32_t own = d.own;
-        du = dist[own];
+        du = SPREAD ? w.sdist[gga_spread(own, w.smask)] : dist[own];
         // SSSP: an owner already lowered and listed again during this step is
         // expanded in the next one with its newer distance, which relaxes
         // every edge at least as far -- expanding it now would only repeat
@@ -324,7 +341,8 @@ __device__ __forceinline__ void expand_batch(const gga_dev_graph &g, const gga_d
         // are never relaxed again.
         const bool go = du < inf && !again && du < thr;
         n = go ? ee - eb : 0u;
-        if (w.last && go) w.last[own] = du;
+        if (!SPREAD && w.last && go) w.last[own] = du;
+        if (SPREAD && go) dist[own] = du;
     }
     constexpr bool cont = CONT && OUT != OUT_CHANGED;
     uint32_t qt = 0;   // vertices queued (wave-uniform)
@@ -399,13 +417,15 @@ __device__ __forceinline__ void expand_batch(const gga_dev_graph &g, const gga_d
                     r0[u] = g.row[v[u]];
                     r1[u] = g.row[v[u] + 1u];
                 }
-                if (OUT == OUT_FLAG) {
-                    (void)atomic_min_u32(&dist[v[u]], alt);  // result unused: no-return atomic
+                uint32_t *const at = SPREAD ? &w.sdist[gga_spread(v[u], w.smask)] : &dist[v[u]];
+                if (OUT == OUT_FLAG && !SPREAD) {
+                    (void)atomic_min_u32(at, alt);  // result unused: no-return atomic
                     imp = true;
                 } else {
-                    const uint32_t old = atomic_min_u32(&dist[v[u]], alt);
+                    const uint32_t old = atomic_min_u32(at, alt);
                     imp = alt < old;
                 }
+                if (SPREAD && imp) dist[v[u]] = alt;
             }
             if (COUNT) cnt.relax += __builtin_amdgcn_readfirstlane((uint32_t)__popcll(__ballot(imp)));
             if (OUT == OUT_CHANGED) {
@@ -542,6 +562,8 @@ __global__ __launch_bounds__(BLOCK) void k_query_init(gga_dev_graph g, gga_dev_w
         w.flag[v] = w.lvl && v == src ? 255u : 0u;
     if (w.last)
         for (uint64_t v = tid; v < g.n; v += nth) w.last[v] = w.inf;
+    if (w.sdist)
+        for (uint64_t i = tid; i <= w.smask; i += nth) w.sdist[i] = i == gga_spread(src, w.smask) ? 0u : w.inf;
     for (uint64_t i = tid; i < 4ull * GGA_CNT_SLOTS; i += nth) w.cnt[i] = 0;
     if (blockIdx.x == 0) {
         const uint32_t cs = g.cstart[src], nch = g.cstart[src + 1] - cs;
@@ -605,7 +627,7 @@ __device__ __forceinline__ bool flag_step(const gga_dev_work &w, uint32_t nq) {
 }
 
 // One step = expand the list of ring slot (step % 3), fill slot (step + 1) % 3.
-template <bool BFS, bool COUNT, bool CONT>
+template <bool BFS, bool COUNT, bool CONT, bool SPREAD = false>
 __device__ __forceinline__ void worklist_step(const gga_dev_graph &g, const gga_dev_work &w,
                                               uint32_t step, uint32_t nq, uint32_t it,
                                               uint32_t *pbuf, uint4 *cq, uint2 *tab, Counters &cnt) {
@@ -670,10 +692,10 @@ __device__ __forceinline__ void worklist_step(const gga_dev_graph &g, const gga_
             expand_level<COUNT, OUT_QUEUE>(g, w, cur, alt, stamp, pbuf, pcount, qout, tail, cnt,
                                            reinterpret_cast<uint32_t *>(tab), bsz);
         else if (flags)
-            expand_batch<BFS, COUNT, OUT_FLAG, CONT>(g, w, cur, it, pbuf, pcount, qout, tail, dummy, cnt, tab, bsz,
+            expand_batch<BFS, COUNT, OUT_FLAG, CONT, SPREAD>(g, w, cur, it, pbuf, pcount, qout, tail, dummy, cnt, tab, bsz,
                                                      thr, follow);
         else
-            expand_batch<BFS, COUNT, OUT_QUEUE, CONT>(g, w, cur, it, pbuf, pcount, qout, tail, dummy, cnt, tab, bsz,
+            expand_batch<BFS, COUNT, OUT_QUEUE, CONT, SPREAD>(g, w, cur, it, pbuf, pcount, qout, tail, dummy, cnt, tab, bsz,
                                                       thr, follow);
         cur = nxt;
         c_next = c_after;
@@ -797,7 +819,7 @@ __device__ __forceinline__ uint32_t hw_place() {
 // and drop to seven): the relax is bound by the latency of its gathers.  (The
 // mesh variants' queues, 8 KB of LDS per wave, leave room for four.)
 // BS: workgroup size, 128, 256 or 512 threads (the tuner times all three).
-template <bool BFS, bool COUNT, bool TL, uint32_t BS, bool CONT>
+template <bool BFS, bool COUNT, bool TL, uint32_t BS, bool CONT, bool SPREAD>
 __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(CONT ? 4 : 8, 8)))
 void k_wl_step(gga_dev_graph g, gga_dev_work w, uint32_t step, gga_wg_record *tl) {
     __shared__ uint32_t s_pbuf[BS / GGA_WAVE][PBUF];
@@ -811,7 +833,7 @@ void k_wl_step(gga_dev_graph g, gga_dev_work w, uint32_t step, gga_wg_record *tl
     if (nq != 0) {
         Counters cnt;
         const uint32_t wv = __builtin_amdgcn_readfirstlane(threadIdx.x / GGA_WAVE);
-        worklist_step<BFS, COUNT, CONT>(g, w, step, nq, it, s_pbuf[wv], s_cq[CONT ? wv : 0], s_tab[wv], cnt);
+        worklist_step<BFS, COUNT, CONT, SPREAD>(g, w, step, nq, it, s_pbuf[wv], s_cq[CONT ? wv : 0], s_tab[wv], cnt);
         publish_counters<COUNT>(w, cnt);
     }
     if (TL) {
@@ -1054,7 +1076,7 @@ __global__ __launch_bounds__(BLOCK) void k_refill_write(gga_dev_graph g, gga_dev
 // relax, count, write, refill -- cost a kernel boundary (~4.5 us) and a host
 // enqueue each whether the step needs them or not: a queue step needs one of
 // the four.
-template <bool BFS, bool CONT>
+template <bool BFS, bool CONT, bool SPREAD>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(CONT ? 4 : 8, 8)))
 void k_wl_phase(gga_dev_graph g, gga_dev_work w, uint32_t launch) {
     __shared__ uint32_t s_pbuf[WAVES][PBUF];
@@ -1083,7 +1105,7 @@ void k_wl_phase(gga_dev_graph g, gga_dev_work w, uint32_t launch) {
     if (phase == GGA_PH_RELAX) {
         Counters cnt;
         const uint32_t wv = __builtin_amdgcn_readfirstlane(threadIdx.x / GGA_WAVE);
-        worklist_step<BFS, false, CONT>(g, w, step, nq, it, s_pbuf[wv], s_cq[CONT ? wv : 0], s_tab[wv], cnt);
+        worklist_step<BFS, false, CONT, SPREAD>(g, w, step, nq, it, s_pbuf[wv], s_cq[CONT ? wv : 0], s_tab[wv], cnt);
     } else if (phase == GGA_PH_COUNT) {
         const ListOut o = list_out(g, w, step);
         uint32_t any = 0;
@@ -1429,17 +1451,20 @@ extern "C" int ggak_topo_step(gga_dev_graph g, gga_dev_work w, int bfs, int coun
 // Kernel variants by (bfs, count, instrumented, mesh continuation) and
 // workgroup size.  The continuation has kernels of its own, so that the
 // registers of the others stay as they were.
-template <bool BFS, bool COUNT, bool TL, bool CONT>
+template <bool BFS, bool COUNT, bool TL, bool CONT, bool SPREAD>
 static const void *wl_fn_c(uint32_t block) {
     switch (block) {
-    case 128: return reinterpret_cast<const void *>(&k_wl_step<BFS, COUNT, TL, 128, CONT>);
-    case 512: return reinterpret_cast<const void *>(&k_wl_step<BFS, COUNT, TL, 512, CONT>);
-    default: return reinterpret_cast<const void *>(&k_wl_step<BFS, COUNT, TL, 256, CONT>);
+    case 128: return reinterpret_cast<const void *>(&k_wl_step<BFS, COUNT, TL, 128, CONT, SPREAD>);
+    case 512: return reinterpret_cast<const void *>(&k_wl_step<BFS, COUNT, TL, 512, CONT, SPREAD>);
+    default: return reinterpret_cast<const void *>(&k_wl_step<BFS, COUNT, TL, 256, CONT, SPREAD>);
     }
 }
+// (spread: SSSP on graphs that are not meshes, see expand_batch)
 template <bool BFS, bool COUNT, bool TL>
-static const void *wl_fn(uint32_t block, int cont) {
-    return cont ? wl_fn_c<BFS, COUNT, TL, true>(block) : wl_fn_c<BFS, COUNT, TL, false>(block);
+static const void *wl_fn(uint32_t block, int cont, int spread) {
+    if constexpr (!BFS)
+        if (spread) return wl_fn_c<BFS, COUNT, TL, false, true>(block);
+    return cont ? wl_fn_c<BFS, COUNT, TL, true, false>(block) : wl_fn_c<BFS, COUNT, TL, false, false>(block);
 }
 template <bool BFS, bool COUNT>
 static const void *persistent_fn(int cont) {
@@ -1451,13 +1476,13 @@ static int use_cont(const gga_dev_work &w) { return GGA_CONT > 0 && w.bmin > 1u;
 // Level-synchronous BFS: worklist and persistent queries without the
 // continuation (which reaches levels out of order).
 extern "C" int ggak_level_sync(gga_dev_work w, int bfs) { return bfs && !use_cont(w); }
-static const void *pick_kernel(int persistent, int bfs, int count, uint32_t block, int cont) {
+static const void *pick_kernel(int persistent, int bfs, int count, uint32_t block, int cont, int spread) {
     if (persistent) {
         if (bfs) return count ? persistent_fn<true, true>(cont) : persistent_fn<true, false>(cont);
         return count ? persistent_fn<false, true>(cont) : persistent_fn<false, false>(cont);
     }
-    if (bfs) return count ? wl_fn<true, true, false>(block, cont) : wl_fn<true, false, false>(block, cont);
-    return count ? wl_fn<false, true, false>(block, cont) : wl_fn<false, false, false>(block, cont);
+    if (bfs) return count ? wl_fn<true, true, false>(block, cont, 0) : wl_fn<true, false, false>(block, cont, 0);
+    return count ? wl_fn<false, true, false>(block, cont, spread) : wl_fn<false, false, false>(block, cont, spread);
 }
 
 extern "C" int ggak_wl_step(gga_dev_graph g, gga_dev_work w, uint32_t step, int bfs, int count,
@@ -1465,9 +1490,9 @@ extern "C" int ggak_wl_step(gga_dev_graph g, gga_dev_work w, uint32_t step, int 
     if (grid == 0 || (block != 128 && block != 256 && block != 512)) return (int)hipErrorInvalidValue;
     void *args[] = {&g, &w, &step, &tl};
     // the instrumented variant always counts (its timeline goes with the work counters)
-    const int cont = use_cont(w);
-    const void *fn = tl ? (bfs ? wl_fn<true, true, true>(block, cont) : wl_fn<false, true, true>(block, cont))
-                        : pick_kernel(0, bfs, count, block, cont);
+    const int cont = use_cont(w), spread = w.sdist != nullptr;
+    const void *fn = tl ? (bfs ? wl_fn<true, true, true>(block, cont, 0) : wl_fn<false, true, true>(block, cont, spread))
+                        : pick_kernel(0, bfs, count, block, cont, spread);
     return (int)hipLaunchKernel(fn, dim3(grid), dim3(block), args, 0, s);
 }
 
@@ -1502,11 +1527,12 @@ extern "C" int ggak_conv(const uint32_t *dist, const uint32_t *fin, uint32_t n, 
 extern "C" int ggak_wl_phase(gga_dev_graph g, gga_dev_work w, uint32_t launch, int bfs, uint32_t grid, hipStream_t s) {
     if (grid == 0) return (int)hipErrorInvalidValue;
     if (bfs) {
-        if (use_cont(w)) k_wl_phase<true, true><<<grid, BLOCK, 0, s>>>(g, w, launch % 3u);
-        else k_wl_phase<true, false><<<grid, BLOCK, 0, s>>>(g, w, launch % 3u);
+        if (use_cont(w)) k_wl_phase<true, true, false><<<grid, BLOCK, 0, s>>>(g, w, launch % 3u);
+        else k_wl_phase<true, false, false><<<grid, BLOCK, 0, s>>>(g, w, launch % 3u);
     } else {
-        if (use_cont(w)) k_wl_phase<false, true><<<grid, BLOCK, 0, s>>>(g, w, launch % 3u);
-        else k_wl_phase<false, false><<<grid, BLOCK, 0, s>>>(g, w, launch % 3u);
+        if (use_cont(w)) k_wl_phase<false, true, false><<<grid, BLOCK, 0, s>>>(g, w, launch % 3u);
+        else if (w.sdist) k_wl_phase<false, false, true><<<grid, BLOCK, 0, s>>>(g, w, launch % 3u);
+        else k_wl_phase<false, false, false><<<grid, BLOCK, 0, s>>>(g, w, launch % 3u);
     }
     return launch_status();
 }
@@ -1546,7 +1572,7 @@ extern "C" uint32_t ggak_wl_grid(int device, int persistent, int bfs, int count,
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess) return 0;
     // (the continuation variants fit as many workgroups: same register cap,
     // LDS well within a CU's; persistent grids take one per CU either way)
-    const void *fn = pick_kernel(persistent, bfs, count, block, 0);
+    const void *fn = pick_kernel(persistent, bfs, count, block, 0, 0);
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, fn, (int)block, 0) != hipSuccess) return 0;
     if (per <= 0) return 0;
     // A grid barrier needs every workgroup resident at once.  On gfx950 the
@@ -1568,7 +1594,7 @@ extern "C" int ggak_persistent(gga_dev_graph g, gga_dev_work w, int bfs, int cou
         khz = 100000;  // 100 MHz
     uint64_t spin_ticks = (uint64_t)spin_limit_ms * (uint64_t)khz;
     void *args[] = {&g, &w, &max_steps, &spin_ticks};
-    hipError_t e = hipLaunchCooperativeKernel(pick_kernel(1, bfs, count, BLOCK, use_cont(w)), dim3(grid),
+    hipError_t e = hipLaunchCooperativeKernel(pick_kernel(1, bfs, count, BLOCK, use_cont(w), 0), dim3(grid),
                                               dim3(BLOCK), args, 0, s);
     if (e != hipSuccess) return (int)e;
     return launch_status();
