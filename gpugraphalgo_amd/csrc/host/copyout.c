@@ -158,6 +158,14 @@ hipError_t gga_copy_out(int device, hipStream_t s, void *dst, const void *src, u
         e = hipMemcpyAsync(dst, src, bytes, known ? hipMemcpyDefault : hipMemcpyDeviceToHost, s);
         return e == hipSuccess ? hipStreamSynchronize(s) : e;
     }
+    if (bytes <= FILL_MIN) {   /* one fill: nothing to overlap */
+        e = hipMemcpyAsync(t->pin, src, bytes, hipMemcpyDeviceToHost, s);
+        const hipError_t es = hipStreamSynchronize(s);
+        if (e == hipSuccess) e = es;
+        if (e == hipSuccess) memcpy(dst, t->pin, bytes);
+        set_give(t);
+        return e;
+    }
     copy_job j;
     memset(&j, 0, sizeof j);
     j.t = t;
@@ -198,6 +206,26 @@ hipError_t gga_copy_out(int device, hipStream_t s, void *dst, const void *src, u
     for (uint32_t i = 0; i < nth; i++) pthread_join(th[i], NULL);
     if (e == hipSuccess && atomic_load(&j.stop)) e = hipErrorUnknown;
     if (e != hipSuccess) hipStreamSynchronize(s);   /* nothing of this copy is left in flight */
+    set_give(t);
+    return e;
+}
+
+hipError_t gga_copy_out2(int device, hipStream_t s, void *dst0, const void *src0, uint64_t bytes0, void *dst1,
+                         const void *src1, uint64_t bytes1)
+{
+    slot_set *t = bytes0 && bytes1 && bytes0 + bytes1 <= FILL_MIN ? set_take(device) : NULL;
+    if (!t) {
+        const hipError_t e = gga_copy_out(device, s, dst0, src0, bytes0);
+        return e == hipSuccess ? gga_copy_out(device, s, dst1, src1, bytes1) : e;
+    }
+    hipError_t e = hipMemcpyAsync(t->pin, src0, bytes0, hipMemcpyDeviceToHost, s);
+    if (e == hipSuccess) e = hipMemcpyAsync(t->pin + bytes0, src1, bytes1, hipMemcpyDeviceToHost, s);
+    const hipError_t es = hipStreamSynchronize(s);
+    if (e == hipSuccess) e = es;
+    if (e == hipSuccess) {
+        memcpy(dst0, t->pin, bytes0);
+        memcpy(dst1, t->pin + bytes0, bytes1);
+    }
     set_give(t);
     return e;
 }

@@ -46,6 +46,9 @@ void gga_msbfs_release(void *state);
  * work queued on s; returns when dst holds them (copyout.c).  Handles that copy
  * out are counted: the pinned slots are given back with the last one. */
 hipError_t gga_copy_out(int device, hipStream_t s, void *dst, const void *src, uint64_t bytes);
+/* Two results, one wait when they are small. */
+hipError_t gga_copy_out2(int device, hipStream_t s, void *dst0, const void *src0, uint64_t bytes0, void *dst1,
+                         const void *src1, uint64_t bytes1);
 void gga_copy_retain(void);
 void gga_copy_release(void);
 

@@ -563,9 +563,8 @@ int gga_graph_chunks(gga_graph *g, uint32_t *chunk_begin, uint32_t *owner)
     HIP_TRY(hipSetDevice(g->device));
     /* the reference's table (NodeSplit's layout), also where the kernels walk a cut one */
     const uint32_t *cb = g->d_rcbeg ? g->d_rcbeg : g->d_cbeg, *co = g->d_rcown ? g->d_rcown : g->d_cown;
-    if (chunk_begin)
-        HIP_TRY(gga_copy_out(g->device, g->stream, chunk_begin, cb, 4ull * ((uint64_t)g->Cref + 1)));
-    if (owner) HIP_TRY(gga_copy_out(g->device, g->stream, owner, co, 4ull * g->Cref));
+    HIP_TRY(gga_copy_out2(g->device, g->stream, chunk_begin, cb, chunk_begin ? 4ull * ((uint64_t)g->Cref + 1) : 0u,
+                          owner, co, owner ? 4ull * g->Cref : 0u));
     return GGA_OK;
 fail:
     return rc;
