@@ -61,7 +61,7 @@ __device__ __forceinline__ void flush_pushes(const gga_dev_graph &g, const uint3
 }
 
 struct ListOut {
-    const uint32_t *cstart;  // first chunk of each vertex (n + 1)
+    const uint32_t *cstart;  // first chunk of each vertex (n + 1); NULL: chunk v is vertex v's only one
     uint32_t *q;             // output list
     uint32_t qcap;           // its capacity
     uint32_t *tiles;         // per-tile counts, then offsets (GGA_TILES(n) entries)
@@ -75,6 +75,12 @@ struct ListOut {
 // thread's ids go to consecutive positions.  Against vertices strided by
 // CBLOCK: R-MAT s22 SSSP 2.24 -> 2.18 ms, the 4096² grid's persistent BFS /
 // SSSP 9.5 / 15.4 -> 8.7 / 14.1 ms.
+//
+// On graphs with one chunk per vertex (meshes, cstart NULL) a chunk's id is its
+// vertex's: the 36 bytes of chunk starts per marked thread go unread, and the
+// write pass ends after its own ids when no thread of the tile has a long run
+// (one barrier, not three).  With the refill's stamps, SSSP on the 4096^2 grid with
+// 0.5% shortcuts 5.47 -> 5.03 ms.
 //
 // A predicate with vec8 reads the marks of a thread's eight vertices with one
 // or two vector loads (mark8: bit i for vertex v + i), and the marked
@@ -97,7 +103,13 @@ __device__ __forceinline__ uint32_t tile_items(const ListOut &o, uint32_t n, uin
                 cs[i] = 0;
                 nch[i] = 0;
             }
-            if (bits) {
+            if (bits && !o.cstart) {
+#pragma unroll
+                for (uint32_t i = 0; i < CITEMS; i++) {
+                    cs[i] = (uint32_t)vb + i;
+                    nch[i] = (bits >> i) & 1u;
+                }
+            } else if (bits) {
                 const uint4 a = *reinterpret_cast<const uint4 *>(o.cstart + vb);
                 const uint4 b = *reinterpret_cast<const uint4 *>(o.cstart + vb + 4);
                 const uint32_t c[9] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w, o.cstart[vb + 8]};
@@ -119,8 +131,8 @@ __device__ __forceinline__ uint32_t tile_items(const ListOut &o, uint32_t n, uin
         cs[i] = 0;
         nch[i] = 0;
         if (v < n && marked((uint32_t)v)) {
-            cs[i] = o.cstart[v];
-            nch[i] = o.cstart[v + 1] - cs[i];
+            cs[i] = o.cstart ? o.cstart[v] : (uint32_t)v;
+            nch[i] = o.cstart ? o.cstart[v + 1] - cs[i] : 1u;
         }
         mine += nch[i];
     }
@@ -194,6 +206,7 @@ __device__ __forceinline__ void write_items(const ListOut &o, const uint32_t *cs
             pending |= 1u << i;
         pos += nch[i];
     }
+    if (!__syncthreads_or(pending != 0u)) return;   // no long run in the tile (meshes: never)
     const uint32_t wv = threadIdx.x / GGA_WAVE, nw = blockDim.x / GGA_WAVE;
     for (;;) {
         if (threadIdx.x == 0) s_nb = 0;
@@ -248,7 +261,11 @@ __device__ __forceinline__ void compact_write_tiles(const ListOut &o, uint32_t n
     uint32_t off = 0, upto = 0;   // off = tiles[0] + ... + tiles[upto - 1]
     for (uint32_t t = blockIdx.x; t < ntiles; t += gridDim.x) {
         uint32_t part = 0, ex;
-        for (uint32_t i = upto + threadIdx.x; i < t; i += blockDim.x) part += o.tiles[i];
+        uint32_t i = upto + threadIdx.x;
+        // (four independent loads at a time: 8 192 tiles are 32 rounds a thread)
+        for (; i + 3u * blockDim.x < t; i += 4u * blockDim.x)
+            part += o.tiles[i] + o.tiles[i + blockDim.x] + o.tiles[i + 2u * blockDim.x] + o.tiles[i + 3u * blockDim.x];
+        for (; i < t; i += blockDim.x) part += o.tiles[i];
         off += block_excl_scan(part, ex, s_wave);
         upto = t;
         uint32_t cs[CITEMS], nch[CITEMS], excl;

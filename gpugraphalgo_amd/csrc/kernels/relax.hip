@@ -649,11 +649,11 @@ __device__ __forceinline__ void worklist_step(const gga_dev_graph &g, const gga_
     constexpr bool LVL = BFS && !CONT;
     const uint32_t wpb = blockDim.x / GGA_WAVE;   // waves per workgroup (128, 256 or 512 threads)
     const uint32_t waves = gridDim.x * wpb;
-    const uint32_t wid = blockIdx.x * wpb + __builtin_amdgcn_readfirstlane(threadIdx.x / GGA_WAVE);
     uint32_t bsz = w.bmin > 1u ? nq >> 10 : nq / ((LVL ? 8u : 16u) * waves);
     bsz = bsz < w.bmin ? w.bmin : bsz;
     bsz = bsz < 1u ? 1u : (bsz > GGA_WAVE ? GGA_WAVE : bsz);
     const uint32_t nbatch = (nq + bsz - 1) / bsz;
+    const uint32_t wid = blockIdx.x * wpb + __builtin_amdgcn_readfirstlane(threadIdx.x / GGA_WAVE);
     const bool flags = flag_step(w, nq);
     const uint32_t l = lane_id();
     const uint32_t thr = w.ctl[GGA_CTL_THR(step % 3u)];
@@ -778,7 +778,7 @@ __device__ __forceinline__ LevelMarked<WRITE> level_marked(const gga_dev_work &w
 // The single list of the plain layout for step `step`.
 __device__ __forceinline__ ListOut list_out(const gga_dev_graph &g, const gga_dev_work &w, uint32_t step) {
     ListOut o;
-    o.cstart = g.cstart;
+    o.cstart = g.C == g.n ? nullptr : g.cstart;   // every vertex has a chunk
     o.q = (step & 1u) ? w.q0 : w.q1;
     o.qcap = w.qcap;
     o.tiles = w.tiles;
@@ -870,15 +870,22 @@ __global__ __launch_bounds__(BLOCK) void k_compact_count(gga_dev_graph g, gga_de
 
 // ---- near-far refill: after a step whose next list came out empty, list
 // the deferred vertices (dist < last) under the next threshold.
+// The count pass stamps what it counts (flag[], all clear when a list is
+// empty), so that the write pass reads n bytes instead of dist and last again.
+__device__ __forceinline__ uint32_t stamps4(uint32_t bits) {   // byte i = bit i
+    return (bits & 1u) | (bits & 2u) << 7 | (bits & 4u) << 14 | (bits & 8u) << 21;
+}
 struct DeferredUnder {
     const uint32_t *dist, *last;
     uint32_t t;
-    uint32_t *mn = nullptr;   // when set: the smallest deferred distance seen (under t or not)
+    uint32_t *mn;    // the smallest deferred distance seen (under t or not)
+    uint8_t *flag;   // gets the stamps
     static constexpr bool vec8 = true;
     __device__ __forceinline__ bool operator()(uint32_t v) const {
         const uint32_t d = dist[v];
         const bool deferred = d < last[v];
-        if (mn && deferred && d < *mn) *mn = d;
+        if (deferred && d < *mn) *mn = d;
+        if (deferred && d < t) flag[v] = 1;
         return deferred && d < t;
     }
     // bit i: vertex v + i is deferred under t (v a multiple of 8); dist may
@@ -899,7 +906,8 @@ struct DeferredUnder {
                 m |= (d[i] < s[i] && d[i] < t) ? 1u << i : 0u;
                 lo = d[i] < s[i] && d[i] < lo ? d[i] : lo;
             }
-            if (mn && lo < *mn) *mn = lo;
+            if (lo < *mn) *mn = lo;
+            if (m) *reinterpret_cast<uint2 *>(flag + v) = make_uint2(stamps4(m), stamps4(m >> 4));
         } else {
 #pragma unroll
             for (uint32_t i = 0; i < 8; i++) m |= (*this)((uint32_t)(v + i)) ? 1u << i : 0u;
@@ -918,7 +926,7 @@ __device__ __forceinline__ void refill_count_body(const gga_dev_graph &g, const 
                                                   uint32_t *s_wave, uint32_t *s_min) {
     const ListOut o = list_out(g, w, step);
     uint32_t m = 0xFFFFFFFFu;   // the thread's smallest deferred distance, gathered by the count
-    const DeferredUnder pred{w.dist, w.last, sat_add(w.ctl[GGA_CTL_THR((step + 1u) % 3u)], w.delta), &m};
+    const DeferredUnder pred{w.dist, w.last, sat_add(w.ctl[GGA_CTL_THR((step + 1u) % 3u)], w.delta), &m, w.flag};
     for (uint32_t t = blockIdx.x; t < GGA_TILES(g.n); t += gridDim.x) {
         m = 0xFFFFFFFFu;
         compact_count_tile(o, g.n, t, pred, s_wave);
@@ -979,8 +987,8 @@ __device__ __forceinline__ void refill_scan_body(const gga_dev_graph &g, const g
 __device__ __forceinline__ void refill_write_body(const gga_dev_graph &g, const gga_dev_work &w, uint32_t step,
                                                   uint32_t *s_wave, uint32_t *stage) {
     const ListOut o = list_out(g, w, step);
-    const DeferredUnder pred{w.dist, w.last, w.ctl[GGA_CTL_RTHR]};
-    for (uint32_t t = blockIdx.x; t < GGA_TILES(g.n); t += gridDim.x) compact_write_tile(o, g.n, t, pred, s_wave, stage);
+    for (uint32_t t = blockIdx.x; t < GGA_TILES(g.n); t += gridDim.x)
+        compact_write_tile(o, g.n, t, StampMarked<true>{w.flag}, s_wave, stage);
 }
 
 // The standalone refill is two launches: its count runs in the compaction's
@@ -1060,7 +1068,7 @@ __device__ __forceinline__ void refill_list_body(const gga_dev_graph &g, const g
         }
         __syncthreads();
     }
-    compact_write_tiles(o, g.n, DeferredUnder{w.dist, w.last, t1}, s_wave, stage);
+    compact_write_tiles(o, g.n, StampMarked<true>{w.flag}, s_wave, stage);
 }
 
 __global__ __launch_bounds__(BLOCK) void k_refill_write(gga_dev_graph g, gga_dev_work w, uint32_t step) {
