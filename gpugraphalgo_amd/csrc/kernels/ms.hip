@@ -238,7 +238,7 @@ __device__ __forceinline__ void follow_pairs(const gga_dev_graph &g, const gga_d
         }
         __builtin_amdgcn_wave_barrier();   // the entries are read before the pushes below write the queue
         for (uint32_t j = sub;; j += 4u) {
-            uint32_t v[G], a[G], dv[G];
+            uint32_t v[G], a[G];
             bool act[G];
 #pragma unroll
             for (uint32_t i = 0; i < G; i++) {
@@ -251,13 +251,8 @@ __device__ __forceinline__ void follow_pairs(const gga_dev_graph &g, const gga_d
 #pragma unroll
             for (uint32_t i = 0; i < G; i++) {
                 if (i * PER >= take) break;
-                dv[i] = ms.D[LM ? (uint64_t)sl[i] * g.n + v[i] : (uint64_t)v[i] * LANES + sl[i]];
-            }
-#pragma unroll
-            for (uint32_t i = 0; i < G; i++) {
-                if (i * PER >= take) break;
                 const uint32_t thr = (uint32_t)__shfl(thr_s, (int)sl[i], GGA_WAVE);
-                const bool pass = act[i] && a[i] >= du[i] && a[i] < inf && a[i] < dv[i];
+                const bool pass = act[i] && a[i] >= du[i] && a[i] < inf;   // (no guard read, see above)
                 const bool imp = relax_pair<LM, true>(g, ms, pass, v[i], sl[i], a[i], thr, cq, qh, qt, list);
                 if (COUNT) {
                     cnt.edges += (uint32_t)__popcll(__ballot(act[i]));

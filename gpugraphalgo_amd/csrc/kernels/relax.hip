@@ -187,9 +187,11 @@ __device__ __forceinline__ bool queue_near(bool near, uint32_t x, uint32_t d, ui
 // What bounds it: the chain of dependent accesses of a round.  A queue entry
 // holds the vertex's edge range, fetched beside the atomic that lowered it,
 // and four neighbouring lanes take a vertex's edges (four at a time), so a
-// round needs no chunk lookup, scan or owner search: edge, dist[v], atomic
-// (it was chunk start, chunk bounds, edge, dist[v], atomic, behind a
-// 6-shuffle search).  With the queue of 512, SSSP: pure 1024^2 grid 8.9 -> 6.2
+// round needs no chunk lookup, scan or owner search; and with no guard read
+// before the atomic it is two accesses, edge and atomic (it was chunk start,
+// chunk bounds, edge, dist[v], atomic, behind a 6-shuffle search).  A thin
+// front leaves the atomic units idle: without the guard SSSP on a pure 1024^2
+// grid went from 4.70 to 4.08 ms, on a 100 x 77 grid from 0.47 to 0.40.  With the queue of 512, SSSP: pure 1024^2 grid 8.9 -> 6.2
 // ms, a 100 x 77 grid 0.80 -> 0.60, 4096^2 with shortcuts 6.8 -> 6.3; BFS on
 // the pure 1024^2 / 4096^2 grid 4.1-4.6 -> 2.9-3.2 / 19-25 -> 13-18 ms.
 template <bool BFS, bool COUNT, int OUT>
@@ -249,12 +251,7 @@ __device__ __forceinline__ void follow_front(const gga_dev_graph &g, const gga_d
 #pragma unroll
             for (uint32_t u = 0; u < G; u++) {
                 if (u * PER >= take) break;
-                cur[u] = dist[v[u]];
-            }
-#pragma unroll
-            for (uint32_t u = 0; u < G; u++) {
-                if (u * PER >= take) break;
-                act[u] = act[u] && alt[u] >= du[u] && alt[u] < inf && alt[u] < cur[u];
+                act[u] = act[u] && alt[u] >= du[u] && alt[u] < inf;
                 if (act[u]) {
                     cur[u] = atomic_min_u32(&dist[v[u]], alt[u]);
                     r0[u] = g.row[v[u]];
