@@ -72,6 +72,14 @@ int ggak_wl_phase(gga_dev_graph g, gga_dev_work w, uint32_t launch, int bfs, uin
  * pinned memory by its device address; the distances -> stage (n words,
  * likewise; NULL: not). */
 int ggak_finish(gga_dev_graph g, gga_dev_work w, uint32_t *host, uint32_t *stage, uint32_t *blocks, hipStream_t s);
+/* A whole query on a graph of at most GGA_SMALL_N vertices in one launch of
+ * one workgroup: w.dist, and through `host` (as ggak_finish: one row of
+ * partials) steps, clock and ctl[TAIL(0)], which is not 0 when the step cap
+ * w.cap ended it.  thin: few edges a vertex, thin fronts; SSSP then runs
+ * near-far with buckets of w.delta (> 0). */
+#define GGA_SMALL_N 12288u   /* 12 bytes of LDS a vertex: 155 KB of 160 with the tables */
+int ggak_small(gga_dev_graph g, gga_dev_work w, uint32_t src, int bfs, int thin, uint32_t *host, uint32_t *stage,
+               hipStream_t s);
 /* Occupancy-bound grid (workgroups of `block` threads) for the worklist
  * kernel, or for the persistent kernel (always 256 threads); 0 on error. */
 uint32_t ggak_wl_grid(int device, int persistent, int bfs, int count, uint32_t block);

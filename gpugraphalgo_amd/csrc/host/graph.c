@@ -708,6 +708,8 @@ typedef struct query_plan {
     uint32_t src, max_iters, epoch;
     uint32_t *stage;   /* pinned area for the distances (device address), or NULL */
     int staged;        /* set when the query left them there */
+    int small, thin;   /* the whole query in one workgroup (ggak_small); ... of few edges a vertex */
+    uint32_t small_delta;
 } query_plan;
 
 static int run_query(gga_graph *g, gga_dev_graph dg, gga_dev_work dw, query_plan *p, gga_opts *o,
@@ -735,6 +737,22 @@ static int run_query(gga_graph *g, gga_dev_graph dg, gga_dev_work dw, query_plan
                        !(own && (o->timeline || o->conv_rows));
     *adv = 0;
 
+    if (p->small) {
+        dw.cap = max_iters;
+        dw.delta = p->small_delta;
+        K_TRY(ggak_small(dg, dw, p->src, bfs, p->thin, g->d_pin, p->stage, g->stream));
+        HIP_TRY(hipStreamSynchronize(g->stream));
+        s->launches = 1;
+        fin = 1;
+        ended = 1;
+        if (g->h_pin[GGA_CTL_TAIL(0)]) {
+            rc = GGA_ETIMEDOUT;
+            gga_set_error("worklist mode: %u steps without convergence", dw.cap);
+            goto fail;
+        }
+        p->staged = p->stage != NULL;
+        goto done;
+    }
     if (!phased) HIP_TRY(hipEventRecord(g->ev[0], g->stream)); /* bfs_sssp.cu:350 */
     K_TRY(ggak_query_init(dg, dw, p->src, p->epoch, g->stream));
     if (mode == GGA_MODE_TOPO) {
@@ -927,6 +945,7 @@ static int run_query(gga_graph *g, gga_dev_graph dg, gga_dev_work dw, query_plan
         HIP_TRY(hipEventElapsedTime(&ktime, g->ev[2], g->ev[3]));
         s->launches = 1;
     }
+done:
     if (!ended) {
         HIP_TRY(hipEventRecord(g->ev[1], g->stream));          /* bfs_sssp.cu:469 */
         K_TRY(ggak_reach(dg, dw, g->stream));
@@ -986,7 +1005,7 @@ static int run_query(gga_graph *g, gga_dev_graph dg, gga_dev_work dw, query_plan
     }
     s->ktime_ms = ktime;
     s->sktime_ms = 0.f;
-    g->last_steps[bfs ? 1 : 0] = s->iterations;
+    if (!p->small) g->last_steps[bfs ? 1 : 0] = s->iterations;   /* (its steps say nothing of a launch's) */
     dfree(g, (void **)&d_tl, tl_bytes);
     dfree(g, (void **)&d_fin, fin_bytes);
     dfree(g, (void **)&d_conv, conv_bytes);
@@ -1017,6 +1036,31 @@ static void plan_query(const gga_graph *g, int bfs, const gga_opts *o, query_pla
     const int near_far = !bfs && (mode == GGA_MODE_WORKLIST || mode == GGA_MODE_PERSISTENT) && d != 0u;
     *delta = near_far ? d : 0u;
     p->max_iters = o->max_iters ? o->max_iters : (g->n + 1u);
+    /* A query that leaves the schedule to the library, on a graph that one
+     * workgroup holds in LDS.  Thin fronts first: a mesh of at most 6 edges a
+     * vertex gains at every size that fits (SSSP / BFS, general -> one
+     * workgroup: 30 x 40 grid 148 / 80 -> 51 / 33 us, 100 x 77 301 / 170 ->
+     * 164 / 93, 110 x 111 413 / 219 -> 244 / 126, 16 x 700 1593 / 720 -> 765 /
+     * 407).  Elsewhere one CU's rate decides: R-MAT of 3.6 k edges 76 / 47 -> 25
+     * / 14 us, 15 k 126 / 58 -> 79 / 33, 20 k 127 / 55 -> 120 / 39, 31 k 140 / 51
+     * -> 177 / 58. */
+    const int thin = mesh_like(g) && g->m <= 6ull * g->n;
+    p->small = (o->mode == GGA_MODE_AUTO || o->mode == GGA_MODE_WORKLIST) && !p->count && !o->timeline &&
+               !o->conv_rows && !o->grid && !o->block && !o->dense_min && !o->delta && !o->sync_every &&
+               !o->max_iters && g->n <= GGA_SMALL_N && (thin || g->m <= 16384u);
+    if (p->small) {
+        /* near-far (thin SSSP): buckets twice as wide as the general path's --
+         * a refill is two barriers here -- at 1 / 2 / 4 times: 100 x 77 grid
+         * 174 / 164 / 173 us, 16 x 700 851 / 765 / 741, 110 x 111 with
+         * shortcuts 140 / 139 / 178; without buckets 160 / 1649 / 148 */
+        const uint32_t width = auto_delta(g, 0);
+        p->mode = GGA_MODE_WORKLIST;
+        p->thin = thin;
+        p->max_iters = 64u * (g->n + 1u);
+        *delta = 0u;
+        p->small_delta = width ? (width < 0x7FFFFFFFu ? 2u * width : width) : 0xFFFFFFFFu;
+        return;
+    }
     if (!o->max_iters && near_far)
         p->max_iters = (uint64_t)64u * (g->n + 1u) < 0xFFFFFFF0ull ? 64u * (g->n + 1u) : 0xFFFFFFF0u;
 }

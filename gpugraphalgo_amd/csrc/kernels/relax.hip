@@ -1312,6 +1312,222 @@ __global__ __launch_bounds__(BLOCK) void k_finish(gga_dev_graph g, gga_dev_work 
     }
 }
 
+// ------------------------------------------------------ small graphs
+// A whole query in one launch of one workgroup: distances, row offsets and both
+// frontier queues in LDS (12 bytes a vertex), col and w read from L2.  On a
+// graph this small every step is a chain of dependent accesses whatever the
+// grid, and the launches around it cost more than the step: here a step is an
+// LDS read, one edge load, an LDS atomic and a workgroup barrier (0.9 us on a
+// 100 x 77 grid).  What bounds it: that chain on meshes, one CU's rate of
+// edges elsewhere (plan_query in host/graph.c has the sizes).
+//
+// A vertex waits in the next queue at most once (bit in `mark`).  Taking it
+// from the queue clears the bit before its distance is read, so an
+// improvement either comes before that read or queues the vertex again.
+//
+// MESH: few edges a vertex; SSSP then lists only distances under a threshold
+// (near-far, buckets of w.delta): the others set the vertex's bit in `far`, and
+// an empty queue is refilled from those under the next threshold.
+constexpr uint32_t SMALL_BLOCK = 1024, SMALL_WAVES = SMALL_BLOCK / GGA_WAVE;
+template <bool BFS, bool MESH>
+__global__ __launch_bounds__(SMALL_BLOCK) void k_small(gga_dev_graph g, gga_dev_work w, uint32_t src, uint32_t *host,
+                                                       uint32_t *stage) {
+    extern __shared__ __align__(16) uint32_t lds[];
+    constexpr bool NEAR = MESH && !BFS;
+    __shared__ uint2 s_tab[MESH ? 1 : SMALL_WAVES][GGA_WAVE];
+    __shared__ uint64_t s_red[2][SMALL_WAVES];
+    __shared__ uint32_t s_len[3], s_low;
+    const uint32_t n = g.n, inf = w.inf, l = lane_id();
+    const uint32_t wv = __builtin_amdgcn_readfirstlane(threadIdx.x / GGA_WAVE);
+    uint32_t *const dist = lds, *const row = dist + n, *const mark = row + n + 1u;
+    uint32_t *const far = mark + (n + 31u) / 32u;   // (near-far only)
+    uint16_t *const q0 = reinterpret_cast<uint16_t *>(NEAR ? far + (n + 31u) / 32u : far), *const q1 = q0 + n;
+    uint2 *const tab = s_tab[MESH ? 0 : wv];
+    uint32_t thr = NEAR ? w.delta : 0xFFFFFFFFu;
+    uint64_t t0 = 0;
+    if (threadIdx.x == 0) t0 = wall_clock64();
+    for (uint32_t v = threadIdx.x; v < n; v += SMALL_BLOCK) {
+        dist[v] = v == src ? 0u : inf;
+        row[v] = g.row[v];
+    }
+    for (uint32_t i = threadIdx.x; i < (n + 31u) / 32u; i += SMALL_BLOCK) {
+        mark[i] = 0u;
+        if (NEAR) far[i] = 0u;
+    }
+    if (threadIdx.x == 0) {
+        row[n] = g.m;
+        q0[0] = (uint16_t)src;
+        s_len[0] = 1u;
+        s_len[1] = s_len[2] = 0u;
+    }
+    __syncthreads();
+    uint32_t step = 0, cur = 0, nf;
+    for (;; step++) {
+        nf = s_len[cur];
+        if (NEAR && nf == 0u) {
+            // the deferred vertices under the next threshold, which starts at
+            // the smallest of them when the bucket after this one is empty
+            if (threadIdx.x == 0) s_low = 0xFFFFFFFFu;
+            __syncthreads();
+            uint32_t low = 0xFFFFFFFFu;
+            for (uint32_t v = threadIdx.x; v < n; v += SMALL_BLOCK)
+                if ((far[v >> 5] >> (v & 31u)) & 1u) low = dist[v] < low ? dist[v] : low;
+            if (low != 0xFFFFFFFFu) atomicMin(&s_low, low);
+            __syncthreads();
+            low = s_low;
+            if (low == 0xFFFFFFFFu) break;
+            thr = sat_add(low > thr ? low : thr, w.delta);
+            uint16_t *const qin = (step & 1u) ? q1 : q0;
+            for (uint32_t v = threadIdx.x; v < n; v += SMALL_BLOCK)
+                if (((far[v >> 5] >> (v & 31u)) & 1u) && dist[v] < thr) {
+                    atomicOr(&mark[v >> 5], 1u << (v & 31u));
+                    qin[atomicAdd(&s_len[cur], 1u)] = (uint16_t)v;
+                }
+            __syncthreads();
+            nf = s_len[cur];
+        }
+        if (nf == 0u || step >= w.cap) break;   // (the same for every thread)
+        const uint32_t nxt = cur == 2u ? 0u : cur + 1u;
+        // the slot after the next: read last in the step before, filled in the next one
+        if (threadIdx.x == 0) s_len[nxt == 2u ? 0u : nxt + 1u] = 0u;
+        const uint16_t *const qin = (step & 1u) ? q1 : q0;
+        uint16_t *const qout = (step & 1u) ? q0 : q1;
+        // lowers dist[v] to alt where `on` and queues v; whole-wave call
+        auto relax = [&](bool on, uint32_t v, uint32_t alt) {
+            bool push = false;
+            if (on && alt < __hip_atomic_fetch_min(&dist[v], alt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)) {
+                const uint32_t bit = 1u << (v & 31u);
+                if (NEAR && alt >= thr) atomicOr(&far[v >> 5], bit);
+                else
+                    push = !(__hip_atomic_fetch_or(&mark[v >> 5], bit, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_WORKGROUP) &
+                             bit);
+            }
+            const uint64_t pm = __ballot(push);
+            if (pm) {
+                uint32_t at = 0;
+                if (l == 0) at = atomicAdd(&s_len[nxt], (uint32_t)__popcll(pm));
+                at = wave_bcast(at, 0) + __builtin_amdgcn_mbcnt_hi((uint32_t)(pm >> 32),
+                                                                  __builtin_amdgcn_mbcnt_lo((uint32_t)pm, 0u));
+                if (push) qout[at] = (uint16_t)v;   // (a vertex once: at < n)
+            }
+        };
+        // out of the queue: its distance from now on.  (Its distance is under
+        // the threshold, so no deferral of it can follow.)
+        auto take = [&](uint32_t x) {
+            if (NEAR) atomicAnd(&far[x >> 5], ~(1u << (x & 31u)));
+            __hip_atomic_fetch_and(&mark[x >> 5], ~(1u << (x & 31u)), __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_WORKGROUP);
+            return __hip_atomic_load(&dist[x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        };
+        if (MESH) {
+            // four neighbouring lanes a vertex, four edges at a time: no scan,
+            // no owner search (as in follow_front)
+            for (uint32_t b = wv * 16u; b < nf; b += SMALL_WAVES * 16u) {
+                const uint32_t i = b + (l >> 2);
+                uint32_t eb = 0, ne = 0, du = inf;
+                if (i < nf) {
+                    const uint32_t x = qin[i];
+                    du = take(x);
+                    eb = row[x];
+                    ne = row[x + 1u] - eb;
+                }
+                for (uint32_t j = l & 3u; __ballot(j < ne) != 0ull; j += 4u) {
+                    const bool on = j < ne;
+                    const uint32_t e = on ? eb + j : 0u;   // (some lane has an edge: slot 0 is in bounds)
+                    const uint32_t v = g.col[e], alt = du + (BFS ? 1u : g.w[e]);
+                    relax(on && alt >= du && alt < inf, v, alt);
+                }
+            }
+            cur = nxt;
+            __syncthreads();
+            continue;
+        }
+        uint32_t bsz = (nf + SMALL_WAVES - 1u) / SMALL_WAVES;
+        bsz = bsz < GGA_WAVE ? bsz : GGA_WAVE;
+        const uint32_t half = bsz <= 1u ? 0u : 1u << (31 - __builtin_clz(bsz - 1u));
+        for (uint32_t b = wv * bsz; b < nf; b += SMALL_WAVES * bsz) {
+            uint32_t eb = 0, ne = 0, du = inf;
+            if (l < bsz && b + l < nf) {
+                const uint32_t x = qin[b + l];
+                du = take(x);
+                eb = row[x];
+                ne = row[x + 1u] - eb;
+            }
+            const uint32_t incl = wave_incl_scan(ne);
+            const uint32_t total = wave_last(incl);
+            tab[l] = make_uint2(eb - (incl - ne), du);   // (as in expand_batch)
+            __builtin_amdgcn_wave_barrier();
+            for (uint32_t base = 0; base < total; base += GGA_WAVE * UNROLL) {
+                uint32_t v[UNROLL], alt[UNROLL], ds[UNROLL], kk[UNROLL], own[UNROLL];
+                const uint32_t left = total - base;
+#pragma unroll
+                for (uint32_t u = 0; u < UNROLL; u++) {
+                    const uint32_t k = base + u * GGA_WAVE + l;
+                    kk[u] = k < total ? k : total - 1u;
+                    own[u] = 0;
+                }
+                for (uint32_t s = half; s != 0; s >>= 1) {
+#pragma unroll
+                    for (uint32_t u = 0; u < UNROLL; u++) {
+                        const uint32_t y = __shfl(incl, (int)(own[u] + s - 1), GGA_WAVE);
+                        own[u] += y <= kk[u] ? s : 0u;
+                    }
+                }
+#pragma unroll
+                for (uint32_t u = 0; u < UNROLL; u++) {
+                    if (u * GGA_WAVE >= left) break;
+                    const uint2 t = tab[own[u]];
+                    ds[u] = t.y;
+                    v[u] = g.col[t.x + kk[u]];
+                    alt[u] = t.y + (BFS ? 1u : g.w[t.x + kk[u]]);
+                }
+#pragma unroll
+                for (uint32_t u = 0; u < UNROLL; u++) {
+                    if (u * GGA_WAVE >= left) break;
+                    relax(base + u * GGA_WAVE + l < total && alt[u] >= ds[u] && alt[u] < inf && alt[u] < dist[v[u]],
+                          v[u], alt[u]);
+                }
+            }
+            __builtin_amdgcn_wave_barrier();
+        }
+        cur = nxt;
+        __syncthreads();
+    }
+    uint64_t reached = 0, mr = 0;
+    for (uint32_t v = threadIdx.x; v < n; v += SMALL_BLOCK) {
+        const uint32_t d = dist[v];
+        w.dist[v] = d;
+        if (stage) stage[v] = d;
+        if (d < inf) {
+            reached += 1u;
+            mr += row[v + 1u] - row[v];
+        }
+    }
+    reached = wave_sum64(reached);
+    mr = wave_sum64(mr);
+    if (l == 0) {
+        s_red[0][wv] = reached;
+        s_red[1][wv] = mr;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        uint64_t *part = reinterpret_cast<uint64_t *>(host + GGA_FIN_PART);
+        uint64_t *clock = reinterpret_cast<uint64_t *>(host + GGA_FIN_CLOCK);
+        reached = mr = 0;
+        for (uint32_t i = 0; i < SMALL_WAVES; i++) {
+            reached += s_red[0][i];
+            mr += s_red[1][i];
+        }
+        part[0] = reached;
+        part[1] = mr;
+        clock[0] = t0;
+        clock[1] = wall_clock64();
+        for (uint32_t i = 0; i < 3; i++) host[GGA_CTL_ITER(i)] = w.epoch;   // (no stamps taken)
+        host[GGA_CTL_STEPS] = step;
+        host[GGA_CTL_ERR] = 0u;
+        host[GGA_CTL_TAIL(0)] = nf;   // not 0: the step cap
+    }
+}
+
 // Fingerprint of dist: sum over v of mix64(v << 32 | dist[v]) (the host's
 // gga_checksum); partials in word 3 of cnt slots [0, REACH_BLOCKS), folded
 // into ctl[RED + 4] (uint64).
@@ -1547,6 +1763,22 @@ extern "C" int ggak_finish(gga_dev_graph g, gga_dev_work w, uint32_t *host, uint
     *blocks = grid_for(g.n, GGA_FIN_BLOCKS);
     k_finish<<<*blocks, BLOCK, 0, s>>>(g, w, host, stage);
     return launch_status();
+}
+
+static uint32_t small_bytes(uint32_t n) { return 4u * n + 4u * (n + 1u) + 8u * ((n + 31u) / 32u) + 4u * n; }
+
+extern "C" int ggak_small(gga_dev_graph g, gga_dev_work w, uint32_t src, int bfs, int thin, uint32_t *host, uint32_t *stage,
+                          hipStream_t s) {
+    if (g.n == 0 || g.n > GGA_SMALL_N || src >= g.n || (thin && !bfs && w.delta == 0u)) return (int)hipErrorInvalidValue;
+    const uint32_t bytes = small_bytes(g.n);
+    const void *fn = bfs ? (thin ? reinterpret_cast<const void *>(&k_small<true, true>)
+                                 : reinterpret_cast<const void *>(&k_small<true, false>))
+                         : (thin ? reinterpret_cast<const void *>(&k_small<false, true>)
+                                 : reinterpret_cast<const void *>(&k_small<false, false>));
+    hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)small_bytes(GGA_SMALL_N));
+    if (e != hipSuccess) return (int)e;
+    void *args[] = {&g, &w, &src, &host, &stage};
+    return (int)hipLaunchKernel(fn, dim3(1), dim3(SMALL_BLOCK), args, bytes, s);
 }
 
 extern "C" int ggak_refill(gga_dev_graph g, gga_dev_work w, uint32_t step, hipStream_t s) {
