@@ -10,8 +10,8 @@
 //
 // Layout: D[v * 32 + lane] (one 128-byte line per vertex).  A half wave
 // relaxes one edge for all 32 lanes: lane s of the half reads dist[u][s] and
-// dist[v][s] (both one coalesced line), col[e] / w[e] are broadcast loads,
-// and the lanes that improved are published with one atomicOr into the
+// dist[v][s] (both one coalesced line), the edge itself comes through LDS,
+// where the wave staged 64 of them, and the lanes that improved are published with one atomicOr into the
 // destination's next mask.  A batch whose chunks carry few lanes each (lanes
 // started far apart on a mesh rarely meet) is instead flattened into
 // (edge, lane) pairs, one per wave lane, so idle lanes cost no slots.  The next list, chosen per step from the length of
@@ -45,10 +45,12 @@ constexpr uint32_t MS_UNROLL = GGA_MS_UNROLL;  // edges per half wave per round
 #define GGA_MS_FLAT_UNROLL 1
 #endif
 constexpr uint32_t FLAT_UNROLL = GGA_MS_FLAT_UNROLL;
+// a batch averaging at most GGA_MS_FLAT lanes per edge slot is flattened (32
+// SSSP lanes on R-MAT s20 at 4 / 6 / 8 / 10 / 16: 3.62 / 3.62 / 3.64 / 3.73 /
+// 4.51 ms; meshes equal: their lanes rarely meet)
 #ifndef GGA_MS_FLAT
-#define GGA_MS_FLAT 16
+#define GGA_MS_FLAT 6
 #endif
-// a batch averaging at most GGA_MS_FLAT lanes per edge slot is flattened
 constexpr uint32_t PBUF = 256;                 // pushed vertices staged per wave before a flush
 // Mesh engines: (vertex, lane) pairs a wave may follow past its batch within
 // one step (0: off), the wave's LDS queue of them, 16-pair groups expanded per
@@ -289,7 +291,8 @@ __device__ __forceinline__ void ms_relax(const gga_dev_graph &g, const gga_dev_m
     const uint32_t nbatch = (nq + bsz - 1) / bsz;
     const uint32_t l = lane_id(), half = l >> 5, s = l & (LANES - 1u);
     const uint32_t unit_word = ms.ctl[GGA_CTL_UNIT];
-    const bool unit = (unit_word >> s) & 1u;
+    const uint32_t bit = 1u << s;
+    const bool unit = (unit_word & bit) != 0u;
     // near-far: an improvement at or beyond the lane's threshold lowers the
     // distance but is deferred (no mask bit, a far bit instead) until a refill
     // reaches it
@@ -385,80 +388,99 @@ __device__ __forceinline__ void ms_relax(const gga_dev_graph &g, const gga_dev_m
             if (CONT && qt != 0u) follow_pairs<COUNT, LM>(g, ms, unit_word, thr_s, cq, qt, list_pair, cnt);
             continue;
         }
-        // edge slot k goes to half (k & 1); slots past the end are clamped to
-        // the last slot so every address below is in bounds
-        for (uint32_t base = 0; base < total; base += 2u * MS_UNROLL) {
-            uint32_t v[MS_UNROLL], wt[MS_UNROLL], du[MS_UNROLL], dv[MS_UNROLL], mm[MS_UNROLL];
-            bool act[MS_UNROLL];
-#pragma unroll
-            for (uint32_t i = 0; i < MS_UNROLL; i++) {
-                const uint32_t k = base + 2u * i + half;
-                act[i] = k < total;
-                const uint32_t kk = act[i] ? k : total - 1u;
+        // 64 edge slots at a time: one per wave lane for the owner search and
+        // the edge, then through LDS two slots (one a half wave) per
+        // relaxation.  Slots past the end are clamped to the last one with an
+        // empty mask, so every address below is in bounds.  Instruction issue
+        // bounds the heavy steps when each half wave searches its own slots
+        // (some 44 vector instructions an edge, 1.0 - 1.1 ms a heavy step of
+        // 32 SSSP lanes on R-MAT s20; now 10, 0.7 ms, with 18.6 M 128-byte
+        // reads and 9.5 M atomic requests behind it): a drain 5.49 -> 3.64 ms,
+        // and 3.39 with no wait for the atomicMin's old value.  That value
+        // only told whether this wave or another lowered the distance past
+        // the guard within the step; whichever it was, the vertex is listed,
+        // so a lane bit set for both adds nothing.  (8 slots a half wave in
+        // flight instead of 4: 4.10 ms at half the waves, 2: 3.90.)
+        for (uint32_t base = 0; base < total; base += GGA_WAVE) {
+            {
+                const uint32_t k = base + l, kk = k < total ? k : total - 1u;
                 const uint32_t j = wave_owner(incl, kk);
                 const uint32_t e = wave_bcast(eb, j) + (kk - wave_bcast(excl, j));
-                const uint32_t uu = wave_bcast(u, j);
-                mm[i] = wave_bcast(m, j);
-                v[i] = g.col[e];
-                wt[i] = g.w[e];
-                // vertex-major: the whole line comes in anyway, every lane loads;
-                // lane-major: only the lanes to relax gather their own word
-                if (LM) du[i] = ((mm[i] >> s) & 1u) ? D[(uint64_t)s * g.n + uu] : inf;
-                else du[i] = D[(uint64_t)uu * LANES + s];
+                const uint32_t uu = wave_bcast(u, j), mj = wave_bcast(m, j);
+                cq[l] = make_uint4(g.col[e], g.w[e], uu, k < total ? mj : 0u);
+                __builtin_amdgcn_wave_barrier();
             }
+            const uint32_t left = total - base < GGA_WAVE ? total - base : GGA_WAVE;
+            for (uint32_t r = 0; r < left; r += 2u * MS_UNROLL) {
+                uint32_t v[MS_UNROLL], wt[MS_UNROLL], du[MS_UNROLL], dv[MS_UNROLL], mm[MS_UNROLL];
 #pragma unroll
-            for (uint32_t i = 0; i < MS_UNROLL; i++) {
-                if (LM) dv[i] = ((mm[i] >> s) & 1u) ? D[(uint64_t)s * g.n + v[i]] : 0u;
-                else dv[i] = D[(uint64_t)v[i] * LANES + s];
-            }
+                for (uint32_t i = 0; i < MS_UNROLL; i++) {
+                    const uint4 t = cq[r + 2u * i + half];   // (r + 2 i + half < 64)
+                    v[i] = t.x;
+                    wt[i] = t.y;
+                    mm[i] = t.w;
+                    // vertex-major: the whole line comes in anyway, every lane loads;
+                    // lane-major: only the lanes to relax gather their own word
+                    if (LM) du[i] = ((t.w >> s) & 1u) ? D[(uint64_t)s * g.n + t.z] : inf;
+                    else du[i] = D[(uint64_t)t.z * LANES + s];
+                    if (LM) dv[i] = ((t.w >> s) & 1u) ? D[(uint64_t)s * g.n + t.x] : 0u;
+                    else dv[i] = D[(uint64_t)t.x * LANES + s];
+                }
 #pragma unroll
-            for (uint32_t i = 0; i < MS_UNROLL; i++) {
-                const bool on = act[i] && ((mm[i] >> s) & 1u) && du[i] < inf;
-                const uint32_t a = du[i] + (unit ? 1u : wt[i]);
-                bool imp = false;
-                if (on && a >= du[i] && a < inf && a < dv[i]) {
-                    const uint32_t old =
-                        atomic_min_u32(&D[LM ? (uint64_t)s * g.n + v[i] : (uint64_t)v[i] * LANES + s], a);
-                    imp = a < old;
-                }
-                const uint64_t bal = __ballot(imp && a < thr_s);
-                const uint32_t hm = (uint32_t)(bal >> (32u * half));
-                bool first = false;
-                if (s == 0 && hm) {
-                    first = __hip_atomic_fetch_or(&mnxt[v[i]], hm, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0u;
-                    __hip_atomic_fetch_or(nl, hm, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
-                }
-                if (ms.far) {
-                    const uint32_t fm = (uint32_t)(__ballot(imp && a >= thr_s) >> (32u * half));
-                    if (s == 0 && fm) {
-                        atomicOr(&ms.far[v[i]], fm);
-                        if ((ms.tfar[v[i] >> 6] & fm) != fm) atomicOr(&ms.tfar[v[i] >> 6], fm);
+                for (uint32_t i = 0; i < MS_UNROLL; i++) {
+                    const bool on = (mm[i] & bit) != 0u;
+                    const uint32_t a = du[i] + (unit ? 1u : wt[i]);
+                    bool imp = false;
+                    if (on && a >= du[i] && a < dv[i]) {   // (dv <= inf: a finite sum of a finite du)
+                        uint32_t *const at = &D[LM ? (uint64_t)s * g.n + v[i] : (uint64_t)v[i] * LANES + s];
+                        if (COUNT) imp = a < atomic_min_u32(at, a);
+                        else {
+                            __hip_atomic_fetch_min(at, a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                            imp = true;   // nobody waits for the old value: see above
+                        }
+                    }
+                    const uint64_t any = __ballot(imp);
+                    if (COUNT) {
+                        cnt.edges += (uint32_t)__popcll(__ballot(on && du[i] < inf));
+                        cnt.relax += (uint32_t)__popcll(any);
+                    }
+                    if (any == 0ull) continue;
+                    const uint64_t bal = __ballot(imp && a < thr_s);
+                    const uint32_t hm = (uint32_t)(bal >> (32u * half));
+                    bool first = false;
+                    if (s == 0 && hm) {
+                        first = __hip_atomic_fetch_or(&mnxt[v[i]], hm, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0u;
+                        __hip_atomic_fetch_or(nl, hm, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+                    }
+                    if (ms.far) {
+                        const uint32_t fm = (uint32_t)(__ballot(imp && a >= thr_s) >> (32u * half));
+                        if (s == 0 && fm) {
+                            atomicOr(&ms.far[v[i]], fm);
+                            if ((ms.tfar[v[i] >> 6] & fm) != fm) atomicOr(&ms.tfar[v[i] >> 6], fm);
+                        }
+                    }
+                    if (push) {
+                        // the improver that found the next mask empty lists the vertex
+                        const uint64_t pm = __ballot(first);
+                        if (pm) {
+                            const uint32_t np = (uint32_t)__popcll(pm);
+                            if (pcount + np > PBUF) {
+                                flush_pushes(g, pbuf, pcount, qout, tail, ms.qcap, ms.ctl);
+                                pcount = 0;
+                            }
+                            if (first) {
+                                const uint32_t pos = pcount + __builtin_amdgcn_mbcnt_hi(
+                                                                  (uint32_t)(pm >> 32),
+                                                                  __builtin_amdgcn_mbcnt_lo((uint32_t)pm, 0u));
+                                pbuf[pos] = v[i];
+                            }
+                            pcount += np;
+                            __builtin_amdgcn_wave_barrier();
+                        }
                     }
                 }
-                if (COUNT) {
-                    cnt.edges += (uint32_t)__popcll(__ballot(on));
-                    cnt.relax += (uint32_t)__popcll(__ballot(imp));
-                }
-                if (push) {
-                    // the improver that found the next mask empty lists the vertex
-                    const uint64_t pm = __ballot(first);
-                    if (pm) {
-                        const uint32_t np = (uint32_t)__popcll(pm);
-                        if (pcount + np > PBUF) {
-                            flush_pushes(g, pbuf, pcount, qout, tail, ms.qcap, ms.ctl);
-                            pcount = 0;
-                        }
-                        if (first) {
-                            const uint32_t pos = pcount + __builtin_amdgcn_mbcnt_hi(
-                                                              (uint32_t)(pm >> 32),
-                                                              __builtin_amdgcn_mbcnt_lo((uint32_t)pm, 0u));
-                            pbuf[pos] = v[i];
-                        }
-                        pcount += np;
-                        __builtin_amdgcn_wave_barrier();
-                    }
-                }
             }
+            __builtin_amdgcn_wave_barrier();   // the slots are read before the next 64 overwrite them
         }
     }
     if (pcount) flush_pushes(g, pbuf, pcount, qout, tail, ms.qcap, ms.ctl);
@@ -567,12 +589,12 @@ template <bool COUNT, bool LM, bool CONT>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(CONT ? 4 : 8, 8)))
 void k_ms_step(gga_dev_graph g, gga_dev_ms ms, uint32_t step) {
     __shared__ uint32_t s_pbuf[WAVES][PBUF], s_nl[WAVES];
-    __shared__ uint4 s_cq[CONT ? WAVES : 1][CONT ? CQ : 1];
+    __shared__ uint4 s_cq[WAVES][CONT ? CQ : GGA_WAVE];
     const uint32_t nq = ms_len(ms, step);
     if (nq == 0) return;
     Counters cnt;
     const uint32_t wv = __builtin_amdgcn_readfirstlane(threadIdx.x / GGA_WAVE);   // wave-uniform
-    ms_relax<COUNT, LM, CONT>(g, ms, step, nq, s_pbuf[wv], &s_nl[wv], s_cq[CONT ? wv : 0], cnt);
+    ms_relax<COUNT, LM, CONT>(g, ms, step, nq, s_pbuf[wv], &s_nl[wv], s_cq[wv], cnt);
     publish_counters<COUNT>(ms, cnt);
 }
 
@@ -736,7 +758,7 @@ __global__ __launch_bounds__(BLOCK) void k_ms_persistent(gga_dev_graph g, gga_de
                                                          uint32_t max_steps, uint64_t spin_ticks) {
     __shared__ uint32_t s_pbuf[WAVES][PBUF];
     __shared__ uint32_t s_wave[WAVES], s_state[2], s_nl[WAVES];
-    __shared__ uint4 s_cq[CONT ? WAVES : 1][CONT ? CQ : 1];
+    __shared__ uint4 s_cq[WAVES][CONT ? CQ : GGA_WAVE];
     uint32_t gen = 0;
     if (threadIdx.x == 0)
         gen = __hip_atomic_load(&ms.ctl[GGA_CTL_BARGEN], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -753,7 +775,7 @@ __global__ __launch_bounds__(BLOCK) void k_ms_persistent(gga_dev_graph g, gga_de
         __syncthreads();
         if (nq == 0 || err) break;
         const uint32_t wv = __builtin_amdgcn_readfirstlane(threadIdx.x / GGA_WAVE);
-        ms_relax<COUNT, LM, CONT>(g, ms, step, nq, s_pbuf[wv], &s_nl[wv], s_cq[CONT ? wv : 0], cnt);
+        ms_relax<COUNT, LM, CONT>(g, ms, step, nq, s_pbuf[wv], &s_nl[wv], s_cq[wv], cnt);
         grid_barrier(ms.ctl, gridDim.x, gen, spin_ticks);
         if (ms_flag_step(ms, nq)) {
             const ListOut o = ms_list_out(g, ms, step);
