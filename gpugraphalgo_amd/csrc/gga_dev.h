@@ -91,7 +91,7 @@ typedef struct gga_wg_record {
  *               finish pass of step s clears the masks it consumed
  *   q0, q1      chunk lists (step s reads q[s & 1])
  *   tiles[GGA_TILES(n) + 1]  compaction counts / offsets */
-#define GGA_MS_RBLOCKS 512u   /* workgroups of the near-far refill (rows of lpart) */
+#define GGA_MS_RBLOCKS 128u   /* most workgroups of the near-far refill (rows of lpart) */
 #define GGA_MS_FAR_TILES(n) (((n) + 63u) / 64u)
 #ifndef GGA_MS_LANES
 #define GGA_MS_LANES 32   /* same value as include/gga.h */

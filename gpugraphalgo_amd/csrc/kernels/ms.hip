@@ -630,11 +630,28 @@ __global__ __launch_bounds__(CBLOCK) void k_ms_write(gga_dev_graph g, gga_dev_ms
 // reads one far-tile word per 64 vertices (the lanes deferred in the tile),
 // the far word of each vertex in a tile with a candidate's lane, and D only
 // where a candidate's bit is set.
-constexpr uint32_t RBLOCKS = GGA_MS_RBLOCKS;
-__global__ __launch_bounds__(BLOCK) void k_ms_tail(gga_dev_graph g, gga_dev_ms ms, uint32_t step) {
+//
+// What bounds it: the workgroups' arrivals -- each releases its row, an L2
+// write-back -- and a chain of dependent loads per tile and wave.  So tiles go
+// to all waves before any wave takes a second, in few workgroups of 16 waves:
+// a refill of a 512^2 grid 105 -> 30-45 us by the even spread (64 tiles a wave
+// before), a burst of 48 queries on two R-MAT s16 and two 512^2 grids 10.9 ->
+// 8.66 ms by it and 7.53 with 32 workgroups of 1024 threads (512 of 256
+// before; 8.17 / 7.84 / 7.58 with 256 / 128 / 64 of 1024).
+constexpr uint32_t RBLOCK = 1024, RWAVES = RBLOCK / GGA_WAVE;
+// 8 tiles a wave up to 128 workgroups, at least 32 where that leaves each wave
+// a tile: 32 lanes on a 1024^2 grid at 32 / 64 / 128 / 256 workgroups 25.6 /
+// 23.4 / 23.3 / 25.1 ms (512 of 256 threads: 31.0), on 4096^2 253 / 222 / 211 /
+// 218 (221).
+static uint32_t tail_blocks(uint32_t n) {
+    const uint32_t tiles = GGA_MS_FAR_TILES(n), one = (tiles + RWAVES - 1u) / RWAVES, b = (tiles + 127u) / 128u;
+    const uint32_t lo = one < 32u ? one : 32u;
+    return b < lo ? lo : (b < GGA_MS_RBLOCKS ? b : GGA_MS_RBLOCKS);
+}
+__global__ __launch_bounds__(RBLOCK) void k_ms_tail(gga_dev_graph g, gga_dev_ms ms, uint32_t step) {
     __shared__ uint32_t s_t1[LANES], s_min[LANES], s_listed, s_last, s_done;
-    __shared__ uint32_t s_pbuf[WAVES][PBUF];
-    __shared__ uint32_t s_red[BLOCK / LANES][LANES];
+    __shared__ uint32_t s_pbuf[RWAVES][PBUF];
+    __shared__ uint32_t s_red[RBLOCK / LANES][LANES];
     ms_finish(g, ms, step);
     if (!ms.far) return;
     const uint32_t sout = (step + 1u) % 3u;
@@ -653,15 +670,17 @@ __global__ __launch_bounds__(BLOCK) void k_ms_tail(gga_dev_graph g, gga_dev_ms m
     if (threadIdx.x == 0) s_listed = 0;
     __syncthreads();
     uint32_t listed = 0, pcount = 0;
-    // Each wave reads 64 consecutive far-tile words in one load, then walks
-    // only the tiles holding a candidate lane's bits, one vertex per lane
-    // (wave-uniform: the pushes below use whole-wave operations).
-    const uint64_t ntiles = GGA_MS_FAR_TILES(g.n);
-    const uint64_t wstride = (uint64_t)gridDim.x * WAVES * GGA_WAVE;
-    for (uint64_t tb = ((uint64_t)blockIdx.x * WAVES + threadIdx.x / GGA_WAVE) * GGA_WAVE; tb < ntiles;
-         tb += wstride) {
+    // Each wave reads up to 64 consecutive far-tile words in one load, then
+    // walks only the tiles holding a candidate lane's bits, one vertex per lane
+    // (wave-uniform: the pushes below use whole-wave operations).  A tile is a
+    // chain of dependent loads (far word, distances), so a graph of fewer
+    // tiles than 64 a wave spreads them over all waves.
+    const uint64_t ntiles = GGA_MS_FAR_TILES(g.n), nwaves = (uint64_t)gridDim.x * RWAVES;
+    const uint64_t even = (ntiles + nwaves - 1u) / nwaves, span = even < GGA_WAVE ? even : GGA_WAVE;
+    for (uint64_t tb = ((uint64_t)blockIdx.x * RWAVES + threadIdx.x / GGA_WAVE) * span; tb < ntiles;
+         tb += nwaves * span) {
         const uint64_t tl = tb + lane_id();
-        uint64_t tm = __ballot(tl < ntiles && (ms.tfar[tl] & cand) != 0u);   // tiles with a candidate's bit
+        uint64_t tm = __ballot(lane_id() < span && tl < ntiles && (ms.tfar[tl] & cand) != 0u);
         while (tm) {
             const uint64_t tile = tb + (uint64_t)__builtin_ctzll(tm);
             tm &= tm - 1u;
@@ -725,7 +744,7 @@ __global__ __launch_bounds__(BLOCK) void k_ms_tail(gga_dev_graph g, gga_dev_ms m
     {
         const uint32_t s = threadIdx.x & (LANES - 1u), grp = threadIdx.x / LANES;
         uint32_t gmin = 0xFFFFFFFFu;
-        for (uint32_t b = grp; b < gridDim.x; b += BLOCK / LANES) {
+        for (uint32_t b = grp; b < gridDim.x; b += RBLOCK / LANES) {
             const uint32_t x = ms.lpart[(uint64_t)b * LANES + s];
             gmin = x < gmin ? x : gmin;
         }
@@ -737,7 +756,7 @@ __global__ __launch_bounds__(BLOCK) void k_ms_tail(gga_dev_graph g, gga_dev_ms m
     if (threadIdx.x < LANES && ((cand >> threadIdx.x) & 1u)) {
         const uint32_t s = threadIdx.x;
         uint32_t gmin = 0xFFFFFFFFu;
-        for (uint32_t k = 0; k < BLOCK / LANES; k++) gmin = s_red[k][s] < gmin ? s_red[k][s] : gmin;
+        for (uint32_t k = 0; k < RBLOCK / LANES; k++) gmin = s_red[k][s] < gmin ? s_red[k][s] : gmin;
         if ((rl >> s) & 1u) ms.ctl[GGA_CTL_LTHR(s)] = sat_add(ms.ctl[GGA_CTL_LTHR(s)], ms.delta);
         else if (gmin != 0xFFFFFFFFu) ms.ctl[GGA_CTL_LTHR(s)] = gmin;
         else atomicOr(&s_done, 1u << s);
@@ -1061,7 +1080,7 @@ extern "C" int ggak_ms_step(gga_dev_graph g, gga_dev_ms ms, uint32_t step, int c
         k_ms_write<<<cg, CBLOCK, 0, s>>>(g, ms, step);
     }
     // lpart holds one row per workgroup of the tail pass
-    k_ms_tail<<<RBLOCKS, BLOCK, 0, s>>>(g, ms, step);
+    k_ms_tail<<<tail_blocks(g.n), RBLOCK, 0, s>>>(g, ms, step);
     return launch_status();
 }
 
