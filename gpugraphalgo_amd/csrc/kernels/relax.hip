@@ -28,8 +28,14 @@
 //     succeeds once per vertex).  Queued vertices are staged in wave-private
 //     LDS and flushed as chunk ids with one atomicAdd per 64 vertices.
 //   flag step (large frontier): fire-and-forget atomicMin and a plain store of
-//     a stamp into flag[v] (a byte array: a quarter of mark[]'s lines); then a three-pass compaction (count per tile, scan of tile
-//     counts, write) rebuilds the list from flag[] with no shared counter.
+//     a stamp into flag[v] (a byte array: a quarter of mark[]'s lines); then
+//     two compaction passes (count per tile, write from the counts before the
+//     tile) rebuild the list from flag[] with no shared counter and take each
+//     stamp back as its vertex is listed.
+// A level-synchronous BFS flag step needs no atomic: the byte is the guard and
+// a level is a plain store.  An uninstrumented worklist query is one launch
+// per phase (relax, count, write, refill; k_wl_phase), and a small graph's
+// whole query one workgroup (k_small).
 // Device-scope atomics on MI355X execute past the per-XCD L2 and atomics on
 // one address serialize (~16 ns each), so no hot path funnels through a single
 // counter: batch assignment is static, work counters are striped, list

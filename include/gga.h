@@ -190,7 +190,8 @@ typedef struct gga_opts {
                              size, else 256; GGA_EINVAL otherwise); PERSISTENT runs 256 */
     uint32_t sync_every;  /* WORKLIST: steps launched per host convergence check (0 -> 8, the
                              first check after one step more than the graph's last query
-                             needed, at most 32) */
+                             needed, at most 32; uninstrumented queries count the phases of
+                             those steps) */
     uint32_t use_graph;   /* multi-source engines: replay steps from captured hipGraphs (six
                              steps per graph) */
     uint32_t count;       /* 1 -> collect edges_inspected / chunks_expanded / relaxations, and
@@ -233,7 +234,8 @@ typedef struct gga_stats {
     uint64_t chunks_expanded; /* I_v  (opts.count) */
     uint64_t relaxations;     /* R: successful atomicMin (opts.count) */
     uint64_t m_reach;         /* sum of out-degrees of reached vertices */
-    uint64_t launches;        /* relax-kernel launches (uninstrumented WORKLIST: launches of its phases) */
+    uint64_t launches;        /* relax-kernel launches (uninstrumented WORKLIST: launches of its phases; 1 for a
+                                 small graph's query, which one workgroup runs) */
     uint32_t pull_levels;     /* gga_multi_bfs: levels run bottom-up */
     uint32_t timeline_records;/* records written to opts.timeline */
     uint32_t timeline_grid;   /* workgroups per step in it */
