@@ -333,7 +333,10 @@ static int graph_create(uint32_t n, uint32_t m, const uint32_t *row_ptr, const u
         goto fail;
     }
     g->skewed = skewed(g, row_ptr);
-    if (g->skewed && (rc = dmalloc(g, (void **)&g->d_sdist, 4ull * gga_spread_words(n)))) goto fail;
+    if (g->skewed && dmalloc(g, (void **)&g->d_sdist, 4ull * gga_spread_words(n))) {
+        gga_clear_error();   /* no room for it: queries relax in place */
+        (void)hipGetLastError();
+    }
     HIP_TRY(hipStreamSynchronize(g->stream));
     *out = g;
     return GGA_OK;
