@@ -1420,7 +1420,9 @@ __global__ __launch_bounds__(SMALL_BLOCK) void k_small(gga_dev_graph g, gga_dev_
             }
         };
         // out of the queue: its distance from now on.  (Its distance is under
-        // the threshold, so no deferral of it can follow.)
+        // the threshold, so no deferral of it can follow.)  By one lane a
+        // vertex: a second clear of the bit could come after another wave has
+        // set it and queued x again, and x would be queued twice, past n.
         auto take = [&](uint32_t x) {
             if (NEAR) atomicAnd(&far[x >> 5], ~(1u << (x & 31u)));
             __hip_atomic_fetch_and(&mark[x >> 5], ~(1u << (x & 31u)), __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_WORKGROUP);
@@ -1434,10 +1436,11 @@ __global__ __launch_bounds__(SMALL_BLOCK) void k_small(gga_dev_graph g, gga_dev_
                 uint32_t eb = 0, ne = 0, du = inf;
                 if (i < nf) {
                     const uint32_t x = qin[i];
-                    du = take(x);
+                    if ((l & 3u) == 0u) du = take(x);   // (one lane: once a vertex)
                     eb = row[x];
                     ne = row[x + 1u] - eb;
                 }
+                du = (uint32_t)__shfl((int)du, (int)(l & ~3u), GGA_WAVE);
                 for (uint32_t j = l & 3u; __ballot(j < ne) != 0ull; j += 4u) {
                     const bool on = j < ne;
                     const uint32_t e = on ? eb + j : 0u;   // (some lane has an edge: slot 0 is in bounds)
