@@ -558,6 +558,7 @@ __global__ __launch_bounds__(BLOCK) void k_fill(uint32_t *p, uint32_t value, uin
 // ring slot 0 = {len, step epoch}; counters and barrier zeroed.
 __global__ __launch_bounds__(BLOCK) void k_query_init(gga_dev_graph g, gga_dev_work w, uint32_t src,
                                                       uint32_t epoch) {
+    const uint64_t t0 = wall_clock64();   // the query's start, before the fills
     const uint64_t tid = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const uint64_t nth = (uint64_t)gridDim.x * blockDim.x;
     for (uint64_t v = tid; v < g.n; v += nth) w.dist[v] = (v == src) ? 0u : w.inf;
@@ -586,7 +587,7 @@ __global__ __launch_bounds__(BLOCK) void k_query_init(gga_dev_graph g, gga_dev_w
                 w.ctl[GGA_CTL_LISTED(i)] = 0;
             }
             w.ctl[GGA_CTL_PHASES] = 0;
-            *reinterpret_cast<uint64_t *>(w.ctl + GGA_CTL_T0) = wall_clock64();
+            *reinterpret_cast<uint64_t *>(w.ctl + GGA_CTL_T0) = t0;
             w.ctl[GGA_CTL_RSTEP] = epoch - 1u;   // no refill yet (step numbers start at epoch)
         }
         if (threadIdx.x < GGA_BAR_GROUPS) w.ctl[GGA_CTL_BARG(threadIdx.x)] = 0;

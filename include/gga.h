@@ -223,7 +223,10 @@ void gga_opts_init(gga_opts *o);
 typedef struct gga_stats {
     uint32_t iterations;      /* relax steps run (reference `iterations`) */
     uint32_t reached;         /* vertices with dist < inf */
-    float    time_ms;         /* device time, dist init -> convergence (reference `time`, bfs_sssp.cu:347-469) */
+    float    time_ms;         /* device time, dist init -> convergence (reference `time`, bfs_sssp.cu:347-469):
+                                 between two events, or, for an uninstrumented WORKLIST query of 256
+                                 threads, the device clock from the first workgroup of the
+                                 initialisation to the first of the kernel that ends the query */
     float    ktime_ms;        /* relax-kernel device time (reference `ktime`); measured with
                                  per-launch events, so only when opts.count is set (they cost
                                  a few us of dispatch gap each) or in PERSISTENT mode */
