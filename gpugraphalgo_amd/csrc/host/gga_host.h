@@ -28,6 +28,9 @@ void gga_graph_set_tuned(gga_graph *g, uint32_t grid, uint32_t dense_min, uint32
 uint32_t gga_graph_tuned_layout(const gga_graph *g);
 /* mode < 0: no tuned mode; delta 0xFFFFFFFF: near-far tuned off, 0: untuned. */
 void gga_graph_set_tuned_sssp(gga_graph *g, int32_t mode, uint32_t delta);
+/* on: no query runs in one workgroup, whatever its graph's size. */
+void gga_graph_set_scheduled(gga_graph *g, int on);
+int gga_graph_one_workgroup(const gga_graph *g);   /* the graph fits such a query */
 uint32_t gga_graph_wmean(const gga_graph *g);
 /* Near-far width a query with opts.delta == 0 would use (0: off). */
 uint32_t gga_graph_auto_delta(const gga_graph *g, int bfs);

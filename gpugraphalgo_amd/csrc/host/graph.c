@@ -62,6 +62,7 @@ struct gga_graph {
     uint32_t tuned_block;        /* worklist workgroup size from gga_tune (0: 256) */
     uint32_t tuned_delta;
     int32_t tuned_mode;          /* 0: none; else GGA_MODE_* + 1 */
+    int scheduled;               /* queries of small graphs take the step schedule too */
     uint32_t last_steps[2];      /* [bfs] relax steps of the last query (AUTO's evidence) */
     uint32_t last_phases[2];     /* [bfs] phases of the last query run one phase per launch */
     uint32_t wmean;              /* mean edge weight, rounded up (>= 1) */
@@ -603,6 +604,8 @@ void gga_graph_set_tuned_sssp(gga_graph *g, int32_t mode, uint32_t delta)
     g->tuned_delta = delta;
 }
 
+void gga_graph_set_scheduled(gga_graph *g, int on) { g->scheduled = on; }
+
 uint32_t gga_graph_wmean(const gga_graph *g) { return g ? g->wmean : 1u; }
 
 uint32_t gga_graph_tuned_layout(const gga_graph *g) { return g->tuned_layout; }
@@ -681,12 +684,17 @@ static int choose_mode(const gga_graph *g, int bfs)
  * sources each: pure 1024^2 grid 5.4-6.6 / 4.3-5.5 / 5.2-6.5 / 5.5-6.5 ms and
  * 8 / 12 / 19 / 35 M edges inspected, 4096^2 grid with 0.5% shortcuts 5.6 /
  * 5.2-5.3 / 5.4 / 6.2-6.3 ms); else off. */
-static uint32_t auto_delta(const gga_graph *g, int bfs)
+static uint32_t default_delta(const gga_graph *g, int bfs)
 {
-    if (g->tuned_delta) return g->tuned_delta == 0xFFFFFFFFu ? 0u : g->tuned_delta;
     if (bfs || !mesh_like(g)) return 0u;
     const uint64_t d = 8ull * g->wmean;
     return d < 0xFFFFFFF0ull ? (uint32_t)d : 0xFFFFFFF0u;
+}
+
+static uint32_t auto_delta(const gga_graph *g, int bfs)
+{
+    if (g->tuned_delta) return g->tuned_delta == 0xFFFFFFFFu ? 0u : g->tuned_delta;
+    return default_delta(g, bfs);
 }
 
 uint32_t gga_graph_auto_delta(const gga_graph *g, int bfs) { return g ? auto_delta(g, bfs) : 0u; }
@@ -1021,6 +1029,13 @@ fail:
     return rc;
 }
 
+static int thin_mesh(const gga_graph *g) { return mesh_like(g) && g->m <= 6ull * g->n; }
+
+int gga_graph_one_workgroup(const gga_graph *g)
+{
+    return g->n <= GGA_SMALL_N && (thin_mesh(g) || g->m <= 16384u);
+}
+
 /* Mode, near-far width and step cap of a query, from the options and what
  * the graph has learned (shared by gga_bfs / gga_sssp and the static-scratch
  * query). */
@@ -1040,23 +1055,24 @@ static void plan_query(const gga_graph *g, int bfs, const gga_opts *o, query_pla
     *delta = near_far ? d : 0u;
     p->max_iters = o->max_iters ? o->max_iters : (g->n + 1u);
     /* A query that leaves the schedule to the library, on a graph that one
-     * workgroup holds in LDS.  Thin fronts first: a mesh of at most 6 edges a
+     * workgroup holds in LDS (unless the tuner found the schedule it chose to
+     * be faster).  Thin fronts first: a mesh of at most 6 edges a
      * vertex gains at every size that fits (SSSP / BFS, general -> one
      * workgroup: 30 x 40 grid 148 / 80 -> 51 / 33 us, 100 x 77 301 / 170 ->
      * 164 / 93, 110 x 111 413 / 219 -> 244 / 126, 16 x 700 1593 / 720 -> 765 /
      * 407).  Elsewhere one CU's rate decides: R-MAT of 3.6 k edges 76 / 47 -> 25
      * / 14 us, 15 k 126 / 58 -> 79 / 33, 20 k 127 / 55 -> 120 / 39, 31 k 140 / 51
      * -> 177 / 58. */
-    const int thin = mesh_like(g) && g->m <= 6ull * g->n;
-    p->small = (o->mode == GGA_MODE_AUTO || o->mode == GGA_MODE_WORKLIST) && !p->count && !o->timeline &&
+    const int thin = thin_mesh(g);
+    p->small = !g->scheduled && (o->mode == GGA_MODE_AUTO || o->mode == GGA_MODE_WORKLIST) && !p->count && !o->timeline &&
                !o->conv_rows && !o->grid && !o->block && !o->dense_min && !o->delta && !o->sync_every &&
-               !o->max_iters && g->n <= GGA_SMALL_N && (thin || g->m <= 16384u);
+               !o->max_iters && gga_graph_one_workgroup(g);
     if (p->small) {
         /* near-far (thin SSSP): buckets twice as wide as the general path's --
          * a refill is two barriers here -- at 1 / 2 / 4 times: 100 x 77 grid
          * 174 / 164 / 173 us, 16 x 700 851 / 765 / 741, 110 x 111 with
          * shortcuts 140 / 139 / 178; without buckets 160 / 1649 / 148 */
-        const uint32_t width = auto_delta(g, 0);
+        const uint32_t width = default_delta(g, 0);
         p->mode = GGA_MODE_WORKLIST;
         p->thin = thin;
         p->max_iters = 64u * (g->n + 1u);
@@ -1091,7 +1107,9 @@ uint32_t gga_graph_default_dense(const gga_graph *g, int mode)
 
 static uint32_t dense_default(const gga_graph *g, const gga_opts *o, int mode)
 {
-    return o->dense_min ? o->dense_min : g->tuned_dense ? g->tuned_dense : gga_graph_default_dense(g, mode);
+    /* a tuned switch belongs to the launch mode it was timed in */
+    const int tuned = g->tuned_dense && (!g->tuned_mode || g->tuned_mode - 1 == mode);
+    return o->dense_min ? o->dense_min : tuned ? g->tuned_dense : gga_graph_default_dense(g, mode);
 }
 
 static int traverse(gga_graph *g, uint32_t src, int bfs, uint32_t *out, const gga_opts *user,

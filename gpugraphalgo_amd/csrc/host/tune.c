@@ -12,11 +12,13 @@
  * is built for workgroups of 128, 256 and 512 threads (2, 4, 8 waves with a
  * per-wave LDS push buffer each); the tuner times the three at their
  * occupancy grids, then the grid (workgroups resident per CU) for the one
- * it keeps.
+ * it keeps.  256 threads run one launch per phase of a step, the others four
+ * launches a step: each is timed as a query with that size runs.
  */
 #define _GNU_SOURCE
 #include <stdlib.h>
 #include <string.h>
+#include <time.h>
 
 #include "gga_host.h"
 
@@ -40,8 +42,17 @@ static void spread_sources(uint32_t n, uint32_t src, uint32_t *srcs)
     for (uint32_t i = 0; i < GGA_MS_LANES; i++) srcs[i] = (uint32_t)((src + (uint64_t)i * (n / GGA_MS_LANES + 1)) % n);
 }
 
-/* Best of three runs (device time, ms) of the tuning objective: one query
- * from src, or with GGA_TUNE_MULTI one 32-lane multi-source run. */
+static double now_ms(void)
+{
+    struct timespec t;
+    clock_gettime(CLOCK_MONOTONIC, &t);
+    return t.tv_sec * 1e3 + t.tv_nsec * 1e-6;
+}
+
+/* Best of three runs (ms of the whole call, which ends with the device idle)
+ * of the tuning objective: one query from src, or with GGA_TUNE_MULTI one
+ * 32-lane multi-source run.  Not the queries' own device times: a query's
+ * launch form decides what those span. */
 static int time_query(gga_graph *g, uint32_t src, int bfs, uint32_t flags, const gga_opts *o, float *ms)
 {
     float best = 0.f;
@@ -50,12 +61,14 @@ static int time_query(gga_graph *g, uint32_t src, int bfs, uint32_t flags, const
     for (int rep = 0; rep < 3; rep++) {
         gga_stats st;
         int rc;
+        const double t0 = now_ms();
         if (flags & GGA_TUNE_MULTI)
             rc = gga_multi_sp(g, srcs, GGA_MS_LANES, bfs ? 0xFFFFFFFFu : 0u, NULL, o, &st);
         else
             rc = bfs ? gga_bfs(g, src, NULL, o, &st) : gga_sssp(g, src, NULL, o, &st);
         if (rc) return rc;
-        if (rep == 0 || st.time_ms < best) best = st.time_ms;
+        const float t = (float)(now_ms() - t0);
+        if (rep == 0 || t < best) best = t;
     }
     *ms = best;
     return GGA_OK;
@@ -70,18 +83,17 @@ static void record(gga_tune_result *r, uint32_t mda, float ms)
     r->ntried++;
 }
 
-int gga_tune(gga_graph *g, uint32_t src, uint32_t flags, gga_tune_result *r)
+static int tune(gga_graph *g, uint32_t src, uint32_t flags, gga_tune_result *r)
 {
     int rc = GGA_OK;
-    if (!g || !r) return GGA_EINVAL;
-    if (src >= gga_graph_n(g)) return GGA_EINVAL;
-    memset(r, 0, sizeof *r);
     r->mode = GGA_MODE_WORKLIST;
-    r->delta = 0xFFFFFFFFu;
     const int bfs = (flags & GGA_TUNE_BFS) ? 1 : 0;
     gga_graph_set_tuned(g, 0, 0, 0);
     gga_graph_set_tuned_sssp(g, -1, 0);
     gga_graph_set_tuned_block(g, 0);
+    /* what opts.delta == 0 means below: the graph's default width */
+    const uint32_t width = gga_graph_auto_delta(g, bfs) ? gga_graph_auto_delta(g, bfs) : 0xFFFFFFFFu;
+    r->delta = width;
     r->block = 256u;
     gga_opts o;
     gga_opts_init(&o);
@@ -120,9 +132,8 @@ int gga_tune(gga_graph *g, uint32_t src, uint32_t flags, gga_tune_result *r)
     r->mda = best_t;
 
     /* 2. grid (workgroups) and 3. the push / compaction switch (single-source
-     * objective, worklist launches of plain Bellman-Ford; the multi-source
-     * engine sizes its own grid) */
-    o.delta = 0xFFFFFFFFu;
+     * objective, worklist launches at the default near-far width; the
+     * multi-source engine sizes its own grid) */
     const uint32_t n = gga_graph_n(g);
     if (flags & GGA_TUNE_MULTI) {
         r->best_ms = best;
@@ -167,44 +178,55 @@ int gga_tune(gga_graph *g, uint32_t src, uint32_t flags, gga_tune_result *r)
             r->dense_min = o.dense_min;
         }
     }
-    /* 4. launch mode and near-far width: the worklist launches and the
-     * persistent kernel, plain Bellman-Ford and buckets of 2, 8, 32 mean
-     * weights (SSSP); the two modes (BFS) */
+    /* 4. launch mode and near-far width: the worklist launches, timed so far
+     * at the default width, and the persistent kernel (its own grid and
+     * switch), plain Bellman-Ford and buckets of 2, 8, 32 mean weights (SSSP);
+     * the two modes (BFS) */
     {
         const uint32_t wm = gga_graph_wmean(g);
         const struct { int32_t mode; uint32_t delta; } cand2[] = {
-            {GGA_MODE_WORKLIST, 0xFFFFFFFFu},  {GGA_MODE_PERSISTENT, 0xFFFFFFFFu},
-            {GGA_MODE_PERSISTENT, 2u * wm},    {GGA_MODE_PERSISTENT, 8u * wm},
-            {GGA_MODE_PERSISTENT, 32u * wm},   {GGA_MODE_WORKLIST, 8u * wm}};
-        const size_t nc = bfs ? 2 : sizeof cand2 / sizeof cand2[0];
-        r->mode = GGA_MODE_WORKLIST;
-        r->delta = 0xFFFFFFFFu;
-        float mbest = best;
+            {GGA_MODE_PERSISTENT, 0xFFFFFFFFu}, {GGA_MODE_WORKLIST, 0xFFFFFFFFu},
+            {GGA_MODE_WORKLIST, 8u * wm},       {GGA_MODE_WORKLIST, 32u * wm},
+            {GGA_MODE_PERSISTENT, 2u * wm},     {GGA_MODE_PERSISTENT, 8u * wm},
+            {GGA_MODE_PERSISTENT, 32u * wm}};
+        const size_t nc = bfs ? 1 : sizeof cand2 / sizeof cand2[0];
+        o.dense_min = r->dense_min;
         for (size_t i = 0; i < nc; i++) {
             gga_opts o2 = o;
             float ms;
             o2.mode = cand2[i].mode;
             o2.delta = cand2[i].delta;
-            if (o2.mode == GGA_MODE_PERSISTENT) o2.grid = 0;   /* one workgroup per CU */
-            if (i == 0) {
-                mbest = best;   /* the configuration timed last above */
-                continue;
+            if (o2.mode == GGA_MODE_WORKLIST && o2.delta == width) continue;   /* timed */
+            if (o2.mode == GGA_MODE_PERSISTENT) {
+                o2.grid = 0;   /* one workgroup per CU */
+                o2.dense_min = 0;
             }
             if ((rc = time_query(g, src, bfs, flags, &o2, &ms))) return rc;
-            if (ms < mbest) {
-                mbest = ms;
+            if (ms < best) {
+                best = ms;
                 r->mode = o2.mode;
                 r->delta = o2.delta;
             }
         }
-        best = mbest;
+        if (r->mode == GGA_MODE_PERSISTENT) r->dense_min = gga_graph_default_dense(g, GGA_MODE_PERSISTENT);
         gga_graph_set_tuned_sssp(g, r->mode, bfs ? 0u : r->delta);
+    }
+    /* 5. a graph that one workgroup holds: all of the above against that */
+    if (gga_graph_one_workgroup(g)) {
+        gga_opts one;
+        float ms;
+        gga_opts_init(&one);
+        one.mode = GGA_MODE_AUTO;
+        gga_graph_set_scheduled(g, 0);
+        if ((rc = time_query(g, src, bfs, flags, &one, &ms))) return rc;
+        if (ms < best) best = ms;
+        else gga_graph_set_scheduled(g, 1);
     }
     r->best_ms = best;
 
     r->layout = gga_tune_layout(g);
 layout:
-    /* 4. multi-source layout: 32 lanes spread over the vertex range */
+    /* 6. multi-source layout: 32 lanes spread over the vertex range */
     if (flags & GGA_TUNE_LAYOUT) {
         uint32_t srcs[GGA_MS_LANES];
         spread_sources(n, src, srcs);
@@ -226,4 +248,16 @@ layout:
     gga_graph_set_tuned(g, r->grid, r->dense_min, (flags & GGA_TUNE_LAYOUT) ? r->layout : 0u);
     gga_graph_set_tuned_block(g, r->block);
     return GGA_OK;
+}
+
+int gga_tune(gga_graph *g, uint32_t src, uint32_t flags, gga_tune_result *r)
+{
+    if (!g || !r) return GGA_EINVAL;
+    if (src >= gga_graph_n(g)) return GGA_EINVAL;
+    memset(r, 0, sizeof *r);
+    /* the sweep times schedules; a graph that one workgroup holds has none */
+    gga_graph_set_scheduled(g, 1);
+    const int rc = tune(g, src, flags, r);
+    if (rc || !gga_graph_one_workgroup(g) || (flags & GGA_TUNE_MULTI)) gga_graph_set_scheduled(g, 0);
+    return rc;
 }

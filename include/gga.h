@@ -418,13 +418,15 @@ int gga_multi_bfs(gga_graph *g, const uint32_t *srcs, uint32_t k, uint32_t *out,
  * Replaces the histogram guess getMaxAllowedOutDegree (graph.h:359-385) and
  * the NodeSplitLevel sweep of mysc (mysc:20-51): the histogram threshold
  * (10 buckets, bfs_sssp.cu:166) seeds the candidates {seed, 16, 32, 64, 128,
- * 256, 1024, maxdeg}; each is timed on one query from src (best of 2 device
- * times), the fastest split is kept, then the worklist grid (default, 1/2,
+ * 256, 1024, maxdeg}; each is timed on one query from src (best of 3 calls,
+ * wall clock), the fastest split is kept, then the worklist grid (default, 1/2,
  * 1/4), the push / compaction switch (dense_min x 1/4, x 4) and the launch
- * mode with the near-far width (worklist / persistent, off / 2 / 8 / 32 mean
- * weights) are timed the same way.  The graph keeps the choices: later
- * queries whose opts leave mode AUTO and grid, dense_min, delta at 0 use
- * them.  GGA_TUNE_LAYOUT also times both multi-source engine layouts on 32
+ * mode with the near-far width (worklist / persistent, the default width /
+ * off / 2 / 8 / 32 mean weights) are timed the same way.  The graph keeps the
+ * choices: later queries whose opts leave mode AUTO and grid, dense_min, delta
+ * at 0 use them.  On a graph small enough for one workgroup to run a whole
+ * query the choices are timed against that at last, and such queries take them
+ * only where they won (best_ms is the faster one's).  GGA_TUNE_LAYOUT also times both multi-source engine layouts on 32
  * spread sources.  Results never depend on any choice. */
 #define GGA_TUNE_BFS     1u   /* tune with BFS queries (default SSSP) */
 #define GGA_TUNE_LAYOUT  2u   /* also measure the multi-source layout */
