@@ -92,6 +92,19 @@ constexpr uint32_t LVL_UNROLL = GGA_LVL_UNROLL;   // the same in expand_level
 #endif
 constexpr uint32_t CQ = GGA_CQ;
 constexpr uint32_t CONT_DEG = 16;
+// A wave stops following once more than CONT_FRONT vertices, plus a quarter of
+// those it followed, wait in its queue.  A mesh front that one wave follows
+// stays thin (its perimeter: some 45 of 256 followed on a grid); on a graph as
+// even in its degrees but without locality -- uniform random edges, a tree --
+// every round queues more than it follows, and the wave runs ahead of the
+// others into vertices that they reach on shorter ways.  Uniform graphs, all
+// 1024 followed -> stopped (and as it was with a queue of 128): BFS on 200 k
+// vertices of degree 16 880 -> 281 us (750), 4 M of degree 4 1767 -> 833
+// (1590), SSSP on 100 k of degree 6 989 -> 769 (900), on a binary tree of 1 M
+// 597 -> 485 (560); grids within 2%.  64 + a quarter: 4096^2 grid with
+// shortcuts BFS 5% slower than following nothing beyond its queue of 128; 384:
+// uniform BFS 444, 4 M 954-1406.
+constexpr uint32_t CONT_FRONT = 128;
 // Only steps whose list is at most this many chunks follow: a thin wavefront
 // leaves most of the chip idle and each step is a chain of dependent loads;
 // a wide one (a mesh with shortcuts, past its first levels) already fills the
@@ -212,6 +225,8 @@ __device__ __forceinline__ void follow_front(const gga_dev_graph &g, const gga_d
     while (qh != qt) {
         __builtin_amdgcn_wave_barrier();
         const uint32_t avail = qt - qh;
+        // (avail > CONT_FRONT + followed / 4: a growing front)
+        if (4u * avail + budget > 4u * CONT_FRONT + (uint32_t)GGA_CONT) budget = 0u;
         // budget spent, or too little room for what a round may queue: the
         // oldest entries are listed
         const bool drain = budget == 0u || CQ - avail < GGA_WAVE * G;
