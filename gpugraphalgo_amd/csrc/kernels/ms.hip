@@ -201,6 +201,15 @@ __device__ __forceinline__ bool relax_pair(const gga_dev_graph &g, const gga_dev
 // SSSP) on the pure 4096^2 grid 246 -> 189-202 ms, a burst of 48 queries on
 // two R-MAT s16 and two 512^2 / 256 x 512 grids 15.2 -> 12.1 ms; queue of 256
 // with one / two groups 198 / 213 ms and 12.6 / 12.3 ms.
+//
+// Once the queue runs full the wave stops and lists what waits: its front
+// grows with every hop, as on uniform random edges, where the pairs it would
+// go on to lower are mostly reached on shorter ways by others.  200 k vertices
+// of degree 16, 1024 followed -> stopped (and with the queue of 128 before): 4
+// SSSP lanes 5.3 -> 3.8 ms (4.0), 8 BFS lanes 3.56 -> 1.45 (2.23), 32 SSSP
+// lanes 13.9 -> 11.5 (13.7); 4 M of degree 4, 8 BFS lanes 19.1 -> 10.9 (18.0);
+// grids within 2%, a 256 x 512 grid with shortcuts 32 lanes 2.35 -> 2.6 ms
+// (4.3).  Stopping at 256 waiting pairs: that grid 2.9 ms, at 192 3.5.
 template <bool COUNT, bool LM, class List>
 __device__ __forceinline__ void follow_pairs(const gga_dev_graph &g, const gga_dev_ms &ms, uint32_t unit_word,
                                              uint32_t thr_s, uint4 *cq, uint32_t qt, const List &list, Counters &cnt) {
@@ -210,7 +219,8 @@ __device__ __forceinline__ void follow_pairs(const gga_dev_graph &g, const gga_d
     while (qh != qt) {
         __builtin_amdgcn_wave_barrier();
         const uint32_t avail = qt - qh;
-        const bool drain = budget == 0u || CQ - avail < GGA_WAVE * G;   // list the oldest pairs
+        if (CQ - avail < GGA_WAVE * G) budget = 0u;   // no room for a round: a growing front
+        const bool drain = budget == 0u;              // list the oldest pairs
         uint32_t take = drain ? GGA_WAVE : PER * G;
         take = take < avail ? take : avail;
         take = drain || take < budget ? take : budget;

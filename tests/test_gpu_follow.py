@@ -4,7 +4,7 @@ wave must not run ahead along them.
 Uniform random graphs, where following every vertex that a wave lowers made a
 BFS inspect 2.8 edges for each of the graph's and following next to none 2.2;
 2.4 lies between.  Results against the oracle, on trees and random graphs of
-several degrees, both queries, both list forms."""
+several degrees, both queries, both list forms, and engine lanes likewise."""
 import numpy as np
 import pytest
 
@@ -58,3 +58,33 @@ def test_results(gpu, make):
                 print(f"[gpu] n={g.n} m={g.m} src={src} {kw}", flush=True)
                 np.testing.assert_array_equal(dg.bfs(src, **kw)[0], want[True])
                 np.testing.assert_array_equal(dg.sssp(src, **kw)[0], want[False])
+
+
+def test_engine_lanes_stop_too(gpu):
+    """Eight BFS lanes of one engine: 1.8 edges inspected for each of the
+    graph's and lane with a short queue, 2.5 following all; 2.15 lies between."""
+    g = uniform(200000, 16 * 200000, 1)
+    srcs = [i * g.n // 8 for i in range(8)]
+    with gga.DeviceGraph(g) as dg:
+        dg.split()
+        for layout in (1, 2):
+            out, st = dg.multi_sp(srcs, bfs_lanes=0xFF, count=True, ms_layout=layout)
+            print(f"[gpu] layout={layout} edges / 8 m = {st['edges_inspected'] / (8 * g.m):.2f}", flush=True)
+            assert st["edges_inspected"] <= 2.15 * 8 * g.m
+            np.testing.assert_array_equal(out[3], oracle.bfs_queue(g.row_ptr, g.dst, srcs[3]))
+
+
+@pytest.mark.parametrize("make", [lambda: uniform(20001, 30001, 2), lambda: uniform(30000, 480000, 4),
+                                  lambda: tree(65535)])
+def test_engine_results(gpu, make):
+    g = make()
+    ones = np.ones(g.m, dtype=np.uint32)
+    srcs = [int(s) for s in np.flatnonzero(g.degrees() > 0)[:: g.n // 20][:9]]
+    want = [oracle.dijkstra(g.row_ptr, g.dst, ones if 0x0F >> i & 1 else g.w, s) for i, s in enumerate(srcs)]
+    with gga.DeviceGraph(g) as dg:
+        dg.split()
+        for kw in ({}, {"ms_layout": 1}, {"use_graph": 1}, {"mode": "persistent"}, {"dense_min": 1}):
+            print(f"[gpu] n={g.n} m={g.m} {kw}", flush=True)
+            out = dg.multi_sp(srcs, bfs_lanes=0x0F, **kw)[0]
+            for i in range(len(srcs)):
+                np.testing.assert_array_equal(out[i], want[i], err_msg=f"lane {i}")
