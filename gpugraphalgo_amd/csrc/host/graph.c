@@ -684,17 +684,22 @@ static int choose_mode(const gga_graph *g, int bfs)
  * sources each: pure 1024^2 grid 5.4-6.6 / 4.3-5.5 / 5.2-6.5 / 5.5-6.5 ms and
  * 8 / 12 / 19 / 35 M edges inspected, 4096^2 grid with 0.5% shortcuts 5.6 /
  * 5.2-5.3 / 5.4 / 6.2-6.3 ms); else off. */
-static uint32_t default_delta(const gga_graph *g, int bfs)
+static uint32_t default_delta(const gga_graph *g, int bfs, uint32_t means)
 {
     if (bfs || !mesh_like(g)) return 0u;
-    const uint64_t d = 8ull * g->wmean;
+    const uint64_t d = (uint64_t)means * g->wmean;
     return d < 0xFFFFFFF0ull ? (uint32_t)d : 0xFFFFFFF0u;
 }
 
+/* Paths and rings (no vertex of more than two arcs) take 32: nothing there is
+ * reached on a second way, so a narrow bucket saves no work and costs a refill
+ * every 8 hops (SSSP on a path of 20 k / 60 k vertices at 8 -> 32: 33.9 ->
+ * 17.1 / 103 -> 52 ms; engine, 4 lanes, 20 k: 63 -> 32; uniform random arcs,
+ * 1.5 a vertex, which the degrees do not tell from paths: 402 -> 517 us). */
 static uint32_t auto_delta(const gga_graph *g, int bfs)
 {
     if (g->tuned_delta) return g->tuned_delta == 0xFFFFFFFFu ? 0u : g->tuned_delta;
-    return default_delta(g, bfs);
+    return default_delta(g, bfs, g->maxdeg <= 2u ? 32u : 8u);
 }
 
 uint32_t gga_graph_auto_delta(const gga_graph *g, int bfs) { return g ? auto_delta(g, bfs) : 0u; }
@@ -1072,7 +1077,7 @@ static void plan_query(const gga_graph *g, int bfs, const gga_opts *o, query_pla
          * a refill is two barriers here -- at 1 / 2 / 4 times: 100 x 77 grid
          * 174 / 164 / 173 us, 16 x 700 851 / 765 / 741, 110 x 111 with
          * shortcuts 140 / 139 / 178; without buckets 160 / 1649 / 148 */
-        const uint32_t width = default_delta(g, 0);
+        const uint32_t width = default_delta(g, 0, 8u);
         p->mode = GGA_MODE_WORKLIST;
         p->thin = thin;
         p->max_iters = 64u * (g->n + 1u);
