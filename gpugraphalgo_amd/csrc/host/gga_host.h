@@ -32,7 +32,7 @@ void gga_graph_set_tuned_sssp(gga_graph *g, int32_t mode, uint32_t delta);
 void gga_graph_set_scheduled(gga_graph *g, int on);
 int gga_graph_one_workgroup(const gga_graph *g);   /* the graph fits such a query */
 uint32_t gga_graph_wmean(const gga_graph *g);
-/* Near-far width a query with opts.delta == 0 would use (0: off). */
+/* Near-far width a WORKLIST query with opts.delta == 0 would use (0: off). */
 uint32_t gga_graph_auto_delta(const gga_graph *g, int bfs);
 int gga_graph_mesh_like(const gga_graph *g);   /* max degree within 4x the mean (+8) */
 uint32_t gga_ms_step_grid(gga_ms *e);          /* an engine's default relax grid (0 on error) */

@@ -695,20 +695,25 @@ static uint32_t default_delta(const gga_graph *g, int bfs, uint32_t means)
  * reached on a second way, so a narrow bucket saves no work and costs a refill
  * every 8 hops (SSSP on a path of 20 k / 60 k vertices at 8 -> 32: 33.9 ->
  * 17.1 / 103 -> 52 ms; engine, 4 lanes, 20 k: 63 -> 32; uniform random arcs,
- * 1.5 a vertex, which the degrees do not tell from paths: 402 -> 517 us). */
-static uint32_t auto_delta(const gga_graph *g, int bfs)
+ * 1.5 a vertex, which the degrees do not tell from paths: 402 -> 517 us).
+ * The persistent kernel takes 16, as a refill is two more grid barriers there
+ * and the next bucket's start a third: SSSP at 8 / 16 on a 4 x 30000 grid 73.8
+ * / 49.9 ms, 30 x 9000 41.6 / 31.7, 300^2 1.83 / 1.69, 1024^2 6.55 / 6.34,
+ * 4096^2 with shortcuts 8.38 / 8.29, 1000^2 with shortcuts 1.39 / 1.52, uniform
+ * random 1 M of degree 4 1.12 / 1.14. */
+static uint32_t auto_delta(const gga_graph *g, int bfs, int mode)
 {
     if (g->tuned_delta) return g->tuned_delta == 0xFFFFFFFFu ? 0u : g->tuned_delta;
-    return default_delta(g, bfs, g->maxdeg <= 2u ? 32u : 8u);
+    return default_delta(g, bfs, g->maxdeg <= 2u ? 32u : mode == GGA_MODE_PERSISTENT ? 16u : 8u);
 }
 
-uint32_t gga_graph_auto_delta(const gga_graph *g, int bfs) { return g ? auto_delta(g, bfs) : 0u; }
+uint32_t gga_graph_auto_delta(const gga_graph *g, int bfs) { return g ? auto_delta(g, bfs, GGA_MODE_WORKLIST) : 0u; }
 
 /* The engines' default bucket width is the single-source one: a burst of 48
  * queries on two R-MAT s16 and two 512^2 / 256 x 512 grids took 17.1 / 11.8 /
  * 12.1 ms at 4 / 8 / 16 mean weights, 32 lanes on the 4096^2 grid 180 / 199 /
  * 189-202 ms. */
-uint32_t gga_graph_engine_delta(const gga_graph *g) { return g ? auto_delta(g, 0) : 0u; }
+uint32_t gga_graph_engine_delta(const gga_graph *g) { return gga_graph_auto_delta(g, 0); }
 int gga_graph_mesh_like(const gga_graph *g) { return g ? mesh_like(g) : 0; }
 
 /* One query on a prepared workspace: dist init, the relax loop of the chosen
@@ -1055,7 +1060,7 @@ static void plan_query(const gga_graph *g, int bfs, const gga_opts *o, query_pla
     /* Bellman-Ford needs at most n + 1 steps (graph.h:122); near-far adds
      * bucket changes and one empty step per jump over empty buckets, so its
      * default cap is only a guard */
-    const uint32_t d = o->delta == 0xFFFFFFFFu ? 0u : (o->delta ? o->delta : auto_delta(g, bfs));
+    const uint32_t d = o->delta == 0xFFFFFFFFu ? 0u : (o->delta ? o->delta : auto_delta(g, bfs, mode));
     const int near_far = !bfs && (mode == GGA_MODE_WORKLIST || mode == GGA_MODE_PERSISTENT) && d != 0u;
     *delta = near_far ? d : 0u;
     p->max_iters = o->max_iters ? o->max_iters : (g->n + 1u);

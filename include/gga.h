@@ -209,8 +209,8 @@ typedef struct gga_opts {
                              wait until the threshold passes them (Davidson et al. 2014), so
                              fewer vertices are expanded more than once; 0 -> the tuned width
                              (gga_tune), else 8 mean edge weights on mesh-like graphs (max
-                             degree within 4x the mean + 8; 32 where it is at most 2), else
-                             off; 0xFFFFFFFF -> off */
+                             degree within 4x the mean + 8; 32 where it is at most 2, 16 in
+                             PERSISTENT mode), else off; 0xFFFFFFFF -> off */
     /* WORKLIST instrumentation (both off when NULL) */
     gga_wg_record *timeline;    /* host buffer: grid records per step, steps in order */
     uint32_t timeline_cap;      /* records it holds; steps beyond it run uninstrumented */
