@@ -58,6 +58,7 @@ typedef struct gga_dev_work {
     uint32_t epoch;      /* step number of the query's first step */
     uint32_t cap;        /* most steps of a query run one phase per launch */
     uint32_t lvl;        /* 1: BFS steps are levels (step epoch + k reaches level k + 1) */
+    uint32_t guard;      /* 1: followed fronts read a distance before its atomic (a mesh with in-hubs) */
 } gga_dev_work;
 
 /* An odd multiplier permutes the residues of a power of two: neighbouring
@@ -119,6 +120,7 @@ typedef struct gga_dev_ms {
     uint32_t *lpart;     /* refill: per-workgroup per-lane minimum deferred distance */
     uint32_t delta;      /* bucket width */
     uint32_t bmin;       /* fewest chunks per wave batch (more on meshes, whose lanes rarely meet) */
+    uint32_t guard;      /* as gga_dev_work.guard */
 } gga_dev_ms;
 typedef struct gga_ms_sources { uint32_t v[GGA_MS_LANES]; } gga_ms_sources;
 typedef struct gga_ms_outputs { uint32_t *p[GGA_MS_LANES]; } gga_ms_outputs;

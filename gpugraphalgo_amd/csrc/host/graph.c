@@ -68,6 +68,7 @@ struct gga_graph {
     uint32_t wmean;              /* mean edge weight, rounded up (>= 1) */
     uint32_t *d_last, *d_tmin;   /* near-far state (allocated on first use) */
     int skewed;                  /* its hubs are neighbours: SSSP spreads its atomics */
+    int in_hubs;                 /* even out-degrees, but hubs among the destinations */
     uint32_t *d_sdist;           /* spread distances (allocated with a skewed graph) */
     void *msbfs;              /* transposed graph + state of gga_multi_bfs (msbfs.c) */
     hipEvent_t ev[4];
@@ -174,6 +175,7 @@ static gga_dev_work dev_work(const gga_graph *g, uint32_t inf)
     w.epoch = 0;
     w.cap = 0xFFFFFFFFu;
     w.lvl = 0;
+    w.guard = g->in_hubs ? 1u : 0u;
     return w;
 }
 
@@ -248,6 +250,36 @@ static int skewed(const gga_graph *g, const uint32_t *row_ptr)
     }
     return 0;
 }
+
+/* Whether a mesh-like graph -- mesh-like by its out-degrees -- has more than
+ * 1/128 of its arcs into 64 neighbouring vertices, a memory channel's fair
+ * share of all (and four times the share of 64 vertices, which is more on small
+ * graphs).  Its followed fronts then read a distance before the atomic on it:
+ * without, atomics of all waves queue at the hub.  4096 arcs, one at a pseudo-
+ * random place of each of as many equal parts, tell (32 expected at the line).
+ * 1 M vertices of 6 arcs, 1/8 of all arcs into one vertex, without / with the
+ * read: SSSP 2.45-3.5 / 1.27-1.39 ms, 8 engine lanes 64 / 9.0; 1/32 into one:
+ * 1.42-1.67 / 1.37-1.53, 23 / 9.2; 1/128 into one: 1.25 / 1.39, 11.6 / 9.2;
+ * 1/64 into 64: 1.10-1.23 / 1.19-1.35, 11.5 / 9.0; pure 1024^2 grid 3.93 /
+ * 5.02. */
+static int in_hubs(const gga_graph *g, const uint32_t *dst)
+{
+    if (!mesh_like(g) || g->m == 0) return 0;
+    const uint32_t parts = g->m < 4096u ? g->m : 4096u;
+    const uint64_t line = parts / 128u, even = 4ull * parts * 64u / g->n;
+    uint16_t *hits = (uint16_t *)calloc((size_t)(g->n / 64u) + 1u, sizeof *hits);
+    if (!hits) return 1;
+    int hot = 0;
+    for (uint32_t i = 0; i < parts && !hot; i++) {
+        const uint64_t lo = (uint64_t)g->m * i / parts, hi = (uint64_t)g->m * (i + 1u) / parts;
+        const uint32_t k = ++hits[dst[lo + gga_splitmix64(i) % (hi - lo)] / 64u];
+        hot = k > line && k > even;
+    }
+    free(hits);
+    return hot;
+}
+
+int gga_graph_in_hubs(const gga_graph *g) { return g ? g->in_hubs : 0; }
 
 static int graph_create(uint32_t n, uint32_t m, const uint32_t *row_ptr, const uint32_t *dst,
                         const uint32_t *w, int device, gga_graph **out)
@@ -333,6 +365,7 @@ static int graph_create(uint32_t n, uint32_t m, const uint32_t *row_ptr, const u
         rc = GGA_EFORMAT;
         goto fail;
     }
+    g->in_hubs = in_hubs(g, dst);
     g->skewed = skewed(g, row_ptr);
     if (g->skewed && dmalloc(g, (void **)&g->d_sdist, 4ull * gga_spread_words(n))) {
         gga_clear_error();   /* no room for it: queries relax in place */

@@ -145,6 +145,7 @@ int gga_ms_create(gga_graph *g, uint32_t inf, uint32_t layout, gga_ms **out)
      * its own wavefront (4096^2 grid, 32 / 8 lanes to convergence: batches
      * of 16, 256 followed pairs: 435 / 173 ms; 4 and 1 024: 343 / 154 ms) */
     e->d.bmin = gga_graph_mesh_like(g) ? GGA_MS_MESH_BMIN : 1u;
+    e->d.guard = gga_graph_in_hubs(g) ? 1u : 0u;
     HIP_TRY(hipSetDevice(e->v.device));
     /* a stream of its own, so that engines of one graph run side by side */
     HIP_TRY(hipStreamSynchronize(e->v.stream));

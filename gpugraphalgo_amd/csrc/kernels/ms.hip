@@ -210,7 +210,7 @@ __device__ __forceinline__ bool relax_pair(const gga_dev_graph &g, const gga_dev
 // lanes 13.9 -> 11.5 (13.7); 4 M of degree 4, 8 BFS lanes 19.1 -> 10.9 (18.0);
 // grids within 2%, a 256 x 512 grid with shortcuts 32 lanes 2.35 -> 2.6 ms
 // (4.3).  Stopping at 256 waiting pairs: that grid 2.9 ms, at 192 3.5.
-template <bool COUNT, bool LM, class List>
+template <bool COUNT, bool LM, bool GUARD, class List>
 __device__ __forceinline__ void follow_pairs(const gga_dev_graph &g, const gga_dev_ms &ms, uint32_t unit_word,
                                              uint32_t thr_s, uint4 *cq, uint32_t qt, const List &list, Counters &cnt) {
     constexpr uint32_t PER = GGA_WAVE / 4u, G = GGA_MS_GROUPS;
@@ -264,7 +264,8 @@ __device__ __forceinline__ void follow_pairs(const gga_dev_graph &g, const gga_d
             for (uint32_t i = 0; i < G; i++) {
                 if (i * PER >= take) break;
                 const uint32_t thr = (uint32_t)__shfl(thr_s, (int)sl[i], GGA_WAVE);
-                const bool pass = act[i] && a[i] >= du[i] && a[i] < inf;   // (no guard read, see above)
+                bool pass = act[i] && a[i] >= du[i] && a[i] < inf;   // (no guard read but on graphs with in-hubs: see follow_front in relax.hip)
+                if (GUARD) pass = pass && a[i] < ms.D[LM ? (uint64_t)sl[i] * g.n + v[i] : (uint64_t)v[i] * LANES + sl[i]];
                 const bool imp = relax_pair<LM, true>(g, ms, pass, v[i], sl[i], a[i], thr, cq, qh, qt, list);
                 if (COUNT) {
                     cnt.edges += (uint32_t)__popcll(__ballot(act[i]));
@@ -395,7 +396,10 @@ __device__ __forceinline__ void ms_relax(const gga_dev_graph &g, const gga_dev_m
                     }
                 }
             }
-            if (CONT && qt != 0u) follow_pairs<COUNT, LM>(g, ms, unit_word, thr_s, cq, qt, list_pair, cnt);
+            if (CONT && qt != 0u) {
+                if (ms.guard) follow_pairs<COUNT, LM, true>(g, ms, unit_word, thr_s, cq, qt, list_pair, cnt);
+                else follow_pairs<COUNT, LM, false>(g, ms, unit_word, thr_s, cq, qt, list_pair, cnt);
+            }
             continue;
         }
         // 64 edge slots at a time: one per wave lane for the owner search and

@@ -121,6 +121,11 @@ struct Counters {
     uint32_t edges = 0, chunks = 0, relax = 0;
 };
 
+// Whether waves follow their front (follow_front): not; without or with a
+// guard read before the atomic; or as w.guard says (kernels that are not built
+// once for each: the read's branch costs a mesh's SSSP 1%).
+enum { FOLLOW_NONE, FOLLOW, FOLLOW_GUARD, FOLLOW_EITHER };
+
 // A lane's chunk in a batch: its edge range [eb, ee) and owner.
 struct ChunkDesc {
     uint32_t eb = 0, ee = 0, own = 0;
@@ -210,10 +215,12 @@ __device__ __forceinline__ bool queue_near(bool near, uint32_t x, uint32_t d, ui
 // before the atomic it is two accesses, edge and atomic (it was chunk start,
 // chunk bounds, edge, dist[v], atomic, behind a 6-shuffle search).  A thin
 // front leaves the atomic units idle: without the guard SSSP on a pure 1024^2
-// grid went from 4.70 to 4.08 ms, on a 100 x 77 grid from 0.47 to 0.40.  With the queue of 512, SSSP: pure 1024^2 grid 8.9 -> 6.2
+// grid went from 4.70 to 4.08 ms, on a 100 x 77 grid from 0.47 to 0.40.  Where
+// many arcs lead to a few neighbouring vertices it is read (w.guard: in_hubs()
+// in host/graph.c has the sizes).  With the queue of 512, SSSP: pure 1024^2 grid 8.9 -> 6.2
 // ms, a 100 x 77 grid 0.80 -> 0.60, 4096^2 with shortcuts 6.8 -> 6.3; BFS on
 // the pure 1024^2 / 4096^2 grid 4.1-4.6 -> 2.9-3.2 / 19-25 -> 13-18 ms.
-template <bool BFS, bool COUNT, int OUT>
+template <bool BFS, bool COUNT, int OUT, bool GUARD>
 __device__ __forceinline__ void follow_front(const gga_dev_graph &g, const gga_dev_work &w, uint32_t it,
                                              uint32_t *pbuf, uint32_t &pcount, uint32_t *qout, uint32_t *tail,
                                              Counters &cnt, uint32_t thr, uint4 *cq, uint32_t qt) {
@@ -268,6 +275,13 @@ __device__ __forceinline__ void follow_front(const gga_dev_graph &g, const gga_d
                 const uint32_t e = act[u] ? eb[u] + j : 0u;   // (the graph has an edge: slot 0 is in bounds)
                 v[u] = g.col[e];
                 alt[u] = du[u] + (BFS ? 1u : g.w[e]);
+            }
+            if (GUARD) {
+                uint32_t d[G];
+#pragma unroll
+                for (uint32_t u = 0; u < G; u++) d[u] = u * PER < take ? dist[v[u]] : 0u;
+#pragma unroll
+                for (uint32_t u = 0; u < G; u++) act[u] = act[u] && alt[u] < d[u];
             }
 #pragma unroll
             for (uint32_t u = 0; u < G; u++) {
@@ -327,7 +341,7 @@ __device__ __forceinline__ void follow_front(const gga_dev_graph &g, const gga_d
 // -> 2186 (the copy falls out of the caches there: see skewed() for the rule).
 // Stores and stamps by everyone who passes the guard, no result awaited, left
 // dist loose enough to expand a quarter more edges (2^22: 2650 us).
-template <bool BFS, bool COUNT, int OUT, bool CONT = false, bool SPREAD = false>
+template <bool BFS, bool COUNT, int OUT, int CONT = FOLLOW_NONE, bool SPREAD = false>
 __device__ __forceinline__ void expand_batch(const gga_dev_graph &g, const gga_dev_work &w,
                                              const ChunkDesc &d, uint32_t it, uint32_t *pbuf,
                                              uint32_t &pcount, uint32_t *qout, uint32_t *tail,
@@ -362,7 +376,7 @@ __device__ __forceinline__ void expand_batch(const gga_dev_graph &g, const gga_d
         if (!SPREAD && w.last && go) w.last[own] = du;
         if (SPREAD && go) dist[own] = du;
     }
-    constexpr bool cont = CONT && OUT != OUT_CHANGED;
+    constexpr bool cont = CONT != FOLLOW_NONE && OUT != OUT_CHANGED;
     uint32_t qt = 0;   // vertices queued (wave-uniform)
     const uint32_t incl = wave_incl_scan(n);
     const uint32_t total = wave_last(incl);
@@ -417,8 +431,8 @@ __device__ __forceinline__ void expand_batch(const gga_dev_graph &g, const gga_d
 #pragma unroll
         for (uint32_t u = 0; u < UNROLL; u++) {
             if (u * GGA_WAVE >= left) break;
-            v[u] = edge_load<CONT>(&g.col[e[u]]);
-            wt[u] = BFS ? 1u : edge_load<CONT>(&g.w[e[u]]);
+            v[u] = edge_load<CONT != FOLLOW_NONE>(&g.col[e[u]]);
+            wt[u] = BFS ? 1u : edge_load<CONT != FOLLOW_NONE>(&g.w[e[u]]);
         }
 #pragma unroll
         for (uint32_t u = 0; u < UNROLL; u++) {
@@ -456,8 +470,12 @@ __device__ __forceinline__ void expand_batch(const gga_dev_graph &g, const gga_d
             list_vertex<BFS && !cont, OUT>(g, w, near && !queued, v[u], it, pbuf, pcount, qout, tail);
         }
     }
-    if (cont && cq && qt != 0u)
-        follow_front<BFS, COUNT, OUT>(g, w, it, pbuf, pcount, qout, tail, cnt, thr, cq, qt);
+    if (cont && cq && qt != 0u) {
+        if (CONT == FOLLOW_GUARD || (CONT == FOLLOW_EITHER && w.guard))
+            follow_front<BFS, COUNT, OUT, true>(g, w, it, pbuf, pcount, qout, tail, cnt, thr, cq, qt);
+        else
+            follow_front<BFS, COUNT, OUT, false>(g, w, it, pbuf, pcount, qout, tail, cnt, thr, cq, qt);
+    }
 }
 
 // Expand one batch of a level-synchronous BFS step (w.lvl): every listed
@@ -646,7 +664,7 @@ __device__ __forceinline__ bool flag_step(const gga_dev_work &w, uint32_t nq) {
 }
 
 // One step = expand the list of ring slot (step % 3), fill slot (step + 1) % 3.
-template <bool BFS, bool COUNT, bool CONT, bool SPREAD = false>
+template <bool BFS, bool COUNT, int CONT, bool SPREAD = false>
 __device__ __forceinline__ void worklist_step(const gga_dev_graph &g, const gga_dev_work &w,
                                               uint32_t step, uint32_t nq, uint32_t it,
                                               uint32_t *pbuf, uint4 *cq, uint2 *tab, Counters &cnt) {
@@ -689,7 +707,7 @@ __device__ __forceinline__ void worklist_step(const gga_dev_graph &g, const gga_
     auto entry = [&](uint64_t bb, bool &ok) -> uint32_t {
         const uint64_t idx = bb * bsz + l;
         ok = bb < nbatch && l < bsz && idx < nq;
-        return ok ? edge_load<CONT>(&qin[idx]) : 0u;
+        return ok ? edge_load<CONT != FOLLOW_NONE>(&qin[idx]) : 0u;
     };
     bool ok_next;
     uint32_t c_next;
@@ -698,12 +716,12 @@ __device__ __forceinline__ void worklist_step(const gga_dev_graph &g, const gga_
         bool ok0;
         const uint32_t c0 = entry(wid, ok0);
         c_next = entry((uint64_t)wid + waves, ok_next);
-        cur = load_chunk<CONT, !LVL>(g, c0, ok0);
+        cur = load_chunk<CONT != FOLLOW_NONE, !LVL>(g, c0, ok0);
     }
     for (uint64_t b = wid; b < nbatch; b += waves) {
         bool ok_after;
         const uint32_t c_after = entry(b + 2ull * waves, ok_after);
-        const ChunkDesc nxt = load_chunk<CONT, !LVL>(g, c_next, ok_next);
+        const ChunkDesc nxt = load_chunk<CONT != FOLLOW_NONE, !LVL>(g, c_next, ok_next);
         if (LVL && flags)
             expand_level<COUNT, OUT_FLAG>(g, w, cur, alt, stamp, pbuf, pcount, qout, tail, cnt,
                                           reinterpret_cast<uint32_t *>(tab), bsz);
@@ -852,7 +870,7 @@ void k_wl_step(gga_dev_graph g, gga_dev_work w, uint32_t step, gga_wg_record *tl
     if (nq != 0) {
         Counters cnt;
         const uint32_t wv = __builtin_amdgcn_readfirstlane(threadIdx.x / GGA_WAVE);
-        worklist_step<BFS, COUNT, CONT, SPREAD>(g, w, step, nq, it, s_pbuf[wv], s_cq[CONT ? wv : 0], s_tab[wv], cnt);
+        worklist_step<BFS, COUNT, CONT ? FOLLOW_EITHER : FOLLOW_NONE, SPREAD>(g, w, step, nq, it, s_pbuf[wv], s_cq[CONT ? wv : 0], s_tab[wv], cnt);
         publish_counters<COUNT>(w, cnt);
     }
     if (TL) {
@@ -1103,7 +1121,7 @@ __global__ __launch_bounds__(BLOCK) void k_refill_write(gga_dev_graph g, gga_dev
 // relax, count, write, refill -- cost a kernel boundary (~4.5 us) and a host
 // enqueue each whether the step needs them or not: a queue step needs one of
 // the four.
-template <bool BFS, bool CONT, bool SPREAD>
+template <bool BFS, int CONT, bool SPREAD>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(CONT ? 4 : 8, 8)))
 void k_wl_phase(gga_dev_graph g, gga_dev_work w, uint32_t launch) {
     __shared__ uint32_t s_pbuf[WAVES][PBUF];
@@ -1177,7 +1195,7 @@ __global__ __launch_bounds__(BLOCK) void k_persistent(gga_dev_graph g, gga_dev_w
         const uint32_t it = w.ctl[GGA_CTL_ITER(sin)];
         if (blockIdx.x == 0 && threadIdx.x == 0) step_bookkeeping(w.ctl, step, it, nq);
         const uint32_t wv = __builtin_amdgcn_readfirstlane(threadIdx.x / GGA_WAVE);
-        worklist_step<BFS, COUNT, CONT>(g, w, step, nq, it, s_pbuf[wv], s_cq[CONT ? wv : 0], s_tab[wv], cnt);
+        worklist_step<BFS, COUNT, CONT ? FOLLOW_EITHER : FOLLOW_NONE>(g, w, step, nq, it, s_pbuf[wv], s_cq[CONT ? wv : 0], s_tab[wv], cnt);
         if (flag_step(w, nq)) {
             const ListOut o = list_out(g, w, step);
             grid_barrier(w.ctl, gridDim.x, gen, spin_ticks);
@@ -1775,12 +1793,14 @@ extern "C" int ggak_conv(const uint32_t *dist, const uint32_t *fin, uint32_t n, 
 extern "C" int ggak_wl_phase(gga_dev_graph g, gga_dev_work w, uint32_t launch, int bfs, uint32_t grid, hipStream_t s) {
     if (grid == 0) return (int)hipErrorInvalidValue;
     if (bfs) {
-        if (use_cont(w)) k_wl_phase<true, true, false><<<grid, BLOCK, 0, s>>>(g, w, launch % 3u);
-        else k_wl_phase<true, false, false><<<grid, BLOCK, 0, s>>>(g, w, launch % 3u);
+        if (use_cont(w) && w.guard) k_wl_phase<true, FOLLOW_GUARD, false><<<grid, BLOCK, 0, s>>>(g, w, launch % 3u);
+        else if (use_cont(w)) k_wl_phase<true, FOLLOW, false><<<grid, BLOCK, 0, s>>>(g, w, launch % 3u);
+        else k_wl_phase<true, FOLLOW_NONE, false><<<grid, BLOCK, 0, s>>>(g, w, launch % 3u);
     } else {
-        if (use_cont(w)) k_wl_phase<false, true, false><<<grid, BLOCK, 0, s>>>(g, w, launch % 3u);
-        else if (w.sdist) k_wl_phase<false, false, true><<<grid, BLOCK, 0, s>>>(g, w, launch % 3u);
-        else k_wl_phase<false, false, false><<<grid, BLOCK, 0, s>>>(g, w, launch % 3u);
+        if (use_cont(w) && w.guard) k_wl_phase<false, FOLLOW_GUARD, false><<<grid, BLOCK, 0, s>>>(g, w, launch % 3u);
+        else if (use_cont(w)) k_wl_phase<false, FOLLOW, false><<<grid, BLOCK, 0, s>>>(g, w, launch % 3u);
+        else if (w.sdist) k_wl_phase<false, FOLLOW_NONE, true><<<grid, BLOCK, 0, s>>>(g, w, launch % 3u);
+        else k_wl_phase<false, FOLLOW_NONE, false><<<grid, BLOCK, 0, s>>>(g, w, launch % 3u);
     }
     return launch_status();
 }
