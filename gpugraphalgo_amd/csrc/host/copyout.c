@@ -11,7 +11,8 @@
  * included); three to fourteen threads are within 5% of each other.
  *
  * Pinning memory takes milliseconds, so slot sets are kept for the next copy of
- * any handle: at most KEPT idle sets, given back when the last handle goes.
+ * any handle: at most KEPT idle sets per device (pinned memory belongs to the
+ * device it was made for), given back when the last handle goes.
  * Each copy holds a set of its own, so copies of different threads, handles
  * and streams do not meet.  The threads live for one copy.
  */
@@ -31,7 +32,8 @@
 #define FILL_MIN (2u << 20)         /* bytes per fill of results below SLOTS * SLOT */
 #define THREADS 4u                  /* at most, beside the calling thread */
 #define PARALLEL (3ull << 20)       /* bytes from which threads are worth their start (~0.1 ms) */
-#define KEPT 2u                     /* idle sets kept */
+#define KEPT 2u                     /* idle sets kept per device */
+#define DEVICES 64                  /* devices with sets; copies of further ones go without */
 
 typedef struct slot_set {
     int device;
@@ -40,7 +42,7 @@ typedef struct slot_set {
 } slot_set;
 
 static pthread_mutex_t mu = PTHREAD_MUTEX_INITIALIZER;
-static slot_set *idle[KEPT];
+static slot_set *idle[DEVICES][KEPT];
 static uint64_t users;              /* live handles */
 
 static void set_free(slot_set *t)
@@ -61,27 +63,27 @@ void gga_copy_retain(void)
 
 void gga_copy_release(void)
 {
-    slot_set *gone[KEPT] = {NULL};
+    slot_set *gone[DEVICES][KEPT];
     pthread_mutex_lock(&mu);
-    if (--users == 0)
-        for (uint32_t i = 0; i < KEPT; i++) {
-            gone[i] = idle[i];
-            idle[i] = NULL;
-        }
+    const int last = --users == 0;
+    if (last) {
+        memcpy(gone, idle, sizeof gone);
+        memset(idle, 0, sizeof idle);
+    }
     pthread_mutex_unlock(&mu);
-    for (uint32_t i = 0; i < KEPT; i++) set_free(gone[i]);
+    for (uint32_t i = 0; last && i < DEVICES * KEPT; i++) set_free(gone[i / KEPT][i % KEPT]);
 }
 
-/* A set for `device` (current): an idle one, or a new one; NULL: no memory. */
+/* A set for `device` (current): an idle one, or a new one; NULL: no memory (or no such sets). */
 static slot_set *set_take(int device)
 {
     slot_set *t = NULL;
+    if (device < 0 || device >= DEVICES) return NULL;
     pthread_mutex_lock(&mu);
-    for (uint32_t i = 0; i < KEPT && !t; i++)
-        if (idle[i] && idle[i]->device == device) {
-            t = idle[i];
-            idle[i] = NULL;
-        }
+    for (uint32_t i = 0; i < KEPT && !t; i++) {
+        t = idle[device][i];
+        idle[device][i] = NULL;
+    }
     pthread_mutex_unlock(&mu);
     if (t) return t;
     t = (slot_set *)calloc(1, sizeof *t);
@@ -101,8 +103,8 @@ static void set_give(slot_set *t)
 {
     pthread_mutex_lock(&mu);
     for (uint32_t i = 0; i < KEPT && t && users; i++)
-        if (!idle[i]) {
-            idle[i] = t;
+        if (!idle[t->device][i]) {
+            idle[t->device][i] = t;
             t = NULL;
         }
     pthread_mutex_unlock(&mu);
