@@ -233,50 +233,57 @@ int gga_graph_free(gga_graph *g)
     return GGA_OK;
 }
 
-/* Whether SSSP spreads its atomics (w.sdist): a graph that is not mesh-like
- * and has 64 neighbouring vertices -- the 256 bytes of dist that share a
- * memory channel -- with more than 1/64 of its edges, twice a channel's fair
- * share of 128 (out-degrees stand in for the in-degrees, which only a pass over
- * all edges would give).  R-MAT hubs are the lowest ids: 4.9% of the edges at
- * 2^17 vertices (SSSP 12% faster spread), 2.1% at 2^20 (15%), 1.6% at 2^21
- * (4%), 1.2% at 2^22 (4% slower). */
-static int skewed(const gga_graph *g, const uint32_t *row_ptr)
+/* Whether more than 1/128 of the arcs lead into 64 neighbouring vertices -- the
+ * 256 bytes of dist that share a memory channel, and a channel's fair share of
+ * all -- and four times the share of 64 vertices, which is more on small graphs.
+ * 4096 arcs, one at a pseudo-random place of each of as many equal parts, tell
+ * (32 expected at the line); out of memory: yes. */
+static int hot_destinations(uint32_t n, uint32_t m, const uint32_t *dst)
 {
-    if (mesh_like(g)) return 0;
-    const uint32_t limit = g->m / 64u;
-    for (uint32_t v = 0; v < g->n; v += 64u) {
-        const uint32_t end = g->n - v > 64u ? v + 64u : g->n;
-        if (row_ptr[end] - row_ptr[v] > limit) return 1;
-    }
-    return 0;
-}
-
-/* Whether a mesh-like graph -- mesh-like by its out-degrees -- has more than
- * 1/128 of its arcs into 64 neighbouring vertices, a memory channel's fair
- * share of all (and four times the share of 64 vertices, which is more on small
- * graphs).  Its followed fronts then read a distance before the atomic on it:
- * without, atomics of all waves queue at the hub.  4096 arcs, one at a pseudo-
- * random place of each of as many equal parts, tell (32 expected at the line).
- * 1 M vertices of 6 arcs, 1/8 of all arcs into one vertex, without / with the
- * read: SSSP 2.45-3.5 / 1.27-1.39 ms, 8 engine lanes 64 / 9.0; 1/32 into one:
- * 1.42-1.67 / 1.37-1.53, 23 / 9.2; 1/128 into one: 1.25 / 1.39, 11.6 / 9.2;
- * 1/64 into 64: 1.10-1.23 / 1.19-1.35, 11.5 / 9.0; pure 1024^2 grid 3.93 /
- * 5.02. */
-static int in_hubs(const gga_graph *g, const uint32_t *dst)
-{
-    if (!mesh_like(g) || g->m == 0) return 0;
-    const uint32_t parts = g->m < 4096u ? g->m : 4096u;
-    const uint64_t line = parts / 128u, even = 4ull * parts * 64u / g->n;
-    uint16_t *hits = (uint16_t *)calloc((size_t)(g->n / 64u) + 1u, sizeof *hits);
+    const uint32_t parts = m < 4096u ? m : 4096u;
+    const uint64_t line = parts / 128u, even = 4ull * parts * 64u / n;
+    uint16_t *hits = (uint16_t *)calloc((size_t)(n / 64u) + 1u, sizeof *hits);
     if (!hits) return 1;
     int hot = 0;
     for (uint32_t i = 0; i < parts && !hot; i++) {
-        const uint64_t lo = (uint64_t)g->m * i / parts, hi = (uint64_t)g->m * (i + 1u) / parts;
+        const uint64_t lo = (uint64_t)m * i / parts, hi = (uint64_t)m * (i + 1u) / parts;
         const uint32_t k = ++hits[dst[lo + gga_splitmix64(i) % (hi - lo)] / 64u];
         hot = k > line && k > even;
     }
     free(hits);
     return hot;
+}
+
+/* Whether SSSP spreads its atomics (w.sdist): a graph that is not mesh-like
+ * and has 64 neighbouring vertices with more than 1/64 of its edges (by
+ * out-degree, which is exact and at hand) and with hot destinations too, by the
+ * sample -- R-MAT hubs are both, under the lowest ids: 4.9% of the edges at 2^17
+ * vertices (SSSP 12% faster spread), 2.1% at 2^20 (15%), 1.6% at 2^21 (4%),
+ * 1.2% at 2^22 (4% slower).  Smaller graphs: R-MAT 2^11 equal, 2^12 - 2^15
+ * 4 - 18% faster, 1 000 vertices of 100 k edges 4% slower (the copy is 256 KiB at
+ * least).  Hubs among the sources alone would pay for the copy and gain nothing:
+ * 1 M vertices of 16, a quarter of the arcs out of 64: 1063 -> 1182 us. */
+static int skewed(const gga_graph *g, const uint32_t *row_ptr, const uint32_t *dst)
+{
+    if (mesh_like(g)) return 0;
+    const uint32_t limit = g->m / 64u;
+    for (uint32_t v = 0; v < g->n; v += 64u) {
+        const uint32_t end = g->n - v > 64u ? v + 64u : g->n;
+        if (row_ptr[end] - row_ptr[v] > limit) return hot_destinations(g->n, g->m, dst);
+    }
+    return 0;
+}
+
+/* Whether a mesh-like graph -- mesh-like by its out-degrees -- has hot
+ * destinations.  Its followed fronts then read a distance before the atomic on
+ * it: without, atomics of all waves queue at the hub.  1 M vertices of 6 arcs,
+ * 1/8 of all arcs into one vertex, without / with the read: SSSP 2.45-3.5 /
+ * 1.27-1.39 ms, 8 engine lanes 64 / 9.0; 1/32 into one: 1.42-1.67 / 1.37-1.53,
+ * 23 / 9.2; 1/128 into one: 1.25 / 1.39, 11.6 / 9.2; 1/64 into 64: 1.10-1.23 /
+ * 1.19-1.35, 11.5 / 9.0; pure 1024^2 grid 3.93 / 5.02. */
+static int in_hubs(const gga_graph *g, const uint32_t *dst)
+{
+    return mesh_like(g) && g->m != 0u && hot_destinations(g->n, g->m, dst);
 }
 
 int gga_graph_in_hubs(const gga_graph *g) { return g ? g->in_hubs : 0; }
@@ -366,7 +373,7 @@ static int graph_create(uint32_t n, uint32_t m, const uint32_t *row_ptr, const u
         goto fail;
     }
     g->in_hubs = in_hubs(g, dst);
-    g->skewed = skewed(g, row_ptr);
+    g->skewed = skewed(g, row_ptr, dst);
     if (g->skewed && dmalloc(g, (void **)&g->d_sdist, 4ull * gga_spread_words(n))) {
         gga_clear_error();   /* no room for it: queries relax in place */
         (void)hipGetLastError();
