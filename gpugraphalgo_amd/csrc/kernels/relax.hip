@@ -1357,8 +1357,8 @@ __global__ __launch_bounds__(BLOCK) void k_finish(gga_dev_graph g, gga_dev_work 
 // frontier queues in LDS (12 bytes a vertex), col and w read from L2.  On a
 // graph this small every step is a chain of dependent accesses whatever the
 // grid, and the launches around it cost more than the step: here a step is an
-// LDS read, one edge load, an LDS atomic and a workgroup barrier (0.9 us on a
-// 100 x 77 grid).  What bounds it: that chain on meshes, one CU's rate of
+// LDS read, one edge load, an LDS atomic and a workgroup barrier (0.7 us:
+// BFS on a 100 x 77 grid, 176 levels in 121 us).  What bounds it: that chain on meshes, one CU's rate of
 // edges elsewhere (plan_query in host/graph.c has the sizes).
 // 1024 / 512 / 256 threads: 100 x 77 grid 164 / 199 / 271 us, 110 x 111 246 /
 // 302 / 427, R-MAT of 15 k edges 79 / 107 / 148.
@@ -1457,9 +1457,12 @@ __global__ __launch_bounds__(SMALL_BLOCK) void k_small(gga_dev_graph g, gga_dev_
         // the threshold, so no deferral of it can follow.)  By one lane a
         // vertex: a second clear of the bit could come after another wave has
         // set it and queued x again, and x would be queued twice, past n.
-        auto take = [&](uint32_t x) {
+        // (Cleared by all four lanes of a group SSSP took 10% longer.)
+        auto clear = [&](uint32_t x) {
             if (NEAR) atomicAnd(&far[x >> 5], ~(1u << (x & 31u)));
             __hip_atomic_fetch_and(&mark[x >> 5], ~(1u << (x & 31u)), __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_WORKGROUP);
+        };
+        auto distance = [&](uint32_t x) {
             return __hip_atomic_load(&dist[x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
         };
         if (MESH) {
@@ -1467,14 +1470,16 @@ __global__ __launch_bounds__(SMALL_BLOCK) void k_small(gga_dev_graph g, gga_dev_
             // no owner search (as in follow_front)
             for (uint32_t b = wv * 16u; b < nf; b += SMALL_WAVES * 16u) {
                 const uint32_t i = b + (l >> 2);
-                uint32_t eb = 0, ne = 0, du = inf;
+                uint32_t x = 0, eb = 0, ne = 0, du = inf;
                 if (i < nf) {
-                    const uint32_t x = qin[i];
-                    if ((l & 3u) == 0u) du = take(x);   // (one lane: once a vertex)
+                    x = qin[i];
                     eb = row[x];
                     ne = row[x + 1u] - eb;
+                    if ((l & 3u) == 0u) clear(x);
                 }
-                du = (uint32_t)__shfl((int)du, (int)(l & ~3u), GGA_WAVE);
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   // the clears before the reads
+                __builtin_amdgcn_wave_barrier();
+                if (i < nf) du = distance(x);
                 for (uint32_t j = l & 3u; __ballot(j < ne) != 0ull; j += 4u) {
                     const bool on = j < ne;
                     const uint32_t e = on ? eb + j : 0u;   // (some lane has an edge: slot 0 is in bounds)
@@ -1493,7 +1498,8 @@ __global__ __launch_bounds__(SMALL_BLOCK) void k_small(gga_dev_graph g, gga_dev_
             uint32_t eb = 0, ne = 0, du = inf;
             if (l < bsz && b + l < nf) {
                 const uint32_t x = qin[b + l];
-                du = take(x);
+                clear(x);
+                du = distance(x);
                 eb = row[x];
                 ne = row[x + 1u] - eb;
             }
