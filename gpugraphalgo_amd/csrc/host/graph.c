@@ -1106,13 +1106,14 @@ static void plan_query(const gga_graph *g, int bfs, const gga_opts *o, query_pla
     p->max_iters = o->max_iters ? o->max_iters : (g->n + 1u);
     /* A query that leaves the schedule to the library, on a graph that one
      * workgroup holds in LDS (unless the tuner found the schedule it chose to
-     * be faster).  Thin fronts first: a mesh of at most 6 edges a
-     * vertex gains at every size that fits (SSSP / BFS, general -> one
-     * workgroup: 30 x 40 grid 148 / 80 -> 51 / 33 us, 100 x 77 301 / 170 ->
-     * 164 / 93, 110 x 111 413 / 219 -> 244 / 126, 16 x 700 1593 / 720 -> 765 /
-     * 407).  Elsewhere one CU's rate decides: R-MAT of 3.6 k edges 76 / 47 -> 25
-     * / 14 us, 15 k 126 / 58 -> 79 / 33, 20 k 127 / 55 -> 120 / 39, 31 k 140 / 51
-     * -> 177 / 58. */
+     * be faster).  Thin fronts first: a mesh of at most 6 edges a vertex gains
+     * at every size that fits (SSSP / BFS, whole call, general -> one
+     * workgroup: 30 x 40 grid 176 / 102 -> 77 / 61 us, 100 x 77 383 / 223 ->
+     * 195 / 135, 110 x 111 478 / 267 -> 268 / 168, 16 x 700 1794 / 783 -> 855 /
+     * 482; uniform random arcs, 12 000 vertices of 6, 549 / 331 -> 203 / 80).
+     * Elsewhere one CU's rate decides: R-MAT of 3.2 k edges 85 / 51 -> 36 / 25,
+     * 12 k 122 / 56 -> 79 / 39; device time, 20 k 127 / 55 -> 120 / 39, 31 k 140
+     * / 51 -> 177 / 58: the line is the last power of two below the loss. */
     const int thin = thin_mesh(g);
     p->small = !g->scheduled && (o->mode == GGA_MODE_AUTO || o->mode == GGA_MODE_WORKLIST) && !p->count && !o->timeline &&
                !o->conv_rows && !o->grid && !o->block && !o->dense_min && !o->delta && !o->sync_every &&

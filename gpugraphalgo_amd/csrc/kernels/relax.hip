@@ -679,7 +679,7 @@ __device__ __forceinline__ void worklist_step(const gga_dev_graph &g, const gga_
     // the next step (R-MAT s22 SSSP, batches per wave 4 / 8 / 16 / 32: 2.33 /
     // 2.17 / 2.14 / 2.26 ms).  Uniform small chunks (meshes, bmin > 1): few
     // large batches -- every batch is a chain of dependent loads -- with one
-    // batch per 1/1024 of the list, but at least bmin chunks (4: each wave
+    // batch per 1/1024 of the list, but at least bmin chunks (2: each wave
     // then follows its own wavefront, see expand_batch).
     // Level-synchronous BFS has nothing to leave to the next step and takes 8
     // batches per wave (R-MAT s22, 4 / 8 / 16 / 32: 773 / 739 / 755 / 802 us)
@@ -1860,8 +1860,11 @@ extern "C" uint32_t ggak_wl_grid(int device, int persistent, int bfs, int count,
     if (persistent) block = BLOCK;
     if (block != 128 && block != 256 && block != 512) return 0;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess) return 0;
-    // (the continuation variants fit as many workgroups: same register cap,
-    // LDS well within a CU's; persistent grids take one per CU either way)
+    // (asked of the variants without followed fronts, 8 of 256 threads per CU.
+    // The mesh variants hold a queue of 8 KB a wave and four fit: their grid is
+    // twice what is resident, and steps are too short for that to show -- the
+    // tuner's grids of a half and a quarter are within 2% on 300^2 and 1024^2.
+    // Persistent grids take one per CU either way.)
     const void *fn = pick_kernel(persistent, bfs, count, block, 0, 0);
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, fn, (int)block, 0) != hipSuccess) return 0;
     if (per <= 0) return 0;

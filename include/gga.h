@@ -182,10 +182,18 @@ typedef struct gga_conv_row {
     double   norm2;
 } gga_conv_row;
 
+/* A WORKLIST / AUTO query with mode, inf and nothing else set, on a graph of at
+ * most 12288 vertices that is mesh-like with at most 6 edges a vertex or has at
+ * most 16384 edges, is run by one workgroup in LDS: it does not read the chunk
+ * table, and its SSSP steps, while each expands what the last one listed, are
+ * not those of the step schedule (a BFS takes its levels).  Any option below,
+ * or opts.count, asks for the schedule; so does gga_tune where it finds that
+ * faster. */
 typedef struct gga_opts {
     int32_t  mode;        /* GGA_MODE_* (default GGA_MODE_AUTO) */
     uint32_t inf;         /* unreached value: GGA_INF (0 -> default) or GGA_REF_INF */
-    uint32_t max_iters;   /* 0 -> n + 1 (the serial bound, graph.h:122) */
+    uint32_t max_iters;   /* 0 -> n + 1 (the serial bound, graph.h:122); 64 (n + 1) with near-far
+                             buckets and for a small graph's query (below) */
     uint32_t block;       /* WORKLIST: workgroup size, 128, 256 or 512 threads (0 -> the tuned
                              size, else 256; GGA_EINVAL otherwise); PERSISTENT runs 256 */
     uint32_t sync_every;  /* WORKLIST: steps launched per host convergence check (0 -> 8, the
