@@ -240,14 +240,14 @@ int gga_graph_free(gga_graph *g)
  * (32 expected at the line); out of memory: yes. */
 static int hot_destinations(uint32_t n, uint32_t m, const uint32_t *dst)
 {
-    const uint32_t parts = m < 4096u ? m : 4096u;
+    const uint32_t parts = m < 4096u ? m : 4096u, part = m / parts;
     const uint64_t line = parts / 128u, even = 4ull * parts * 64u / n;
     uint16_t *hits = (uint16_t *)calloc((size_t)(n / 64u) + 1u, sizeof *hits);
     if (!hits) return 1;
     int hot = 0;
     for (uint32_t i = 0; i < parts && !hot; i++) {
-        const uint64_t lo = (uint64_t)m * i / parts, hi = (uint64_t)m * (i + 1u) / parts;
-        const uint32_t k = ++hits[dst[lo + gga_splitmix64(i) % (hi - lo)] / 64u];
+        const uint32_t at = (uint32_t)((gga_splitmix64(i) >> 32) * part >> 32);   /* < part */
+        const uint32_t k = ++hits[dst[i * part + at] / 64u];
         hot = k > line && k > even;
     }
     free(hits);
