@@ -260,7 +260,7 @@ static int hot_destinations(uint32_t n, uint32_t m, const uint32_t *dst)
  * sample -- R-MAT hubs are both, under the lowest ids: 4.9% of the edges at 2^17
  * vertices (SSSP 12% faster spread), 2.1% at 2^20 (15%), 1.6% at 2^21 (4%),
  * 1.2% at 2^22 (4% slower).  Smaller graphs: R-MAT 2^11 equal, 2^12 - 2^15
- * 4 - 18% faster, 1 000 vertices of 100 k edges 4% slower (the copy is 256 KiB at
+ * 6 - 18% faster, 1 000 vertices of 100 k edges 4% slower (the copy is 256 KiB at
  * least).  Hubs among the sources alone would pay for the copy and gain nothing:
  * 1 M vertices of 16, a quarter of the arcs out of 64: 1063 -> 1182 us. */
 static int skewed(const gga_graph *g, const uint32_t *row_ptr, const uint32_t *dst)
